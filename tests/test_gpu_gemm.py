@@ -1,0 +1,73 @@
+"""The matrix-core product (ut_gemm.hip: five or more activation rows) against
+the closed form of the integer arithmetic, bit for bit, and against the
+one-row GEMV's rows.  The sums are exact integers, so the tolerance is zero.
+"""
+import numpy as np
+import pytest
+import torch
+
+from conftest import dev, host
+from qgen import INT4, INT8, gemv_closed_form, rand_qtensor
+
+pytestmark = pytest.mark.gpu
+
+# weight tiles of 256 rows and their remainders, K steps of 128 columns and
+# their tails, rows that are not 16-byte aligned, a payload's last bytes
+SHAPES = [(1, 1), (5, 17), (15, 16), (256, 128), (257, 160), (300, 1000), (1003, 1537), (64, 31),
+          (576, 7168), (255, 4096)]
+SEQS = [5, 15, 16, 17, 32, 33, 70]
+
+
+def run(ctx, q, x):
+    out = torch.full((x.shape[0], q.out_dim), float("nan"), device="cuda:0")
+    q.matmul(out, dev(x), x.shape[0])
+    return host(out)
+
+
+@pytest.mark.parametrize("fmt", [INT8, INT4])
+@pytest.mark.parametrize("o,i", SHAPES)
+def test_gemm_is_the_closed_form(ctx, fmt, o, i):
+    import undertow_amd as U
+    rng = np.random.default_rng(o * 7 + i + fmt)
+    payload, scales = rand_qtensor(rng, fmt, o, i)
+    q = U.QTensor(ctx, fmt, payload, scales, o, i)
+    x = rng.standard_normal((max(SEQS), i)).astype(np.float32)
+    x[1] = 0.0
+    x[2] *= 1e-30
+    x[3, 0] = 1e30
+    want = gemv_closed_form(fmt, payload, scales, o, i, x)
+    one = run(ctx, q, x[4:5])
+    for seq in SEQS:
+        got = run(ctx, q, x[:seq])
+        assert np.array_equal(got, want[:seq]), seq
+        assert np.array_equal(got[4:5], one)
+
+
+@pytest.mark.parametrize("fmt", [INT8, INT4])
+def test_gemm_largest_codes_do_not_overflow(ctx, fmt):
+    """65,536 columns (the widest the int32 plane sums take) of extreme codes
+    and digits: every x~ is 2^22, whose planes are 0, 0 and 64."""
+    import undertow_amd as U
+    o, i, seq = 17, 65536, 6
+    payload = (np.full((o, i), -127, np.int8) if fmt == INT8 else np.full((o, i // 2), 0x88, np.uint8))
+    scales = np.ones(o, np.float32)
+    x = np.full((seq, i), np.float32(1.0))
+    x[1] = -1.0
+    x[2] = np.float32(0.99999988)  # x~ = 2^22 - 1 rounds up to 2^22 at E = 0
+    x[3, ::2] = np.float32(0.50196) # digits near the balanced limit
+    q = U.QTensor(ctx, fmt, payload, scales, o, i)
+    assert np.array_equal(run(ctx, q, x), gemv_closed_form(fmt, payload, scales, o, i, x))
+
+
+def test_gemm_nonfinite_rows_are_nan(ctx):
+    import undertow_amd as U
+    rng = np.random.default_rng(5)
+    payload, scales = rand_qtensor(rng, INT8, 40, 256)
+    x = rng.standard_normal((9, 256)).astype(np.float32)
+    want = gemv_closed_form(INT8, payload, scales, 40, 256, x)
+    x[2, 7] = np.inf
+    x[5, 255] = np.nan
+    got = run(ctx, U.QTensor(ctx, INT8, payload, scales, 40, 256), x)
+    assert np.isnan(got[[2, 5]]).all()
+    ok = [r for r in range(9) if r not in (2, 5)]
+    assert np.array_equal(got[ok], want[ok])

@@ -1,0 +1,37 @@
+// ut_gemm.h -- quantized matrix products over more rows than the skinny
+// GEMVs take (prompts): internal interface of ut_gemm.hip.
+#pragma once
+
+#include "ut_internal.h"
+
+namespace ut {
+
+// A batch of activation rows as base-256 digit planes: plane p of row m is
+// the kp bytes at p + (m*3 + p)*kp, zero past K (kp: K rounded up to 128),
+// exps[m] the row's exponent (XDigits).
+struct DigitPlanes {
+    int8_t *p = nullptr;
+    int64_t kp = 0;
+    int32_t *exps = nullptr;
+};
+inline int64_t planes_pitch(int64_t K) { return (K + 127) / 128 * 128; }
+size_t planes_bytes(int64_t M, int64_t K);
+DigitPlanes planes_view(void *base, int64_t M, int64_t K);
+// Digitises x [M, K] (row stride ldx), f32 or bf16.
+int32_t launch_planes(ut_ctx *ctx, const float *x, int64_t ldx, int64_t M, int64_t K,
+                      const DigitPlanes &pl);
+int32_t launch_planes(ut_ctx *ctx, const uint16_t *x, int64_t ldx, int64_t M, int64_t K,
+                      const DigitPlanes &pl);
+
+// The fewest rows that take the matrix-core GEMM; four-row GEMV passes over
+// the weight are slower from the second pass on (five rows, GEMV passes
+// against GEMM: int8 7168 x 16384 63.7 -> 43.9 us, 576 x 7168 25.0 -> 18.8,
+// 256 x 256 13.4 -> 9.8, int4 7168 x 2048 21.9 -> 12.9).
+constexpr int64_t kGemmMinRows = 5;
+bool gemm_ok(const ut_qtensor *w, int64_t M);
+// out[m, o] (+)= x[m] . w[o] for M digitised rows; the values are the
+// GEMVs', bit for bit.
+int32_t launch_gemm(ut_ctx *ctx, const ut_qtensor *w, const DigitPlanes &x, int64_t M, float *out,
+                    int64_t ldo, int accumulate);
+
+}  // namespace ut

@@ -1,0 +1,292 @@
+// ut_gemm.hip -- QTensor::matmul (undertow-quant/src/qtensor.rs:281-319) on
+// gfx950 for more rows than the skinny GEMVs take: digit planes of the
+// activations and the matrix-core product (ut_gemm_core.h).
+#include "ut_gemm.h"
+
+#include "ut_gemm_core.h"
+
+namespace ut {
+
+// ------------------------------------------------------- digit planes ---
+size_t planes_bytes(int64_t M, int64_t K) {
+    return (((size_t)M * 4 + 255) & ~size_t(255)) + (size_t)M * 3 * planes_pitch(K);
+}
+DigitPlanes planes_view(void *base, int64_t M, int64_t K) {
+    DigitPlanes d;
+    d.exps = (int32_t *)base;
+    d.p = (int8_t *)base + (((size_t)M * 4 + 255) & ~size_t(255));
+    d.kp = planes_pitch(K);
+    return d;
+}
+
+__device__ __forceinline__ float plane_value(const float *x, int64_t k) { return x[k]; }
+__device__ __forceinline__ float plane_value(const uint16_t *x, int64_t k) {
+    return __uint_as_float((uint32_t)x[k] << 16);
+}
+__device__ __forceinline__ void plane_load4(const float *x, int64_t k, float (&v)[4]) {
+    const float4 f = ld_global<float4>(x + k);
+    v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w;
+}
+__device__ __forceinline__ void plane_load4(const uint16_t *x, int64_t k, float (&v)[4]) {
+    const uint2 u = ld_global<uint2>(x + k);
+    v[0] = __uint_as_float(u.x << 16); v[1] = __uint_as_float(u.x & 0xffff0000u);
+    v[2] = __uint_as_float(u.y << 16); v[3] = __uint_as_float(u.y & 0xffff0000u);
+}
+
+// One workgroup per row: max|x|, exponent, then four columns a time into
+// one word per plane.  Rows of up to kPlaneRegs * 1024 columns stay in
+// registers between the two passes.  Bound by the row's read: one round
+// trip (512 rows of 16,384 columns: 33.5 MB in, 25 MB out).
+constexpr int kPlaneRegs = 8;
+template <typename T, bool VEC>
+__global__ __launch_bounds__(256) void k_planes(const T *__restrict__ x, int64_t ldx, int64_t K,
+                                                int8_t *__restrict__ pl, int64_t kp,
+                                                int32_t *__restrict__ exps) {
+    __shared__ uint32_t red[4];
+    const int64_t m = blockIdx.x;
+    const int tid = threadIdx.x;
+    const T *xr = x + m * ldx;
+    float v[kPlaneRegs][4];
+    auto load = [&](int64_t c, float (&o)[4]) {
+        if (VEC && c + 4 <= K) {
+            plane_load4(xr, c, o);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; j++) o[j] = c + j < K ? plane_value(xr, c + j) : 0.0f;
+        }
+    };
+    uint32_t mx = 0;
+#pragma unroll
+    for (int i = 0; i < kPlaneRegs; i++) {
+        const int64_t c = 4 * (tid + 256 * (int64_t)i);
+        if (c < kp) load(c, v[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < kPlaneRegs; i++)
+        if (4 * (tid + 256 * (int64_t)i) < kp)
+#pragma unroll
+            for (int j = 0; j < 4; j++) mx = max(mx, __float_as_uint(fabsf(v[i][j])));
+    for (int64_t c = 4 * (tid + 256 * (int64_t)kPlaneRegs); c < K; c += 1024) {
+        float t[4];
+        load(c, t);
+#pragma unroll
+        for (int j = 0; j < 4; j++) mx = max(mx, __float_as_uint(fabsf(t[j])));
+    }
+    mx = block_reduce(mx, [](uint32_t a, uint32_t b) { return a > b ? a : b; }, red);
+    // non-finite rows (|x| bits >= +inf) produce NaN outputs downstream
+    const bool bad = mx >= 0x7f800000u;
+    int E = 0;
+    if (!bad && mx != 0) (void)frexpf(__uint_as_float(mx), &E);
+    const int sh = bad ? INT32_MIN : 22 - E;
+    if (tid == 0) exps[m] = bad ? INT32_MIN : E - 22;
+    auto put = [&](int64_t c, const float (&o)[4]) {
+        uint32_t w[3];
+        digit_words<UT_FMT_INT8>(o, 4, sh, w);
+#pragma unroll
+        for (int p = 0; p < 3; p++) *(uint32_t *)(pl + (m * 3 + p) * kp + c) = bad ? 0u : w[p];
+    };
+#pragma unroll
+    for (int i = 0; i < kPlaneRegs; i++) {
+        const int64_t c = 4 * (tid + 256 * (int64_t)i);
+        if (c < kp) put(c, v[i]);
+    }
+    for (int64_t c = 4 * (tid + 256 * (int64_t)kPlaneRegs); c < kp; c += 1024) {
+        float t[4];
+        load(c, t);
+        put(c, t);
+    }
+}
+
+template <typename T>
+static int32_t planes_t(ut_ctx *ctx, const T *x, int64_t ldx, int64_t M, int64_t K,
+                        const DigitPlanes &pl) {
+    if (M <= 0) return UT_OK;
+    const bool vec = ((uintptr_t)x % (4 * sizeof(T))) == 0 && ldx % 4 == 0;
+    int tok = timing_begin(ctx, "planes");
+    if (vec)
+        hipLaunchKernelGGL((k_planes<T, true>), dim3((unsigned)M), dim3(256), 0, ctx->stream, x, ldx,
+                           K, pl.p, pl.kp, pl.exps);
+    else
+        hipLaunchKernelGGL((k_planes<T, false>), dim3((unsigned)M), dim3(256), 0, ctx->stream, x,
+                           ldx, K, pl.p, pl.kp, pl.exps);
+    timing_end(ctx, tok);
+    return launch_check(ctx, "k_planes");
+}
+int32_t launch_planes(ut_ctx *ctx, const float *x, int64_t ldx, int64_t M, int64_t K,
+                      const DigitPlanes &pl) {
+    return planes_t(ctx, x, ldx, M, K, pl);
+}
+int32_t launch_planes(ut_ctx *ctx, const uint16_t *x, int64_t ldx, int64_t M, int64_t K,
+                      const DigitPlanes &pl) {
+    return planes_t(ctx, x, ldx, M, K, pl);
+}
+
+// --------------------------------------------------------------- GEMM ---
+struct GemmArgs {
+    const uint8_t *w;
+    const float *scales;
+    int64_t O, row_bytes;  // weight rows, bytes from one to the next (all of them read)
+    const uint8_t *end;
+    const int8_t *pl;
+    int64_t kp;
+    const int32_t *exps;
+    int64_t M;
+    float *out;
+    int64_t ldo;
+    int accumulate;
+    // units = weight tiles x K splits; a unit's activation tiles run on one XCD
+    int to, tm, ks;
+    int64_t kslice;
+    int64_t *part;  // ks > 1: totals [ks][M][O]
+};
+
+// Up to about 32 rows the weights' read bounds it (int8 7168 x 16384 from
+// memory: 16 rows 47 us, 2.5 TB/s; the four-row GEMV passes took 118 us),
+// beyond that the matrix cores (512 rows 290 us, 1.24 POP/s of digit
+// products against 3,611 us; 129280 x 7168 2,100 against 19,492 us).
+constexpr int kGemmTO = 4;
+template <int FMT, int TM, bool UNAL>
+__global__ __launch_bounds__(kGemmThreads, 2) void k_gemm(GemmArgs a) {
+    __shared__ uint4 lds[gemm_lds_uint4<TM>()];
+    // consecutive workgroups go to the 8 XCDs in turn: the activation tiles
+    // of one weight tile are given to one XCD, so its L2 serves the weights
+    // to all but the first of them
+    const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
+    const int unit = (j / a.tm) * 8 + xcd, mt = j % a.tm;
+    if (unit >= a.to * a.ks) return;
+    const int ot = unit % a.to, z = unit / a.to;
+    const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, q = lane >> 4;
+    const int64_t o0 = (int64_t)ot * (64 * kGemmTO) + (tid >> 6) * (16 * kGemmTO);
+    const int64_t m0 = (int64_t)mt * (16 * TM);
+    GemmRows<kGemmTO> rows;
+#pragma unroll
+    for (int t = 0; t < kGemmTO; t++) {
+        const int64_t o = o0 + 16 * t + r;
+        rows.row[t] = a.w + (o < a.O ? o : a.O - 1) * a.row_bytes;
+    }
+    rows.end = a.end;
+    const int8_t *src[gemm_stage_n<TM>()];
+#pragma unroll
+    for (int i = 0; i < gemm_stage_n<TM>(); i++) {
+        const GemmChunk c = gemm_chunk(tid + i * kGemmThreads);
+        const int64_t m = m0 + c.m < a.M ? m0 + c.m : a.M - 1;
+        src[i] = a.pl + (m * 3 + (c.p < 3 ? c.p : 0)) * a.kp + c.off;
+    }
+    const int64_t kb = z * a.kslice, ke = kb + a.kslice < a.kp ? kb + a.kslice : a.kp;
+    ut_i32x4 acc[kGemmTO][TM][3];
+    gemm_tile<FMT, kGemmTO, TM, UNAL>(rows, a.row_bytes, kb, ke, src, lds, acc);
+#pragma unroll
+    for (int t = 0; t < kGemmTO; t++) {
+        const int64_t o = o0 + 16 * t + 4 * q;
+#pragma unroll
+        for (int n = 0; n < TM; n++) {
+            const int64_t m = m0 + 16 * n + r;
+            if (m >= a.M || o >= a.O) continue;
+            int64_t S[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) S[i] = gemm_total(acc[t][n], i);
+            if (a.ks > 1) {
+                int64_t *p = a.part + ((int64_t)z * a.M + m) * a.O + o;
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    if (o + i < a.O) p[i] = S[i];
+                continue;
+            }
+            const int32_t e = gemm_exp<FMT>(a.exps[m]);
+            float *po = a.out + m * a.ldo + o;
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (o + i < a.O) {
+                    const float v = int_total_to_f32(S[i], e, ld_global_f32(a.scales + o + i));
+                    po[i] = a.accumulate ? __fadd_rn(po[i], v) : v;
+                }
+        }
+    }
+}
+
+// The K splits' totals summed and scaled (exact integers: any order).
+template <int FMT>
+__global__ __launch_bounds__(256) void k_gemm_sum(GemmArgs a) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x, n = a.M * a.O;
+    if (i >= n) return;
+    const int64_t m = i / a.O, o = i - m * a.O;
+    int64_t S = 0;
+    for (int z = 0; z < a.ks; z++) S += a.part[z * n + i];
+    const float v = int_total_to_f32(S, gemm_exp<FMT>(a.exps[m]), a.scales[o]);
+    float *po = a.out + m * a.ldo + o;
+    *po = a.accumulate ? __fadd_rn(*po, v) : v;
+}
+
+bool gemm_ok(const ut_qtensor *w, int64_t M) {
+    // 65,536 columns: the planes' int32 sums (K x 128 x 128) cannot overflow
+    return M >= kGemmMinRows && (w->fmt == UT_FMT_INT8 || w->fmt == UT_FMT_INT4) &&
+           w->in_dim >= 1 && w->in_dim <= 65536;
+}
+
+int32_t launch_gemm(ut_ctx *ctx, const ut_qtensor *w, const DigitPlanes &x, int64_t M, float *out,
+                    int64_t ldo, int accumulate) {
+    GemmArgs a{};
+    a.w = (const uint8_t *)w->payload;
+    a.scales = w->scales;
+    a.O = w->out_dim;
+    a.row_bytes = w->row_bytes;
+    a.end = a.w + w->out_dim * w->row_bytes;
+    a.pl = x.p;
+    a.kp = x.kp;
+    a.exps = x.exps;
+    a.out = out;
+    a.ldo = ldo;
+    a.accumulate = accumulate;
+    const bool unal = ((uintptr_t)w->payload & 15) != 0 || w->row_bytes % 16 != 0;
+    const int64_t cap = unal ? 1 << 20 : 1 << 24;  // rows per launch: grids stay in 31 bits
+    for (int64_t s0 = 0; s0 < M; s0 += cap) {
+        a.M = M - s0 < cap ? M - s0 : cap;
+        a.pl = x.p + s0 * 3 * x.kp;
+        a.exps = x.exps + s0;
+        a.out = out + s0 * ldo;
+        const int tmr = a.M <= 16 ? 1 : a.M <= 32 ? 2 : 2;
+        a.to = (int)((a.O + 64 * kGemmTO - 1) / (64 * kGemmTO));
+        a.tm = (int)((a.M + 16 * tmr - 1) / (16 * tmr));
+        // split K until the launch has two workgroups per CU, at least two
+        // steps each, partials within their buffer
+        int64_t ks = (2 * ctx->multiprocessors) / ((int64_t)a.to * a.tm);
+        const int64_t steps = a.kp / kGemmStep;
+        if (ks > steps / 2) ks = steps / 2;
+        while (ks > 1 && ks * a.M * a.O * 8 > kSplitKPartBytes) ks--;
+        if (ks < 1) ks = 1;
+        a.kslice = (steps + ks - 1) / ks * kGemmStep;
+        a.ks = (int)((a.kp + a.kslice - 1) / a.kslice);
+        if (a.ks > 1) UT_TRY(splitk_buffer(ctx, &a.part));
+        const int64_t units = (int64_t)a.to * a.ks;
+        const dim3 grid((unsigned)((units + 7) / 8 * 8 * a.tm));
+        int tok = timing_begin(ctx, "gemm");
+#define UT_GM(F, T, U) hipLaunchKernelGGL((k_gemm<F, T, U>), grid, dim3(kGemmThreads), 0, ctx->stream, a)
+#define UT_GMT(F, U)                    \
+    do {                                \
+        if (tmr == 1) UT_GM(F, 1, U);   \
+        else UT_GM(F, 2, U);            \
+    } while (0)
+        if (w->fmt == UT_FMT_INT8) {
+            if (unal) UT_GMT(UT_FMT_INT8, true);
+            else UT_GMT(UT_FMT_INT8, false);
+        } else {
+            if (unal) UT_GMT(UT_FMT_INT4, true);
+            else UT_GMT(UT_FMT_INT4, false);
+        }
+#undef UT_GMT
+#undef UT_GM
+        UT_TRY(launch_check(ctx, "k_gemm"));
+        if (a.ks > 1) {
+            const dim3 sg((unsigned)((a.M * a.O + 255) / 256));
+            if (w->fmt == UT_FMT_INT8)
+                hipLaunchKernelGGL(k_gemm_sum<UT_FMT_INT8>, sg, dim3(256), 0, ctx->stream, a);
+            else
+                hipLaunchKernelGGL(k_gemm_sum<UT_FMT_INT4>, sg, dim3(256), 0, ctx->stream, a);
+            UT_TRY(launch_check(ctx, "k_gemm_sum"));
+        }
+        timing_end(ctx, tok);
+    }
+    return UT_OK;
+}
+
+}  // namespace ut

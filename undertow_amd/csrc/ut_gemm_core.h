@@ -1,0 +1,187 @@
+// ut_gemm_core.h -- the tile of the matrix-core product of quantized weights
+// with digitised activation rows.
+//
+// A row of the product is S = sum_k x~[k] q[k] over the activation's integer
+// form x~ (ut_internal.h), which three balanced base-256 digits hold: the
+// tile multiplies the weight codes with the three digit planes on
+// v_mfma_i32_16x16x64_i8 and adds S = a0 + 256 a1 + 65536 a2 in 64 bits, so
+// the totals are the GEMVs' whatever the tile or the K split.
+//
+// A workgroup of four waves takes 64*TO weight rows (TO tiles of 16 per
+// wave) against 16*TM activation rows.  The weights go from memory straight
+// to the registers of the one wave that uses them (each lane a 16-byte
+// piece of one row); only the digit planes, which all four waves read, go
+// through LDS: at TO = 4 each digit fragment read feeds four matrix
+// instructions, so LDS runs at half the matrix cores' time.  Both are
+// fetched a step of 128 columns ahead; the barrier waits for LDS only, so
+// the weight loads stay in flight across it.  LDS rows of 128 bytes keep
+// their 16-byte chunks XOR-swizzled by the row's low three bits: eight lanes
+// that read one chunk of eight rows use all 32 banks.
+#pragma once
+
+#include "ut_gemv_mfma.h"
+
+namespace ut {
+
+constexpr int kGemmThreads = 256;
+constexpr int kGemmStep = 128;  // columns per step (two matrix instructions deep)
+template <int TM> __host__ __device__ constexpr int gemm_lds_uint4() {
+    return 2 * TM * 48 * (kGemmStep / 16);  // two buffers of 48 TM plane rows
+}
+template <int TM> constexpr int gemm_stage_n() { return (TM * 48 * 8 + kGemmThreads - 1) / kGemmThreads; }
+
+// Where a lane's weights come from: row bases (this lane's row of each
+// tile), and for rows that are not 16-byte aligned the payload's end.
+template <int TO> struct GemmRows {
+    const uint8_t *row[TO];
+    const uint8_t *end;
+};
+
+// 16 bytes at p + off of a weight row of `len` bytes.  Aligned rows clamp a
+// chunk past the row to its last one (its columns meet zero digits); others
+// read the chunk unaligned, or byte by byte where it would leave the payload.
+template <bool UNAL>
+__device__ __forceinline__ uint4 gemm_ld16(const uint8_t *p, int64_t off, int64_t len,
+                                           const uint8_t *end) {
+    if constexpr (!UNAL) return ld_global<uint4>(p + (off < len ? off : len - 16));
+    uint4 v = make_uint4(0, 0, 0, 0);
+    if (off >= len) return v;
+    const uint8_t *q = p + off;
+    if (q + 16 <= end) {
+        typedef unsigned int u32x4u __attribute__((ext_vector_type(4), aligned(1)));
+        const u32x4u t = *(const __attribute__((address_space(1))) u32x4u *)q;
+        return make_uint4(t.x, t.y, t.z, t.w);
+    }
+    uint32_t w[4] = {0, 0, 0, 0};
+    const int n = (int)(end - q);
+    for (int i = 0; i < n; i++) w[i >> 2] |= (uint32_t)q[i] << (8 * (i & 3));
+    return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+// One step's weights of TO tiles: int8 two 16-byte pieces per row (columns
+// 64s + 16q of the step for matrix instruction s and lane quarter q), int4
+// one (columns 32q + 16s).
+template <int FMT, int TO> struct GemmA {
+    static constexpr int NP = FMT == UT_FMT_INT8 ? 2 : 1;
+    uint4 v[TO][NP];
+};
+template <int FMT, int TO, bool UNAL>
+__device__ __forceinline__ void gemm_load_a(GemmA<FMT, TO> &a, const GemmRows<TO> &r, int64_t col,
+                                            int64_t len, int q) {
+#pragma unroll
+    for (int t = 0; t < TO; t++)
+#pragma unroll
+        for (int i = 0; i < GemmA<FMT, TO>::NP; i++) {
+            const int64_t off = FMT == UT_FMT_INT8 ? col + 64 * i + 16 * q : col / 2 + 16 * q;
+            a.v[t][i] = gemm_ld16<UNAL>(r.row[t], off, len, r.end);
+        }
+}
+// The A operand of matrix instruction s: 16 codes per lane.  int4 codes come
+// out times 16 (a nibble in the byte's high half is its own sign extension),
+// which the epilogue's exponent takes back.
+template <int FMT, int TO>
+__device__ __forceinline__ ut_i32x4 gemm_frag_a(const GemmA<FMT, TO> &a, int t, int s) {
+    ut_i32x4 f;
+    if constexpr (FMT == UT_FMT_INT8) {
+        const uint4 v = a.v[t][s];
+        f[0] = (int)v.x; f[1] = (int)v.y; f[2] = (int)v.z; f[3] = (int)v.w;
+    } else {
+        const uint4 v = a.v[t][0];
+        const uint32_t u[2] = {s ? v.z : v.x, s ? v.w : v.y};
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const uint32_t lo = (u[j] << 4) & 0xF0F0F0F0u, hi = u[j] & 0xF0F0F0F0u;
+            f[2 * j] = (int)__builtin_amdgcn_perm(hi, lo, 0x05010400u);
+            f[2 * j + 1] = (int)__builtin_amdgcn_perm(hi, lo, 0x07030602u);
+        }
+    }
+    return f;
+}
+template <int FMT> __device__ __forceinline__ int32_t gemm_exp(int32_t e) {
+    return FMT == UT_FMT_INT4 && e != INT32_MIN ? e - 4 : e;
+}
+
+// acc[t][n][p] += tile over columns [kb, ke) (kb a multiple of 128, columns
+// past K zero in the planes).  src[i]: the digit bytes of this thread's
+// staging chunk i at column 0 (its chunk offset included).
+template <int FMT, int TO, int TM, bool UNAL>
+__device__ __forceinline__ void gemm_tile(const GemmRows<TO> &rows, int64_t len, int64_t kb,
+                                          int64_t ke, const int8_t *const (&src)[gemm_stage_n<TM>()],
+                                          uint4 *lds, ut_i32x4 (&acc)[TO][TM][3]) {
+    constexpr int NB = gemm_stage_n<TM>(), CH = TM * 48 * 8;
+    const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, q = lane >> 4;
+#pragma unroll
+    for (int t = 0; t < TO; t++)
+#pragma unroll
+        for (int n = 0; n < TM; n++)
+#pragma unroll
+            for (int p = 0; p < 3; p++) acc[t][n][p] = ut_i32x4{0, 0, 0, 0};
+    uint4 b[NB];
+    auto load_b = [&](int64_t k) {
+#pragma unroll
+        for (int i = 0; i < NB; i++)
+            if (tid + i * kGemmThreads < CH) b[i] = ld_global<uint4>(src[i] + k);
+    };
+    auto store_b = [&](uint4 *dst) {
+#pragma unroll
+        for (int i = 0; i < NB; i++)
+            if (tid + i * kGemmThreads < CH) dst[tid + i * kGemmThreads] = b[i];
+    };
+    auto compute = [&](const GemmA<FMT, TO> &a, const uint4 *buf) {
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+            const int chunk = (FMT == UT_FMT_INT8 ? 4 * s + q : 2 * q + s) ^ (r & 7);
+            ut_i32x4 f[TO];
+#pragma unroll
+            for (int t = 0; t < TO; t++) f[t] = gemm_frag_a<FMT, TO>(a, t, s);
+#pragma unroll
+            for (int n = 0; n < TM; n++)
+#pragma unroll
+                for (int p = 0; p < 3; p++) {
+                    const uint4 v = buf[((n * 3 + p) * 16 + r) * 8 + chunk];
+                    const ut_i32x4 w{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
+#pragma unroll
+                    for (int t = 0; t < TO; t++)
+                        acc[t][n][p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(f[t], w, acc[t][n][p], 0, 0, 0);
+                }
+        }
+    };
+    auto barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+    GemmA<FMT, TO> cur, nxt;
+    load_b(kb);
+    gemm_load_a<FMT, TO, UNAL>(cur, rows, kb, len, q);
+    store_b(lds);
+    barrier();
+    int o = 0;
+    for (int64_t k = kb; k < ke; k += kGemmStep) {
+        const bool more = k + kGemmStep < ke;
+        if (more) {
+            load_b(k + kGemmStep);
+            gemm_load_a<FMT, TO, UNAL>(nxt, rows, k + kGemmStep, len, q);
+        }
+        compute(cur, lds + o);
+        o = CH - o;
+        if (more) {
+            store_b(lds + o);
+            cur = nxt;
+        }
+        barrier();
+    }
+}
+
+// The exact total of one accumulator element.
+__device__ __forceinline__ int64_t gemm_total(const ut_i32x4 (&a)[3], int j) {
+    return (int64_t)a[0][j] + ((int64_t)a[1][j] << 8) + ((int64_t)a[2][j] << 16);
+}
+
+// A thread's staging chunk: plane row (of 48 TM, tile-major: 16 activation
+// rows of one plane after another) and 16-byte chunk within the step.
+struct GemmChunk {
+    int m, p, off;
+};
+__device__ __forceinline__ GemmChunk gemm_chunk(int c) {
+    const int rr = c >> 3, n = rr / 48, x = rr - 48 * n;
+    return {16 * n + (x & 15), x >> 4, ((c & 7) ^ (rr & 7)) * 16};
+}
+
+}  // namespace ut

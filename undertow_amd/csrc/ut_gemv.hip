@@ -2,9 +2,11 @@
 // 281-493 and the kernels it dispatches to, kernels.rs:21-81 /
 // avx512.rs:197-267): activation digitisation, the fast skinny GEMV
 // (int4 / int8 / f32 weights, 1..4 activation rows per pass) and a generic
-// kernel for shapes the fast one does not take.
+// kernel for shapes the fast one does not take.  More rows of int4 / int8
+// weights go to the matrix-core product of ut_gemm.hip.
 #include <atomic>
 #include "ut_argmax.h"
+#include "ut_gemm.h"
 #include "ut_gemv_core.h"
 #include "ut_gemv_mfma.h"
 #include "ut_moe.h"
@@ -1575,7 +1577,17 @@ int32_t gemv(ut_ctx *ctx, const GemvArgs &ga) {
 }
 
 size_t matmul_digit_bytes(int64_t M, int64_t K) {
-    return xdigits_bytes(M, K, XD_DIG4 | XD_DIG8 | XD_XT);
+    const size_t b = xdigits_bytes(M, K, XD_DIG4 | XD_DIG8 | XD_XT), p = planes_bytes(M, K);
+    return b > p ? b : p;
+}
+
+// A batch's base-256 digits are the GEMM's planes where rows need no padding.
+static bool xdigits_planes(const XDigits &xd, int64_t K, DigitPlanes *pl) {
+    if (!xd.dig8 || planes_pitch(K) != K || ((uintptr_t)xd.dig8 & 15)) return false;
+    pl->p = (int8_t *)xd.dig8;
+    pl->kp = K;
+    pl->exps = xd.exps;
+    return true;
 }
 
 // ------------------------------------------------------ fast int8 ---
@@ -1676,6 +1688,9 @@ int32_t matmul_digits(ut_ctx *ctx, const ut_qtensor *w, const float *x, const XD
     // (qtensor.rs:385-398): activations quantised per row from x itself
     if (ctx->fast_int8 && w->fmt == UT_FMT_INT8 && M > 0)
         return matmul_fast_i8(ctx, w, out, ldo, accumulate, x, M);
+    DigitPlanes pl;
+    if (gemm_ok(w, M) && xdigits_planes(xd, w->in_dim, &pl))
+        return launch_gemm(ctx, w, pl, M, out, ldo, accumulate);
     GemvArgs ga;
     ga.w = w;
     ga.M = M;
@@ -1727,6 +1742,11 @@ int32_t matmul_dev(ut_ctx *ctx, const ut_qtensor *w, const float *x, int64_t M, 
     if (M <= 0) return UT_OK;
     if (ctx->fast_int8 && w->fmt == UT_FMT_INT8)
         return matmul_fast_i8(ctx, w, out, ldo, accumulate, x, M);
+    if (gemm_ok(w, M)) {
+        const DigitPlanes pl = planes_view(digit_scratch, M, w->in_dim);
+        UT_TRY(launch_planes(ctx, x, w->in_dim, M, w->in_dim, pl));
+        return launch_gemm(ctx, w, pl, M, out, ldo, accumulate);
+    }
     GemvArgs ga;
     ga.w = w;
     ga.M = M;
@@ -1777,6 +1797,13 @@ extern "C" int32_t ut_qtensor_matmul(ut_ctx *ctx, const ut_qtensor *qt, float *o
     // Int8 { .. } if fast_int8_enabled() (qtensor.rs:385-398)
     if (qt->fmt == UT_FMT_INT8 && ctx->fast_int8)
         return matmul_fast_i8(ctx, qt, out_dev, qt->out_dim, 0, x_dev, seq);
+    if (gemm_ok(qt, seq)) {
+        ScratchPlan plan;
+        plan.add(planes_bytes(seq, qt->in_dim));
+        std::vector<void *> ptrs;
+        UT_TRY(scratch_acquire(ctx, plan, ptrs));
+        return matmul_dev(ctx, qt, x_dev, seq, out_dev, qt->out_dim, 0, ptrs[0]);
+    }
     GemvArgs ga;
     ga.w = qt;
     ga.M = seq;

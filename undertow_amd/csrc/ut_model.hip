@@ -10,6 +10,7 @@
 #include <string>
 #include <unordered_map>
 
+#include "ut_gemm.h"
 #include "ut_mla.h"
 #include "ut_moe.h"
 #include "ut_ops.h"
@@ -521,16 +522,30 @@ int32_t mlp_rows_fast(ut_session *s, const MlpW &w, const float *x, int64_t rows
     return launch_check(ctx, "k_add_rows");
 }
 
-// Digit forms the given weights need from one shared activation.
-int dig_flags(std::initializer_list<const ut_qtensor *> ws) {
+// Digit forms the given weights need from one shared activation of `rows`
+// rows.  Rows for the GEMM (gemm_ok) come as base-256 digits where its
+// planes need no padding; otherwise proj() digitises the f32 rows itself.
+int dig_flags(std::initializer_list<const ut_qtensor *> ws, int64_t rows) {
     int f = 0;
     for (const ut_qtensor *w : ws) {
         if (!w || w->fmt == UT_FMT_F32) continue;
+        if (gemm_ok(w, rows)) {
+            if (planes_pitch(w->in_dim) == w->in_dim) f |= XD_DIG8;
+            continue;
+        }
         const bool fast = (w->fmt == UT_FMT_INT4 ? w->in_dim % 32 == 0 : w->in_dim % 16 == 0) &&
                           ((uintptr_t)w->payload & 15) == 0;
         f |= fast ? xdigit_flags_for(w->fmt, w->in_dim) : XD_XT;
     }
     return f;
+}
+
+// out = x . w^T for normed rows x (f32) with digits xd made for dig_flags.
+int32_t proj(ut_session *s, const ut_qtensor *w, const float *x, const XDigits &xd, int64_t rows,
+             float *out, int64_t ldo) {
+    if (gemm_ok(w, rows) && !(xd.dig8 && planes_pitch(w->in_dim) == w->in_dim))
+        return mm(s, w, x, rows, out, ldo);
+    return matmul_digits(s->ctx, w, x, xd, rows, out, ldo, 0);
 }
 
 // Whether any of the weights reads its activation as f32 (f32 weights:
@@ -816,7 +831,7 @@ int32_t mla_forward(ut_session *s, const LayerW &L, const float *x, const XDigit
     const int64_t qh = nope + rope;
     const float scale = 1.0f / sqrtf((float)qh);  // config.rs:142-144
     const int64_t pos_base = kv.len;
-    const bool pair = !fast8(s) && L.lora && L.kv_a->fmt == L.q_a->fmt && L.kv_a->fmt != UT_FMT_F32 &&
+    const bool pair = !fast8(s) && L.lora && !gemm_ok(L.kv_a, rows) && L.kv_a->fmt == L.q_a->fmt && L.kv_a->fmt != UT_FMT_F32 &&
                       L.kv_a->in_dim == L.q_a->in_dim && L.kv_a->row_bytes == L.q_a->row_bytes &&
                       gemv_fast_ok(L.kv_a) && gemv_fast_ok(L.q_a);
     // with the pair's split-K partials deferred, one launch finishes both
@@ -876,7 +891,7 @@ int32_t mla_forward(ut_session *s, const LayerW &L, const float *x, const XDigit
         if (fused) ga.defer = &pp;
         UT_TRY(gemv(ctx, ga));
     } else {
-        UT_TRY(matmul_digits(ctx, L.kv_a, x, xd, rows, w.comp, Lr + rope, 0));
+        UT_TRY(proj(s, L.kv_a, x, xd, rows, w.comp, Lr + rope));
     }
     // one row: q_b normalises q_a itself while staging it (the same digits
     // as the row digitiser's), so mla_pre only sums q_a's partials
@@ -899,7 +914,7 @@ int32_t mla_forward(ut_session *s, const LayerW &L, const float *x, const XDigit
         gq.norm_eps = c.rms_norm_eps;
         UT_TRY(gemv(ctx, gq));
     } else if (fused && pp.ks > 1) {
-        const int qf = dig_flags({L.q_b});
+        const int qf = dig_flags({L.q_b}, rows);
         const XDigits qd = xdigits_view(w.digB, rows, c.q_lora_rank, qf);
         UT_TRY(launch_mla_pre(ctx, pp, Lr + rope, xd.exps, L.kv_a->scales, L.q_a->scales, rows,
                               c.q_lora_rank, L.q_a_norm, c.rms_norm_eps,
@@ -908,13 +923,13 @@ int32_t mla_forward(ut_session *s, const LayerW &L, const float *x, const XDigit
         UT_TRY(matmul_digits(ctx, L.q_b, w.qa_n, qd, rows, w.q, heads * qh, 0));
     } else {
         if (L.lora) {
-            if (!pair) UT_TRY(matmul_digits(ctx, L.q_a, x, xd, rows, w.qa, c.q_lora_rank, 0));
+            if (!pair) UT_TRY(proj(s, L.q_a, x, xd, rows, w.qa, c.q_lora_rank));
             XDigits qd;
             UT_TRY(norm_dig(s, w.qa, c.q_lora_rank, L.q_a_norm, c.q_lora_rank, rows, w.qa_n,
-                            c.q_lora_rank, w.digB, dig_flags({L.q_b}), &qd));
-            UT_TRY(matmul_digits(ctx, L.q_b, w.qa_n, qd, rows, w.q, heads * qh, 0));
+                            c.q_lora_rank, w.digB, dig_flags({L.q_b}, rows), &qd));
+            UT_TRY(proj(s, L.q_b, w.qa_n, qd, rows, w.q, heads * qh));
         } else {
-            UT_TRY(matmul_digits(ctx, L.q_proj, x, xd, rows, w.q, heads * qh, 0));
+            UT_TRY(proj(s, L.q_proj, x, xd, rows, w.q, heads * qh));
         }
         UT_TRY(launch_kv_append(ctx, w.comp, rows, Lr, rope, L.kv_a_norm, c.rms_norm_eps,
                                 kv.latent, kv.krot, kv.kc, pos_base, m->rope_table));
@@ -982,7 +997,7 @@ NormNext next_norm(ut_session *s, const float *norm_w, int flags, int64_t rows, 
     return nx;
 }
 
-int input_flags(const LayerW &L) { return dig_flags({L.q_a, L.q_proj, L.kv_a}); }
+int input_flags(const LayerW &L, int64_t rows) { return dig_flags({L.q_a, L.q_proj, L.kv_a}, rows); }
 bool input_f32(const LayerW &L) { return f32_reader({L.q_a, L.q_proj, L.kv_a}); }
 
 // run_layer (model.rs:127-183) / the per-layer body of prefill (:470-526).
@@ -997,7 +1012,7 @@ int32_t run_layer(ut_session *s, const LayerW &L, float *x, int64_t rows, KvCach
     Workspace &w = s->ws;
     XDigits xd;
     if (pre) xd = *pre;
-    else UT_TRY(norm_dig(s, x, H, L.input_norm, H, rows, w.normed, H, w.digA, input_flags(L), &xd));
+    else UT_TRY(norm_dig(s, x, H, L.input_norm, H, rows, w.normed, H, w.digA, input_flags(L, rows), &xd));
     int f = 0;
     if (L.dense) f = dig_flags_fmt(L.mlp.fmt, H);
     else {
@@ -1088,7 +1103,7 @@ int32_t prefill_dev(ut_session *s, const int32_t *ids, int64_t n, const int32_t 
     const size_t nl = m->layers.size();
     const bool emb_norm = fuse && nl > 0 && embed_norm_ok(m->embed, H, w.x, m->layers[0].input_norm);
     if (emb_norm) {
-        const NormNext n0 = next_norm(s, m->layers[0].input_norm, input_flags(m->layers[0]), n,
+        const NormNext n0 = next_norm(s, m->layers[0].input_norm, input_flags(m->layers[0], n), n,
                                       &cur, input_f32(m->layers[0]));
         UT_TRY(launch_embed_norm(ctx, m->embed, ids_dev ? ids_dev : w.ids, n, w.x, H, n0));
     } else {
@@ -1098,9 +1113,9 @@ int32_t prefill_dev(ut_session *s, const int32_t *ids, int64_t n, const int32_t 
         NormNext nx;
         if (fuse)
             nx = li + 1 < nl ? next_norm(s, m->layers[li + 1].input_norm,
-                                         input_flags(m->layers[li + 1]), n, &nxt,
+                                         input_flags(m->layers[li + 1], n), n, &nxt,
                                          input_f32(m->layers[li + 1]))
-                             : next_norm(s, m->final_norm, dig_flags({m->lm_head}), n, &nxt,
+                             : next_norm(s, m->final_norm, dig_flags({m->lm_head}, n), n, &nxt,
                                          f32_reader({m->lm_head}));
         if (fuse && li + 1 == nl && m->has_mtp) {
             // the last combine also keeps the finished rows for the MTP head
@@ -1118,7 +1133,7 @@ int32_t prefill_dev(ut_session *s, const int32_t *ids, int64_t n, const int32_t 
     XDigits fd = cur;
     if (!fuse || nl == 0)
         UT_TRY(norm_dig(s, w.x, H, m->final_norm, H, n, w.normed, H, w.digA,
-                        dig_flags({m->lm_head}), &fd));
+                        dig_flags({m->lm_head}, n), &fd));
     // the argmax rows, then the sticky error word at am[n] and, with device
     // ids (a verify step), the rows' ids past the first (its drafts) at
     // am[n + 1 ...]: one readback carries them all
@@ -1127,7 +1142,7 @@ int32_t prefill_dev(ut_session *s, const int32_t *ids, int64_t n, const int32_t 
     if (n <= 4)
         return matmul_digits_argmax(ctx, m->lm_head, w.normed, fd, n, w.logits, w.am, w.argm,
                                     w.err, tail, ntail);
-    UT_TRY(matmul_digits(ctx, m->lm_head, w.normed, fd, n, w.logits, V, 0));
+    UT_TRY(proj(s, m->lm_head, w.normed, fd, n, w.logits, V));
     return launch_argmax(ctx, w.logits, n, V, V, w.am, w.argm, w.err, tail, ntail);
 }
 
@@ -1256,7 +1271,7 @@ int32_t draft_rows_dev(ut_session *s, const int32_t *host_ids, int in_slot,
         ga.exps_out = w.vexps;
         // the MTP layer's input norm in eh_proj's split sum where it can run
         if (fuse_next_ok(s, rows)) {
-            pre_nx = next_norm(s, m->mtp_layer.input_norm, input_flags(m->mtp_layer), rows, &pre_xd,
+            pre_nx = next_norm(s, m->mtp_layer.input_norm, input_flags(m->mtp_layer, rows), rows, &pre_xd,
                                input_f32(m->mtp_layer));
             ga.next = &pre_nx;
             ga.next_done = &pre_done;
@@ -1273,7 +1288,7 @@ int32_t draft_rows_dev(ut_session *s, const int32_t *host_ids, int in_slot,
     if (fuse_next_ok(s, rows)) {
         // the layer's last combine normalises every row; the head reads the last
         XDigits all;
-        const NormNext nx = next_norm(s, m->mtp_norm, dig_flags({m->mtp_head}), rows, &all,
+        const NormNext nx = next_norm(s, m->mtp_norm, dig_flags({m->mtp_head}, 1), rows, &all,
                                       f32_reader({m->mtp_head}));
         UT_TRY(run_layer(s, m->mtp_layer, w.x, rows, s->mtp_kv, pre_done ? &pre_xd : nullptr, &nx));
         hd_ = xdigits_rows(all, rows - 1);
@@ -1281,7 +1296,7 @@ int32_t draft_rows_dev(ut_session *s, const int32_t *host_ids, int in_slot,
     } else {
         UT_TRY(run_layer(s, m->mtp_layer, w.x, rows, s->mtp_kv));
         UT_TRY(norm_dig(s, w.x + (rows - 1) * H, H, m->mtp_norm, H, 1, w.normed, H, w.digA,
-                        dig_flags({m->mtp_head}), &hd_));
+                        dig_flags({m->mtp_head}, 1), &hd_));
     }
     return matmul_digits_argmax(ctx, m->mtp_head, hn, hd_, 1, w.logits, draft_dev, w.argm, nullptr);
 }
