@@ -22,6 +22,17 @@ int32_t launch_planes(ut_ctx *ctx, const float *x, int64_t ldx, int64_t M, int64
                       const DigitPlanes &pl);
 int32_t launch_planes(ut_ctx *ctx, const uint16_t *x, int64_t ldx, int64_t M, int64_t K,
                       const DigitPlanes &pl);
+// Digitises h = silu(g) * u of M rows [M, I].
+int32_t launch_silu_planes(ut_ctx *ctx, const float *g, const float *u, int64_t M, int64_t I,
+                           const DigitPlanes &pl);
+// A batch's base-256 digits are the GEMM's planes where rows need no padding.
+inline bool xdigits_planes(const XDigits &xd, int64_t K, DigitPlanes *pl) {
+    if (!xd.dig8 || planes_pitch(K) != K || ((uintptr_t)xd.dig8 & 15)) return false;
+    pl->p = (int8_t *)xd.dig8;
+    pl->kp = K;
+    pl->exps = xd.exps;
+    return true;
+}
 
 // The fewest rows that take the matrix-core GEMM; four-row GEMV passes over
 // the weight are slower from the second pass on (five rows, GEMV passes

@@ -19,40 +19,65 @@ DigitPlanes planes_view(void *base, int64_t M, int64_t K) {
     return d;
 }
 
-__device__ __forceinline__ float plane_value(const float *x, int64_t k) { return x[k]; }
-__device__ __forceinline__ float plane_value(const uint16_t *x, int64_t k) {
-    return __uint_as_float((uint32_t)x[k] << 16);
-}
-__device__ __forceinline__ void plane_load4(const float *x, int64_t k, float (&v)[4]) {
-    const float4 f = ld_global<float4>(x + k);
-    v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w;
-}
-__device__ __forceinline__ void plane_load4(const uint16_t *x, int64_t k, float (&v)[4]) {
-    const uint2 u = ld_global<uint2>(x + k);
-    v[0] = __uint_as_float(u.x << 16); v[1] = __uint_as_float(u.x & 0xffff0000u);
-    v[2] = __uint_as_float(u.y << 16); v[3] = __uint_as_float(u.y & 0xffff0000u);
-}
+// A row's values: f32, bf16 (widened), or silu(g) * u of an MLP's two halves
+// (undertow-quant/src/lib.rs:121; model.rs:241-247).
+struct RowF32 {
+    const float *x;
+    int64_t ld;
+    __device__ __forceinline__ float at(int64_t m, int64_t k) const { return x[m * ld + k]; }
+    __device__ __forceinline__ void at4(int64_t m, int64_t k, float (&v)[4]) const {
+        const float4 f = ld_global<float4>(x + m * ld + k);
+        v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w;
+    }
+    bool vec() const { return ((uintptr_t)x & 15) == 0 && ld % 4 == 0; }
+};
+struct RowBf16 {
+    const uint16_t *x;
+    int64_t ld;
+    __device__ __forceinline__ float at(int64_t m, int64_t k) const {
+        return __uint_as_float((uint32_t)x[m * ld + k] << 16);
+    }
+    __device__ __forceinline__ void at4(int64_t m, int64_t k, float (&v)[4]) const {
+        const uint2 u = ld_global<uint2>(x + m * ld + k);
+        v[0] = __uint_as_float(u.x << 16); v[1] = __uint_as_float(u.x & 0xffff0000u);
+        v[2] = __uint_as_float(u.y << 16); v[3] = __uint_as_float(u.y & 0xffff0000u);
+    }
+    bool vec() const { return ((uintptr_t)x & 7) == 0 && ld % 4 == 0; }
+};
+struct RowSilu {
+    const float *g, *u;
+    int64_t ld;
+    static __device__ __forceinline__ float h(float g, float u) {
+        return __fmul_rn(g / (1.0f + expf(-g)), u);
+    }
+    __device__ __forceinline__ float at(int64_t m, int64_t k) const {
+        return h(g[m * ld + k], u[m * ld + k]);
+    }
+    __device__ __forceinline__ void at4(int64_t m, int64_t k, float (&v)[4]) const {
+        const float4 a = ld_global<float4>(g + m * ld + k), b = ld_global<float4>(u + m * ld + k);
+        v[0] = h(a.x, b.x); v[1] = h(a.y, b.y); v[2] = h(a.z, b.z); v[3] = h(a.w, b.w);
+    }
+    bool vec() const { return (((uintptr_t)g | (uintptr_t)u) & 15) == 0 && ld % 4 == 0; }
+};
 
 // One workgroup per row: max|x|, exponent, then four columns a time into
-// one word per plane.  Rows of up to kPlaneRegs * 1024 columns stay in
+// one word per plane.  The first kPlaneRegs * 1024 columns stay in
 // registers between the two passes.  Bound by the row's read: one round
 // trip (512 rows of 16,384 columns: 33.5 MB in, 25 MB out).
 constexpr int kPlaneRegs = 8;
-template <typename T, bool VEC>
-__global__ __launch_bounds__(256) void k_planes(const T *__restrict__ x, int64_t ldx, int64_t K,
-                                                int8_t *__restrict__ pl, int64_t kp,
-                                                int32_t *__restrict__ exps) {
+template <typename Row, bool VEC>
+__global__ __launch_bounds__(256) void k_planes(Row row, int64_t K, int8_t *__restrict__ pl,
+                                                int64_t kp, int32_t *__restrict__ exps) {
     __shared__ uint32_t red[4];
     const int64_t m = blockIdx.x;
     const int tid = threadIdx.x;
-    const T *xr = x + m * ldx;
     float v[kPlaneRegs][4];
     auto load = [&](int64_t c, float (&o)[4]) {
         if (VEC && c + 4 <= K) {
-            plane_load4(xr, c, o);
+            row.at4(m, c, o);
         } else {
 #pragma unroll
-            for (int j = 0; j < 4; j++) o[j] = c + j < K ? plane_value(xr, c + j) : 0.0f;
+            for (int j = 0; j < 4; j++) o[j] = c + j < K ? row.at(m, c + j) : 0.0f;
         }
     };
     uint32_t mx = 0;
@@ -97,28 +122,31 @@ __global__ __launch_bounds__(256) void k_planes(const T *__restrict__ x, int64_t
     }
 }
 
-template <typename T>
-static int32_t planes_t(ut_ctx *ctx, const T *x, int64_t ldx, int64_t M, int64_t K,
+template <typename Row>
+static int32_t planes_t(ut_ctx *ctx, const char *name, const Row &row, int64_t M, int64_t K,
                         const DigitPlanes &pl) {
     if (M <= 0) return UT_OK;
-    const bool vec = ((uintptr_t)x % (4 * sizeof(T))) == 0 && ldx % 4 == 0;
-    int tok = timing_begin(ctx, "planes");
-    if (vec)
-        hipLaunchKernelGGL((k_planes<T, true>), dim3((unsigned)M), dim3(256), 0, ctx->stream, x, ldx,
+    int tok = timing_begin(ctx, name);
+    if (row.vec())
+        hipLaunchKernelGGL((k_planes<Row, true>), dim3((unsigned)M), dim3(256), 0, ctx->stream, row,
                            K, pl.p, pl.kp, pl.exps);
     else
-        hipLaunchKernelGGL((k_planes<T, false>), dim3((unsigned)M), dim3(256), 0, ctx->stream, x,
-                           ldx, K, pl.p, pl.kp, pl.exps);
+        hipLaunchKernelGGL((k_planes<Row, false>), dim3((unsigned)M), dim3(256), 0, ctx->stream, row,
+                           K, pl.p, pl.kp, pl.exps);
     timing_end(ctx, tok);
     return launch_check(ctx, "k_planes");
 }
 int32_t launch_planes(ut_ctx *ctx, const float *x, int64_t ldx, int64_t M, int64_t K,
                       const DigitPlanes &pl) {
-    return planes_t(ctx, x, ldx, M, K, pl);
+    return planes_t(ctx, "planes", RowF32{x, ldx}, M, K, pl);
 }
 int32_t launch_planes(ut_ctx *ctx, const uint16_t *x, int64_t ldx, int64_t M, int64_t K,
                       const DigitPlanes &pl) {
-    return planes_t(ctx, x, ldx, M, K, pl);
+    return planes_t(ctx, "planes", RowBf16{x, ldx}, M, K, pl);
+}
+int32_t launch_silu_planes(ut_ctx *ctx, const float *g, const float *u, int64_t M, int64_t I,
+                           const DigitPlanes &pl) {
+    return planes_t(ctx, "silu_planes", RowSilu{g, u, I}, M, I, pl);
 }
 
 // --------------------------------------------------------------- GEMM ---

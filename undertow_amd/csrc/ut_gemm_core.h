@@ -13,8 +13,8 @@
 // piece of one row); only the digit planes, which all four waves read, go
 // through LDS: at TO = 4 each digit fragment read feeds four matrix
 // instructions, so LDS runs at half the matrix cores' time.  Both are
-// fetched a step of 128 columns ahead; the barrier waits for LDS only, so
-// the weight loads stay in flight across it.  LDS rows of 128 bytes keep
+// fetched a step of 128 columns ahead; the barrier waits for LDS only, so the
+// loads stay in flight across it.  LDS rows of 128 bytes keep
 // their 16-byte chunks XOR-swizzled by the row's low three bits: eight lanes
 // that read one chunk of eight rows use all 32 banks.
 #pragma once
@@ -101,13 +101,18 @@ template <int FMT> __device__ __forceinline__ int32_t gemm_exp(int32_t e) {
     return FMT == UT_FMT_INT4 && e != INT32_MIN ? e - 4 : e;
 }
 
-// acc[t][n][p] += tile over columns [kb, ke) (kb a multiple of 128, columns
+// acc[t][n][p] = tile over columns [kb, ke) (kb a multiple of 128, columns
 // past K zero in the planes).  src[i]: the digit bytes of this thread's
-// staging chunk i at column 0 (its chunk offset included).
-template <int FMT, int TO, int TM, bool UNAL>
+// staging chunk i at column 0 (its chunk offset included).  D (even): steps
+// held in registers, D - 1 of them in flight while one computes.  Four
+// measured no better than two at 5 to 64 rows (int8 7168 x 16384 at 5 rows
+// 44.2 against 43.7 us) and worse at 512 (int4 18432 x 7168 272 against
+// 260 us).
+template <int FMT, int TO, int TM, bool UNAL, int D = 2>
 __device__ __forceinline__ void gemm_tile(const GemmRows<TO> &rows, int64_t len, int64_t kb,
                                           int64_t ke, const int8_t *const (&src)[gemm_stage_n<TM>()],
                                           uint4 *lds, ut_i32x4 (&acc)[TO][TM][3]) {
+    static_assert(D % 2 == 0, "the LDS buffer of a step is its slot's parity");
     constexpr int NB = gemm_stage_n<TM>(), CH = TM * 48 * 8;
     const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, q = lane >> 4;
 #pragma unroll
@@ -116,56 +121,58 @@ __device__ __forceinline__ void gemm_tile(const GemmRows<TO> &rows, int64_t len,
         for (int n = 0; n < TM; n++)
 #pragma unroll
             for (int p = 0; p < 3; p++) acc[t][n][p] = ut_i32x4{0, 0, 0, 0};
-    uint4 b[NB];
-    auto load_b = [&](int64_t k) {
+    GemmA<FMT, TO> a[D];
+    uint4 b[D][NB];
+    const int n = (int)((ke - kb + kGemmStep - 1) / kGemmStep);
+    auto load = [&](int d, int i) {
+        const int64_t k = kb + (int64_t)i * kGemmStep;
 #pragma unroll
-        for (int i = 0; i < NB; i++)
-            if (tid + i * kGemmThreads < CH) b[i] = ld_global<uint4>(src[i] + k);
+        for (int j = 0; j < NB; j++)
+            if (tid + j * kGemmThreads < CH) b[d][j] = ld_global<uint4>(src[j] + k);
+        gemm_load_a<FMT, TO, UNAL>(a[d], rows, k, len, q);
     };
-    auto store_b = [&](uint4 *dst) {
+    auto store_b = [&](int d, int buf) {
 #pragma unroll
-        for (int i = 0; i < NB; i++)
-            if (tid + i * kGemmThreads < CH) dst[tid + i * kGemmThreads] = b[i];
+        for (int j = 0; j < NB; j++)
+            if (tid + j * kGemmThreads < CH) lds[buf * CH + tid + j * kGemmThreads] = b[d][j];
     };
-    auto compute = [&](const GemmA<FMT, TO> &a, const uint4 *buf) {
+    auto compute = [&](const GemmA<FMT, TO> &av, const uint4 *buf) {
 #pragma unroll
         for (int s = 0; s < 2; s++) {
             const int chunk = (FMT == UT_FMT_INT8 ? 4 * s + q : 2 * q + s) ^ (r & 7);
             ut_i32x4 f[TO];
 #pragma unroll
-            for (int t = 0; t < TO; t++) f[t] = gemm_frag_a<FMT, TO>(a, t, s);
+            for (int t = 0; t < TO; t++) f[t] = gemm_frag_a<FMT, TO>(av, t, s);
 #pragma unroll
-            for (int n = 0; n < TM; n++)
+            for (int m = 0; m < TM; m++)
 #pragma unroll
                 for (int p = 0; p < 3; p++) {
-                    const uint4 v = buf[((n * 3 + p) * 16 + r) * 8 + chunk];
+                    const uint4 v = buf[((m * 3 + p) * 16 + r) * 8 + chunk];
                     const ut_i32x4 w{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
 #pragma unroll
                     for (int t = 0; t < TO; t++)
-                        acc[t][n][p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(f[t], w, acc[t][n][p], 0, 0, 0);
+                        acc[t][m][p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(f[t], w, acc[t][m][p], 0, 0, 0);
                 }
         }
     };
+    // LDS-only barrier: the loads of later steps stay in flight across it
     auto barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-    GemmA<FMT, TO> cur, nxt;
-    load_b(kb);
-    gemm_load_a<FMT, TO, UNAL>(cur, rows, kb, len, q);
-    store_b(lds);
+#pragma unroll
+    for (int d = 0; d < D; d++)
+        if (d < n) load(d, d);
+    store_b(0, 0);
     barrier();
-    int o = 0;
-    for (int64_t k = kb; k < ke; k += kGemmStep) {
-        const bool more = k + kGemmStep < ke;
-        if (more) {
-            load_b(k + kGemmStep);
-            gemm_load_a<FMT, TO, UNAL>(nxt, rows, k + kGemmStep, len, q);
+    for (int base = 0; base < n; base += D) {
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+            const int i = base + d;
+            if (i < n) {
+                compute(a[d], lds + (d & 1) * CH);
+                if (i + 1 < n) store_b((d + 1) % D, (d + 1) & 1);
+                if (i + D < n) load(d, i + D);
+                barrier();
+            }
         }
-        compute(cur, lds + o);
-        o = CH - o;
-        if (more) {
-            store_b(lds + o);
-            cur = nxt;
-        }
-        barrier();
     }
 }
 

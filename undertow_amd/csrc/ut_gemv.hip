@@ -1581,15 +1581,6 @@ size_t matmul_digit_bytes(int64_t M, int64_t K) {
     return b > p ? b : p;
 }
 
-// A batch's base-256 digits are the GEMM's planes where rows need no padding.
-static bool xdigits_planes(const XDigits &xd, int64_t K, DigitPlanes *pl) {
-    if (!xd.dig8 || planes_pitch(K) != K || ((uintptr_t)xd.dig8 & 15)) return false;
-    pl->p = (int8_t *)xd.dig8;
-    pl->kp = K;
-    pl->exps = xd.exps;
-    return true;
-}
-
 // ------------------------------------------------------ fast int8 ---
 // The opt-in fast-int8 path (undertow-quant/src/lib.rs:31-59,
 // avx512.rs:221-242).  k_act_quant_i8: one workgroup per activation row,

@@ -13,6 +13,7 @@
 #include "ut_gemm.h"
 #include "ut_mla.h"
 #include "ut_moe.h"
+#include "ut_moe_rows.h"
 #include "ut_ops.h"
 #include "ut_safetensors.h"
 #include "ut_sample.h"
@@ -112,6 +113,10 @@ struct Workspace {
     void *digits = nullptr, *moe = nullptr, *mla = nullptr, *argm = nullptr;
     void *digA = nullptr, *digB = nullptr;  // activation digits shared by consumers
     float *fast = nullptr;  // the fast-int8 path's MLP rows
+    // more than four rows: an MLP's two halves, and the grouped experts'
+    // scratch (moe_rows_bytes)
+    float *mlp_g = nullptr, *mlp_u = nullptr;
+    void *moe_rows = nullptr;
 };
 
 }  // namespace
@@ -381,7 +386,7 @@ int32_t ws_reserve(ut_session *s, int64_t rows) {
     size_t iqabs = F(R * heads * Lr), iqrope = F(R * heads * c.qk_rope_head_dim + 1);
     size_t iclat = F(R * heads * Lr), ictx = F(R * heads * c.v_head_dim);
     size_t ilog = F(R * c.vocab_size), iemb = F(R * H), icat = F(R * 2 * H);
-    size_t irl = F(4 * E), irw = F(4 * k), irid = F(4 * k), iids = F(R), iam = F(2 * R + 1), ierr = F(1);
+    size_t irl = F(R * E), irw = F(R * k), irid = F(R * k), iids = F(R), iam = F(2 * R + 1), ierr = F(1);
     size_t ivids = F(8);
     size_t ivmax = F(R * absorb_v_parts(heads, c.v_head_dim)), ivexp = F(R);
     size_t idig = plan.add(matmul_digit_bytes(R, kmax));
@@ -394,6 +399,13 @@ int32_t ws_reserve(ut_session *s, int64_t rows) {
     // up, h [4][max inter], the choices' outputs [4][k][H] and a shared
     // MLP's [4][H]
     size_t ifast = F(3 * 4 * max_inter(m) + 4 * (k > 0 ? k : 1) * H + 4 * H);
+    size_t img = 0, imu = 0, imr = 0;
+    if (R > 4) {
+        img = F(R * max_inter(m));
+        imu = F(R * max_inter(m));
+        const int64_t kk = k > 0 ? k : 1, ch = moe_rows_chunk(kk);
+        imr = plan.add(moe_rows_bytes(R < ch ? R : ch, kk, E > 0 ? E : 1, H, c.moe_intermediate_size, true));
+    }
     size_t total = 0;
     for (size_t b : plan.sizes) total += b;
     if (w.base) {
@@ -437,6 +449,11 @@ int32_t ws_reserve(ut_session *s, int64_t rows) {
     w.digits = p[idig]; w.moe = p[imoes]; w.mla = p[imla]; w.argm = p[iarg];
     w.digA = p[idA]; w.digB = p[idB];
     w.fast = (float *)p[ifast];
+    if (R > 4) {
+        w.mlp_g = (float *)p[img];
+        w.mlp_u = (float *)p[imu];
+        w.moe_rows = p[imr];
+    }
     w.rows = R;
     UT_CHECK_HIP(ctx, hipMemsetAsync(w.err, 0, 4, ctx->stream));
     return UT_OK;
@@ -569,6 +586,30 @@ int32_t norm_dig(ut_session *s, const float *x, int64_t ldx, const float *w, int
     *xd = xdigits_view(buf, rows, n, flags);
     return launch_rmsnorm_digitize(s->ctx, x, ldx, rows, n, w, c.rms_norm_eps, out, ldo, *xd,
                                    flags);
+}
+
+// Whether an MLP's rows run as three products over all rows (mlp_rows).
+bool mlp_gemm_ok(const ut_session *s, const MlpW &w, int64_t rows) {
+    return !fast8(s) && gemm_ok(w.gate, rows) && gemm_ok(w.up, rows) && gemm_ok(w.down, rows);
+}
+
+// An MLP over rows of normed x (digits xd made for it where they need no
+// padding) as the products gate and up, h = silu(g) * u digitised, and down:
+// out (+)= down(h).
+int32_t mlp_rows(ut_session *s, const MlpW &w, const float *x, const XDigits &xd, int64_t rows,
+                 float *out, int accumulate) {
+    ut_ctx *ctx = s->ctx;
+    const int64_t H = hd(s->m), I = w.inter;
+    DigitPlanes pl;
+    if (!xdigits_planes(xd, H, &pl)) {
+        pl = planes_view(s->ws.digits, rows, H);
+        UT_TRY(launch_planes(ctx, x, H, rows, H, pl));
+    }
+    UT_TRY(launch_gemm(ctx, w.gate, pl, rows, s->ws.mlp_g, I, 0));
+    UT_TRY(launch_gemm(ctx, w.up, pl, rows, s->ws.mlp_u, I, 0));
+    const DigitPlanes hp = planes_view(s->ws.digits, rows, I);
+    UT_TRY(launch_silu_planes(ctx, s->ws.mlp_g, s->ws.mlp_u, rows, I, hp));
+    return launch_gemm(ctx, w.down, hp, rows, out, H, accumulate);
 }
 
 // An MLP (dense FFN or shared expert) over rows, added into out
@@ -755,6 +796,67 @@ int32_t moe_forward(ut_session *s, const LayerW &L, const float *x, const XDigit
         }
         mc.next = next;
         UT_TRY(moe_pass(s->ctx, mc, s->ws.moe));
+    }
+    return UT_OK;
+}
+
+// Whether a MoE layer's rows run as grouped products (moe_forward_rows).
+bool moe_gemm_ok(const ut_session *s, const LayerW &L, int64_t rows) {
+    const ut_model_config &c = s->m->c;
+    return !fast8(s) && !s->m->store &&
+           moe_rows_ok(L.expert_fmt, rows, c.n_routed_experts, c.hidden_size,
+                       c.moe_intermediate_size) &&
+           (!L.has_shared || mlp_gemm_ok(s, L.shared, rows));
+}
+
+// moe_forward (model.rs:195-286) over a prompt's rows of normed x (digits
+// xd), added with the shared expert into out (the residual): all rows routed
+// at once and every expert's weights read once for the rows that chose it.
+int32_t moe_forward_rows(ut_session *s, const LayerW &L, const float *x, const XDigits &xd,
+                         int64_t rows, float *out) {
+    ut_model *m = s->m;
+    ut_ctx *ctx = s->ctx;
+    const ut_model_config &c = m->c;
+    Workspace &w = s->ws;
+    const int64_t H = c.hidden_size, E = c.n_routed_experts, k = c.num_experts_per_tok;
+    for (int64_t s0 = 0; s0 < rows; s0 += 4) {
+        const int64_t M = rows - s0 < 4 ? rows - s0 : 4;
+        if (rowdot_f32_ok(L.gate, M) && ((uintptr_t)(x + s0 * H) & 15) == 0)
+            UT_TRY(launch_rowdot_f32(ctx, L.gate, x + s0 * H, M, w.rlogits + s0 * E, E));
+        else
+            UT_TRY(mm(s, L.gate, x + s0 * H, M, w.rlogits + s0 * E, E));
+    }
+    UT_TRY(launch_route(ctx, w.rlogits, L.bias, rows, E, (int)k, (int)c.n_group, (int)c.topk_group,
+                        c.norm_topk_prob, c.routed_scaling_factor, w.rids, w.rw));
+    if (L.has_shared) UT_TRY(mlp_rows(s, L.shared, x, xd, rows, w.moe_out, 0));
+    DigitPlanes pl;
+    const bool have = xdigits_planes(xd, H, &pl);
+    const int64_t chunk = moe_rows_chunk(k);
+    for (int64_t s0 = 0; s0 < rows; s0 += chunk) {
+        MoeRows r;
+        r.fmt = L.expert_fmt;
+        r.tbl = L.experts;
+        r.E = E;
+        r.H = H;
+        r.I = c.moe_intermediate_size;
+        r.M = rows - s0 < chunk ? rows - s0 : chunk;
+        r.k = (int)k;
+        r.ids = w.rids + s0 * k;
+        r.weights = w.rw + s0 * k;
+        DigitPlanes pr = pl;
+        if (have) {
+            pr.p += s0 * 3 * pl.kp;
+            pr.exps += s0;
+            r.planes = &pr;
+        } else {
+            r.x = x + s0 * H;
+        }
+        r.shared = L.has_shared ? w.moe_out + s0 * H : nullptr;
+        r.out = out + s0 * H;
+        r.ldo = H;
+        r.accumulate = 1;
+        r.err_flag = w.err;
+        UT_TRY(launch_moe_rows(ctx, r, w.moe_rows));
     }
     return UT_OK;
 }
@@ -1013,8 +1115,11 @@ int32_t run_layer(ut_session *s, const LayerW &L, float *x, int64_t rows, KvCach
     XDigits xd;
     if (pre) xd = *pre;
     else UT_TRY(norm_dig(s, x, H, L.input_norm, H, rows, w.normed, H, w.digA, input_flags(L, rows), &xd));
+    // a prompt's rows: the MLPs as products, the experts as grouped products
+    const bool big = L.dense ? mlp_gemm_ok(s, L.mlp, rows) : moe_gemm_ok(s, L, rows);
     int f = 0;
-    if (L.dense) f = dig_flags_fmt(L.mlp.fmt, H);
+    if (big) f = planes_pitch(H) == H ? XD_DIG8 : 0;
+    else if (L.dense) f = dig_flags_fmt(L.mlp.fmt, H);
     else {
         f = dig_flags_fmt(L.expert_fmt, H);
         if (L.has_shared) f |= dig_flags_fmt(L.shared.fmt, H);
@@ -1028,6 +1133,9 @@ int32_t run_layer(ut_session *s, const LayerW &L, float *x, int64_t rows, KvCach
                        &post_done));
     if (post_done) xd = pd;
     else UT_TRY(norm_dig(s, x, H, L.post_norm, H, rows, w.normed, H, w.digA, f, &xd));
+    if (big)
+        return L.dense ? mlp_rows(s, L.mlp, w.normed, xd, rows, x, 1)
+                       : moe_forward_rows(s, L, w.normed, xd, rows, x);
     if (L.dense) return mlp_add(s, L.mlp, w.normed, xd, rows, x, nullptr, next);
     if (fast8(s)) return moe_forward_fast(s, L, w.normed, rows, x);
     // x += (routed + shared) (model.rs:282-284 then the residual add)

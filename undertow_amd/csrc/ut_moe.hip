@@ -25,6 +25,7 @@
 #include <mutex>
 #include "ut_gemv_core.h"
 #include "ut_moe.h"
+#include "ut_moe_rows.h"
 #include "ut_gemv_mfma.h"
 #include "ut_rowdig.h"
 #include "ut_ops.h"
@@ -2347,14 +2348,62 @@ void ut_expert_table_free(ut_expert_table *t) {
 
 namespace {
 
+// Rows already routed in calls of the grouped products (moe_rows_chunk rows
+// each); *done: the rows finished so.  Nothing is done where the path does
+// not take the shape, where its scratch cannot be had, or where it would
+// have to grow while the stream is captured: the four-row passes then run,
+// with the same results.
+int32_t moe_experts_grouped(ut_ctx *ctx, const ut_expert_table *tbl, const int32_t *ids_dev,
+                            const float *weights_dev, int64_t rows, int32_t top_k,
+                            const float *x_dev, const uint16_t *xh_dev, float *out_dev,
+                            int32_t *flag, int64_t *done) {
+    *done = 0;
+    const int64_t H = tbl->hidden, chunk = moe_rows_chunk(top_k);
+    if (!moe_rows_ok(tbl->fmt, rows, tbl->n, H, tbl->inter)) return UT_OK;
+    ScratchPlan plan;
+    plan.add(moe_rows_bytes(rows < chunk ? rows : chunk, top_k, tbl->n, H, tbl->inter, true));
+    if (plan.sizes[0] > ctx->scratch.bytes) {
+        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(ctx->stream, &st) != hipSuccess) {
+            (void)hipGetLastError();
+            return UT_OK;
+        }
+        if (st != hipStreamCaptureStatusNone) return UT_OK;
+    }
+    std::vector<void *> ptrs;
+    const int32_t rc = scratch_acquire(ctx, plan, ptrs);
+    if (rc == UT_ERR_OOM) return UT_OK;
+    UT_TRY(rc);
+    for (int64_t s0 = 0; rows - s0 >= kGemmMinRows; s0 = *done) {
+        MoeRows c;
+        c.fmt = tbl->fmt;
+        c.tbl = tbl->ptrs;
+        c.E = tbl->n;
+        c.H = H;
+        c.I = tbl->inter;
+        c.M = rows - s0 < chunk ? rows - s0 : chunk;
+        c.k = top_k;
+        c.ids = ids_dev + s0 * top_k;
+        c.weights = weights_dev + s0 * top_k;
+        if (xh_dev) c.xh = xh_dev + s0 * H;
+        else c.x = x_dev + s0 * H;
+        c.out = out_dev + s0 * H;
+        c.ldo = H;
+        c.err_flag = flag;
+        UT_TRY(launch_moe_rows(ctx, c, ptrs[0]));
+        *done = s0 + c.M;
+    }
+    return UT_OK;
+}
+
 // The routed-expert block over rows already routed, in passes of up to four
 // rows, with `scratch` (moe_layout's bytes at four rows) as working memory.
 int32_t moe_experts_rows(ut_ctx *ctx, const ut_expert_table *tbl, const int32_t *ids_dev,
                          const float *weights_dev, int64_t rows, int32_t top_k, const float *x_dev,
                          float *out_dev, void *scratch, int32_t *flag,
-                         const uint16_t *xh_dev = nullptr) {
+                         const uint16_t *xh_dev = nullptr, int64_t first = 0) {
     const int64_t maxM = 4;
-    for (int64_t s0 = 0; s0 < rows; s0 += maxM) {
+    for (int64_t s0 = first; s0 < rows; s0 += maxM) {
         MoeCall c;
         c.fmt = tbl->fmt;
         c.tbl = tbl->ptrs;
@@ -2375,6 +2424,26 @@ int32_t moe_experts_rows(ut_ctx *ctx, const ut_expert_table *tbl, const int32_t 
         UT_TRY(moe_pass(ctx, c, scratch));
     }
     return UT_OK;
+}
+
+// Rows already routed, f32 (x_dev) or bf16 (xh_dev) activations.
+int32_t moe_experts_any(ut_ctx *ctx, const ut_expert_table *tbl, const int32_t *ids_dev,
+                        const float *weights_dev, int64_t rows, int32_t top_k, const float *x_dev,
+                        const uint16_t *xh_dev, float *out_dev) {
+    int32_t *flag = nullptr;
+    UT_TRY(device_error_flag(ctx, &flag));
+    int64_t done = 0;
+    UT_TRY(moe_experts_grouped(ctx, tbl, ids_dev, weights_dev, rows, top_k, x_dev, xh_dev, out_dev,
+                               flag, &done));
+    if (done == rows) return UT_OK;
+    const int64_t maxM = 4;
+    const int64_t slots = moe_slots((int)maxM, top_k, tbl->n, -1);
+    ScratchPlan plan;
+    plan.add(moe_layout(maxM, top_k, slots, tbl->hidden, tbl->inter, tbl->fmt).total);
+    std::vector<void *> ptrs;
+    UT_TRY(scratch_acquire(ctx, plan, ptrs));
+    return moe_experts_rows(ctx, tbl, ids_dev, weights_dev, rows, top_k, x_dev, out_dev, ptrs[0],
+                            flag, xh_dev, done);
 }
 
 // bf16 activations are read 8 bytes (four values) at a time: 16-byte
@@ -2462,16 +2531,7 @@ int32_t ut_moe_experts(ut_ctx *ctx, const ut_expert_table *tbl, const int32_t *i
     UT_TRY(moe_experts_check(ctx, "ut_moe_experts", tbl, ids_dev, weights_dev, rows, top_k, x_dev,
                              out_dev));
     if (rows == 0) return UT_OK;
-    const int64_t maxM = 4;
-    const int64_t slots = moe_slots((int)maxM, top_k, tbl->n, -1);
-    ScratchPlan plan;
-    plan.add(moe_layout(maxM, top_k, slots, tbl->hidden, tbl->inter, tbl->fmt).total);
-    std::vector<void *> ptrs;
-    UT_TRY(scratch_acquire(ctx, plan, ptrs));
-    int32_t *flag = nullptr;
-    UT_TRY(device_error_flag(ctx, &flag));
-    return moe_experts_rows(ctx, tbl, ids_dev, weights_dev, rows, top_k, x_dev, out_dev, ptrs[0],
-                            flag);
+    return moe_experts_any(ctx, tbl, ids_dev, weights_dev, rows, top_k, x_dev, nullptr, out_dev);
 }
 
 int32_t ut_moe_experts_noalloc(ut_ctx *ctx, const ut_expert_table *tbl, const int32_t *ids_dev,
@@ -2532,6 +2592,12 @@ int32_t moe_route_experts_any(ut_ctx *ctx, const char *fn, const ut_expert_table
     if (xh_dev && !bf16_rows_ok(ctx, fn, xh_dev, tbl->hidden)) return UT_ERR_ARG;
     if (rows == 0) return UT_OK;
     const int64_t maxM = 4;
+    if (rows > maxM) {
+        // every row routed in one launch, then the experts of all rows
+        UT_TRY(launch_route(ctx, logits_dev, bias_dev, rows, tbl->n, top_k, n_group, topk_group,
+                            norm_topk_prob, routed_scaling_factor, ids_dev, weights_dev));
+        return moe_experts_any(ctx, tbl, ids_dev, weights_dev, rows, top_k, x_dev, xh_dev, out_dev);
+    }
     const int64_t slots = moe_slots((int)maxM, top_k, tbl->n, -1);
     ScratchPlan plan;
     plan.add(moe_layout(maxM, top_k, slots, tbl->hidden, tbl->inter, tbl->fmt).total);
@@ -2539,37 +2605,34 @@ int32_t moe_route_experts_any(ut_ctx *ctx, const char *fn, const ut_expert_table
     UT_TRY(scratch_acquire(ctx, plan, ptrs));
     int32_t *flag = nullptr;
     UT_TRY(device_error_flag(ctx, &flag));
-    for (int64_t s0 = 0; s0 < rows; s0 += maxM) {
-        MoeCall c;
-        c.fmt = tbl->fmt;
-        c.tbl = tbl->ptrs;
-        c.E = tbl->n;
-        c.H = tbl->hidden;
-        c.I = tbl->inter;
-        c.M = (int)((rows - s0) < maxM ? (rows - s0) : maxM);
-        c.k = top_k;
-        // the choices: routed inside the gate/up launch where that applies
-        // (one row, the one-wave router), else by a route launch first
-        c.route_logits = logits_dev + s0 * tbl->n;
-        c.route_bias = bias_dev;
-        c.route_ng = n_group;
-        c.route_tg = topk_group;
-        c.route_norm = norm_topk_prob;
-        c.route_scale = routed_scaling_factor;
-        c.route_ids = ids_dev + s0 * top_k;
-        c.route_w = weights_dev + s0 * top_k;
-        c.ids = c.route_ids;
-        c.weights = c.route_w;
-        if (xh_dev)
-            c.xh = xh_dev + s0 * tbl->hidden;
-        else
-            c.x = x_dev + s0 * tbl->hidden;
-        c.out = out_dev + s0 * tbl->hidden;
-        c.ldo = tbl->hidden;
-        c.err_flag = flag;
-        UT_TRY(moe_pass(ctx, c, ptrs[0]));
-    }
-    return UT_OK;
+    MoeCall c;
+    c.fmt = tbl->fmt;
+    c.tbl = tbl->ptrs;
+    c.E = tbl->n;
+    c.H = tbl->hidden;
+    c.I = tbl->inter;
+    c.M = (int)rows;
+    c.k = top_k;
+    // the choices: routed inside the gate/up launch where that applies
+    // (one row, the one-wave router), else by a route launch first
+    c.route_logits = logits_dev;
+    c.route_bias = bias_dev;
+    c.route_ng = n_group;
+    c.route_tg = topk_group;
+    c.route_norm = norm_topk_prob;
+    c.route_scale = routed_scaling_factor;
+    c.route_ids = ids_dev;
+    c.route_w = weights_dev;
+    c.ids = c.route_ids;
+    c.weights = c.route_w;
+    if (xh_dev)
+        c.xh = xh_dev;
+    else
+        c.x = x_dev;
+    c.out = out_dev;
+    c.ldo = tbl->hidden;
+    c.err_flag = flag;
+    return moe_pass(ctx, c, ptrs[0]);
 }
 
 }  // namespace
@@ -2615,16 +2678,7 @@ int32_t ut_moe_experts_bf16(ut_ctx *ctx, const ut_expert_table *tbl, const int32
                              fake, out_dev));
     if (!bf16_rows_ok(ctx, "ut_moe_experts_bf16", x_dev, tbl->hidden)) return UT_ERR_ARG;
     if (rows == 0) return UT_OK;
-    const int64_t maxM = 4;
-    const int64_t slots = moe_slots((int)maxM, top_k, tbl->n, -1);
-    ScratchPlan plan;
-    plan.add(moe_layout(maxM, top_k, slots, tbl->hidden, tbl->inter, tbl->fmt).total);
-    std::vector<void *> ptrs;
-    UT_TRY(scratch_acquire(ctx, plan, ptrs));
-    int32_t *flag = nullptr;
-    UT_TRY(device_error_flag(ctx, &flag));
-    return moe_experts_rows(ctx, tbl, ids_dev, weights_dev, rows, top_k, nullptr, out_dev, ptrs[0],
-                            flag, x_dev);
+    return moe_experts_any(ctx, tbl, ids_dev, weights_dev, rows, top_k, nullptr, x_dev, out_dev);
 }
 
 }  // extern "C"
