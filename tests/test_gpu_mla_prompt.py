@@ -1,0 +1,46 @@
+"""Matrix-core attention over a prompt's rows (more than 16 rows in a call:
+positions split by how many rows there are, or not at all) against float64
+and against the same rows in calls of up to 16.
+
+Bound: products keep hi*hi + hi*lo + lo*hi of bf16 hi/lo parts, 2^-16 of each
+product, so a score of standard deviation 1.7 (values up to 8) moves by about
+1e-4 and the context by that share of its largest value.
+"""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def f64(qabs, qr, lat, kr, base, scale):
+    s = (torch.einsum("rhl,tl->rht", qabs.double(), lat.double()) +
+         torch.einsum("rhp,tp->rht", qr.double(), kr.double())) * scale
+    R, T = qabs.shape[0], lat.shape[0]
+    t = torch.arange(T, device=s.device)
+    n = base + 1 + torch.arange(R, device=s.device)
+    s.masked_fill_(t[None, None] >= n[:, None, None], float("-inf"))
+    return torch.einsum("rht,tl->rhl", torch.softmax(s, -1), lat.double())
+
+
+# one slice a row (1,024 column groups), several, a tail tile of one
+# position, contexts that end inside the first slice, fewer heads
+@pytest.mark.parametrize("R,H,T", [(17, 128, 17), (17, 128, 700), (33, 32, 33), (40, 64, 2049),
+                                   (100, 128, 100), (257, 128, 257), (260, 128, 900)])
+def test_prompt_rows(ctx, R, H, T):
+    import undertow_amd as U
+    g = torch.Generator(device="cuda").manual_seed(R * T)
+    rnd = lambda *s: torch.randn(s, device="cuda", generator=g)
+    qabs, qr, lat, kr = rnd(R, H, 512), rnd(R, H, 64), rnd(T, 512), rnd(T, 64)
+    base, scale = T - R, float(1 / np.sqrt(192.0))
+    kc = U.mla_cache_split(ctx, lat, kr)
+    got = U.mla_attend_split(ctx, qabs, qr, kc, base, scale)
+    want = f64(qabs, qr, lat, kr, base, scale)
+    tol = 1e-4 * max(1.0, float(want.abs().max()))
+    assert float((got - want).abs().max()) <= tol
+    assert torch.equal(U.mla_attend(ctx, qabs, qr, lat, kr, base, scale), got)
+    few = torch.cat([U.mla_attend_split(ctx, qabs[r:r + 16].contiguous(), qr[r:r + 16].contiguous(),
+                                        kc, base + r, scale) for r in range(0, R, 16)])
+    assert float((got - few).abs().max()) <= tol
+    # no further from float64 than the short calls
+    assert float((got - want).norm()) <= 1.05 * float((few - want).norm())

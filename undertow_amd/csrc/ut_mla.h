@@ -12,6 +12,11 @@ size_t mla_scratch_bytes(int64_t R, int64_t H, int64_t L, int64_t P, int64_t T);
 // of the f32 cache).  Taken for 32k heads, latent 512 and rope 64, up to a
 // context length T whose slice count fits the combine.
 bool mla_kc_ok(int64_t H, int64_t L, int64_t P, int64_t T);
+// A model's attention over R rows: the rows per launch_mla_attend* call (all
+// for the matrix-core kernel, else as many as 64 MB of slice partials hold,
+// at least 16), and the scratch that any call of up to R rows takes.
+int64_t mla_rows_per_call(int64_t R, int64_t H, int64_t L, int64_t P, int64_t T);
+size_t mla_rows_scratch_bytes(int64_t R, int64_t H, int64_t L, int64_t P, int64_t T);
 size_t mla_kc_scratch_bytes(int64_t R, int64_t H, int64_t L, int64_t T);
 int32_t launch_mla_cache_split(ut_ctx *ctx, const float *latent, const float *krot, int64_t T,
                                int64_t L, int64_t P, __bf16 *kc);

@@ -229,6 +229,10 @@ struct MlaMfmaArgs {
     float scale;
     int groups, nslice;  // column groups of 32, slices in the grid
     float *part_m, *part_l, *part_o;  // [j][col], [j][col], [j][L][col]
+    // a prompt's rows (mla_prompt_slice): the slice length, and for one
+    // slice the output itself
+    int64_t slen;
+    float *clat;
 };
 
 constexpr int kRowChunks = 144;       // 16-byte chunks per position (576 hi + 576 lo)
@@ -263,6 +267,10 @@ __device__ __forceinline__ float pair_sum(float v) {
 constexpr int kTile16 = 16;
 constexpr int kTile16Bytes = kTile16 * kRowChunks * 16;  // 36864
 
+// PROMPT: the rows of a prompt (mla_prompt_slice's slice length), longest
+// contexts first so that the launch ends on short ones; with one slice per
+// row the workgroup writes the finished context (no partials, no combine).
+template <bool PROMPT>
 __global__ __launch_bounds__(256, 2) void k_mla_mfma16(MlaMfmaArgs a) {
     constexpr int KS = 9, MT = 4, D = 576;
     typedef __bf16 bf16x8l_t __attribute__((ext_vector_type(8)));
@@ -272,12 +280,12 @@ __global__ __launch_bounds__(256, 2) void k_mla_mfma16(MlaMfmaArgs a) {
     // [dim half][column][position], rows padded to 20 floats
     __shared__ __attribute__((aligned(16))) float sS[2][32][kTile16 + 4];
     const int b = blockIdx.x, x8 = b & 7, q = b >> 3;
-    const int group = q % a.groups;
-    const int slice = (q / a.groups) * 8 + x8;
+    const int group = PROMPT ? a.groups - 1 - b / a.nslice : q % a.groups;
+    const int slice = PROMPT ? b % a.nslice : (q / a.groups) * 8 + x8;
     const int c0 = group * 32;
     const int r = c0 / a.H;
     const int64_t n_ctx = a.pos.get() + r + 1;
-    const int64_t slen = mla_mfma_slice(n_ctx);
+    const int64_t slen = PROMPT ? a.slen : mla_mfma_slice(n_ctx);
     const int64_t p0 = (int64_t)slice * slen;
     if (slice >= a.nslice || p0 >= n_ctx) return;  // uniform per workgroup
     const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
@@ -364,7 +372,10 @@ __global__ __launch_bounds__(256, 2) void k_mla_mfma16(MlaMfmaArgs a) {
         for (int e = 1; e < 8; e++) mt_ = fmaxf(mt_, p[e]);
         mt_ = pair_max(mt_);
         // the exponent offset moves only on a jump of more than kMlaHeadroom
-        const bool jump = mt_ > m_run + kMlaHeadroom;
+        // (a prompt's slice is long enough to meet its maximum late: there the
+        // offset follows it, so the largest weight is 1, which bf16 parts hold
+        // exactly; with the headroom the error against float64 was 4% larger)
+        const bool jump = mt_ > m_run + (PROMPT ? 0.0f : kMlaHeadroom);
         const float m_new = jump ? mt_ : m_run;
         if (__any(jump)) {
             const float alpha = __expf(m_run - m_new);
@@ -408,6 +419,18 @@ __global__ __launch_bounds__(256, 2) void k_mla_mfma16(MlaMfmaArgs a) {
         if (t0 + kTile16 < tend) tile(sT1, sT0, t0 + kTile16);
     }
     // ---- slice partials: O^T register i is dim 128*w + 32*mt + (i/4)*8 + kh*4 + i%4
+    if (PROMPT && a.nslice == 1) {
+        const float inv = 1.0f / l_run;
+        float *po = a.clat + (int64_t)col * L + 128 * w + kh * 4;
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                *(float4 *)(po + 32 * mt + 8 * i) =
+                    make_float4(__fmul_rn(o[mt][4 * i], inv), __fmul_rn(o[mt][4 * i + 1], inv),
+                                __fmul_rn(o[mt][4 * i + 2], inv), __fmul_rn(o[mt][4 * i + 3], inv));
+        return;
+    }
     const int64_t RH = a.RH;
     if (w == 0 && kh == 0) {
         a.part_m[(int64_t)slice * RH + col] = m_run;
@@ -468,6 +491,7 @@ __global__ __launch_bounds__(NT) void k_mla_combine_mfma(const float *__restrict
                                                          const float *__restrict__ part_l,
                                                          const float *__restrict__ part_o,
                                                          int RH, int H, int L, PosRef pos,
+                                                         int64_t slice_len,
                                                          float *__restrict__ clat) {
     static_assert(NT % 64 == 0 && 1024 % NT == 0 && NT >= 256, "whole waves, 256 outputs");
     constexpr int VT = 1024 / NT;                                               // virtual per thread
@@ -484,7 +508,7 @@ __global__ __launch_bounds__(NT) void k_mla_combine_mfma(const float *__restrict
     // the slice count is the same for the workgroup's 32 columns (one query
     // row: 32 | H)
     const int64_t n_ctx = pos.get() + col / H + 1;
-    const int64_t slen = mla_mfma_slice(n_ctx);
+    const int64_t slen = slice_len > 0 ? slice_len : mla_mfma_slice(n_ctx);
     const int ns = (int)((n_ctx + slen - 1) / slen);
     // merge-pass loads: columns 4*c4.., dim dy, slices [j0, j1) of each part
     const int c4 = tid & 7, dy = (tid >> 3) & 7, p0 = tid >> 6;
@@ -593,8 +617,30 @@ static bool mla_mfma_ok(int64_t H, int64_t L, int64_t P, int64_t T) {
 
 bool mla_kc_ok(int64_t H, int64_t L, int64_t P, int64_t T) { return mla_mfma_ok(H, L, P, T); }
 
+// A call of more than kMlaPromptRows rows: its R*H/32 column groups fill the
+// chip by themselves, so positions are split only as far as that needs
+// (kMlaPromptWGs workgroups; 512 are resident at once) instead of by the
+// context length, and not at all from 1,024 groups on.  512 rows over 512
+// positions: 168 us, and 1,004 us with the slices of the context length (16 a row,
+// whose partials alone are 2.1 GB).
+constexpr int64_t kMlaPromptRows = 16, kMlaPromptWGs = 1024;
+static int64_t mla_prompt_nslice(int64_t R, int64_t H, int64_t T) {  // at most
+    const int64_t groups = R * H / 32;
+    int64_t ns = (kMlaPromptWGs + groups - 1) / groups;
+    const int64_t tiles = (T + kTile16 - 1) / kTile16;
+    if (ns > (tiles + 1) / 2) ns = (tiles + 1) / 2;  // two tiles a slice at least
+    return ns < kCombineSmallSlices ? ns : kCombineSmallSlices;
+}
+static int64_t mla_prompt_slice(int64_t R, int64_t H, int64_t T) {
+    const int64_t ns = mla_prompt_nslice(R, H, T), tiles = (T + kTile16 - 1) / kTile16;
+    return (tiles + ns - 1) / ns * kTile16;
+}
+static bool mla_prompt(int64_t R) { return R > kMlaPromptRows; }
+
 static size_t mla_mfma_scratch_bytes(int64_t R, int64_t H, int64_t L, int64_t T) {
-    const size_t ns = (size_t)mla_mfma_nslice(T), RH = (size_t)(R * H);
+    const size_t ns = (size_t)(mla_prompt(R) ? mla_prompt_nslice(R, H, T) : mla_mfma_nslice(T)),
+                 RH = (size_t)(R * H);
+    if (mla_prompt(R) && ns == 1) return 0;
     return ((ns * RH * 4 + 255) & ~size_t(255)) * 2 + ((ns * L * RH * 4 + 255) & ~size_t(255));
 }
 
@@ -610,6 +656,22 @@ size_t mla_scratch_bytes(int64_t R, int64_t H, int64_t L, int64_t P, int64_t T) 
     return mla_mfma_ok(H, L, P, T)
                ? mla_mfma_scratch_bytes(R, H, L, T) + (size_t)T * (L + P) * 4 + 256
                : mla_split_scratch_bytes(R, H, L, T);
+}
+
+int64_t mla_rows_per_call(int64_t R, int64_t H, int64_t L, int64_t P, int64_t T) {
+    if (mla_mfma_ok(H, L, P, T)) return R;
+    const int64_t per = (int64_t)mla_split_scratch_bytes(1, H, L, T), n = (int64_t(64) << 20) / per;
+    return n < 16 ? 16 : n;
+}
+
+size_t mla_rows_scratch_bytes(int64_t R, int64_t H, int64_t L, int64_t P, int64_t T) {
+    const int64_t per = mla_rows_per_call(R, H, L, P, T), n = R < per ? R : per;
+    size_t most = 0;
+    for (int64_t r = 1; r <= n; r++) {
+        const size_t b = mla_scratch_bytes(r, H, L, P, T);
+        if (b > most) most = b;
+    }
+    return most;
 }
 
 size_t mla_kc_scratch_bytes(int64_t R, int64_t H, int64_t L, int64_t T) {
@@ -636,8 +698,11 @@ int32_t launch_mla_attend_kc(ut_ctx *ctx, const float *qabs, const float *qrope,
                        "16-byte aligned cache and at most %d slices", kMlaMaxSlices);
         return UT_ERR_SHAPE;
     }
-    const int64_t RH = R * H, ns = mla_mfma_nslice(T);
-    MlaMfmaArgs a;
+    const bool prompt = mla_prompt(R) && !ctx->step_pos;
+    MlaMfmaArgs a{};
+    a.slen = prompt ? mla_prompt_slice(R, H, T) : 0;
+    a.clat = clat;
+    const int64_t RH = R * H, ns = prompt ? (T + a.slen - 1) / a.slen : mla_mfma_nslice(T);
     a.qabs = qabs; a.qrope = qrope; a.kc = kc;
     a.H = (int)H; a.L = (int)L; a.P = (int)P; a.RH = (int)RH;
     a.pos = pos_ref(ctx, pos_base);
@@ -650,9 +715,14 @@ int32_t launch_mla_attend_kc(ut_ctx *ctx, const float *qabs, const float *qrope,
     a.groups = (int)(RH / 32);  // 32 columns per workgroup
     const int64_t nwg = (int64_t)a.groups * ((ns + 7) / 8 * 8);
     int tok = timing_begin(ctx, "mla_mfma");
-    hipLaunchKernelGGL(k_mla_mfma16, dim3((unsigned)nwg), dim3(256), 0, ctx->stream, a);
+    if (prompt)
+        hipLaunchKernelGGL(k_mla_mfma16<true>, dim3((unsigned)(a.groups * ns)), dim3(256), 0,
+                           ctx->stream, a);
+    else
+        hipLaunchKernelGGL(k_mla_mfma16<false>, dim3((unsigned)nwg), dim3(256), 0, ctx->stream, a);
     timing_end(ctx, tok);
     UT_TRY(launch_check(ctx, "k_mla_mfma"));
+    if (prompt && ns == 1) return UT_OK;
     tok = timing_begin(ctx, "mla_combine");
     const dim3 cgrid((unsigned)(RH / 32), (unsigned)(L / 8));
     // up to 64 slices: 256-thread workgroups once the grid exceeds one per
@@ -661,19 +731,19 @@ int32_t launch_mla_attend_kc(ut_ctx *ctx, const float *qabs, const float *qrope,
     if (a.nslice <= kCombineSmallSlices && (int64_t)cgrid.x * cgrid.y > ctx->multiprocessors)
         hipLaunchKernelGGL((k_mla_combine_mfma<kCombineSmallSlices, UT_MLA_COMBINE_SMALL_NT>), cgrid,
                            dim3(UT_MLA_COMBINE_SMALL_NT), 0, ctx->stream, a.part_m, a.part_l,
-                           a.part_o, (int)RH, (int)H, (int)L, a.pos, clat);
+                           a.part_o, (int)RH, (int)H, (int)L, a.pos, a.slen, clat);
     else if (a.nslice <= kCombineSmallSlices)
         hipLaunchKernelGGL((k_mla_combine_mfma<kCombineSmallSlices, 1024>), cgrid, dim3(1024), 0,
                            ctx->stream, a.part_m, a.part_l, a.part_o, (int)RH, (int)H, (int)L,
-                           a.pos, clat);
+                           a.pos, a.slen, clat);
     else if (a.nslice <= 2 * kCombineSmallSlices)
         hipLaunchKernelGGL((k_mla_combine_mfma<2 * kCombineSmallSlices, 1024>), cgrid, dim3(1024), 0,
                            ctx->stream, a.part_m, a.part_l, a.part_o, (int)RH, (int)H, (int)L,
-                           a.pos, clat);
+                           a.pos, a.slen, clat);
     else
         hipLaunchKernelGGL((k_mla_combine_mfma<kMlaMaxSlices, 1024>), cgrid, dim3(1024), 0,
                            ctx->stream, a.part_m, a.part_l, a.part_o, (int)RH, (int)H, (int)L,
-                           a.pos, clat);
+                           a.pos, a.slen, clat);
     timing_end(ctx, tok);
     return launch_check(ctx, "k_mla_combine_mfma");
 }

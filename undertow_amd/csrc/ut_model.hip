@@ -163,7 +163,6 @@ struct ut_session {
 
 namespace {
 
-constexpr int64_t kMlaRowsPerCall = 16;
 constexpr int64_t kPinIds = 16384;   // ints of the upload slot (the last 8: verify ids)
 constexpr int64_t kPinBack = 64;     // ints of the readback slot (argmax rows, drafts, flag)
 
@@ -393,7 +392,7 @@ int32_t ws_reserve(ut_session *s, int64_t rows) {
     size_t idA = plan.add(matmul_digit_bytes(R, kmax));
     size_t idB = plan.add(matmul_digit_bytes(R, kmax));
     size_t imoes = plan.add(moe_bytes);
-    size_t imla = plan.add(mla_scratch_bytes(R < kMlaRowsPerCall ? R : kMlaRowsPerCall, heads, Lr, c.qk_rope_head_dim, s->cap));
+    size_t imla = plan.add(mla_rows_scratch_bytes(R, heads, Lr, c.qk_rope_head_dim, s->cap));
     size_t iarg = plan.add(argmax_scratch_bytes(R, c.vocab_size) + 256);
     // the fast-int8 path's MLP and expert rows (four rows at a time): gate,
     // up, h [4][max inter], the choices' outputs [4][k][H] and a shared
@@ -1039,10 +1038,9 @@ int32_t mla_forward(ut_session *s, const LayerW &L, const float *x, const XDigit
     kv.len = pos_base + rows;
     UT_TRY(launch_absorb_q(ctx, L.kv_b, w.q, rows, heads, nope, rope, vh, w.qabs, w.qrope,
                            pos_base, m->rope_table));
-    // query rows in groups of kMlaRowsPerCall (bounded scratch; a row's
-    // result does not depend on its group)
-    for (int64_t r0 = 0; r0 < rows; r0 += kMlaRowsPerCall) {
-        const int64_t rn = rows - r0 < kMlaRowsPerCall ? rows - r0 : kMlaRowsPerCall;
+    const int64_t per = mla_rows_per_call(rows, heads, Lr, rope, s->cap);
+    for (int64_t r0 = 0; r0 < rows; r0 += per) {
+        const int64_t rn = rows - r0 < per ? rows - r0 : per;
         if (kv.kc)
             UT_TRY(launch_mla_attend_kc(ctx, w.qabs + r0 * heads * Lr, w.qrope + r0 * heads * rope,
                                         kv.kc, rn, heads, Lr, rope, pos_base + r0, scale,
