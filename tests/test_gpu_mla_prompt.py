@@ -44,3 +44,19 @@ def test_prompt_rows(ctx, R, H, T):
     assert float((got - few).abs().max()) <= tol
     # no further from float64 than the short calls
     assert float((got - want).norm()) <= 1.05 * float((few - want).norm())
+
+
+@pytest.mark.parametrize("R,H,T", [(16, 128, 16), (16, 128, 513), (20, 128, 100), (17, 128, 128),
+                                   (128, 32, 128), (4, 128, 33)])
+def test_rows_merge_equals_single_rows(ctx, R, H, T):
+    """Calls that keep the slices of the context length merge them with the
+    same sums whatever kernel merges: rows equal their own one-row calls."""
+    import undertow_amd as U
+    g = torch.Generator(device="cuda").manual_seed(R + T)
+    rnd = lambda *s: torch.randn(s, device="cuda", generator=g)
+    qabs, qr, lat, kr = rnd(R, H, 512), rnd(R, H, 64), rnd(T, 512), rnd(T, 64)
+    kc, scale = U.mla_cache_split(ctx, lat, kr), float(1 / np.sqrt(192.0))
+    got = U.mla_attend_split(ctx, qabs, qr, kc, T - R, scale)
+    one = torch.cat([U.mla_attend_split(ctx, qabs[r:r + 1].contiguous(), qr[r:r + 1].contiguous(),
+                                        kc, T - R + r, scale) for r in range(R)])
+    assert torch.equal(got, one)

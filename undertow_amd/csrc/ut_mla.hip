@@ -602,6 +602,70 @@ __global__ __launch_bounds__(NT) void k_mla_combine_mfma(const float *__restrict
     }
 }
 
+// The same merge where up to 16 slices a row meet many rows: each of
+// k_mla_combine_mfma's sixteen parts is then one slice, so a thread adds its
+// dims' slices one after another and the sums are that kernel's, bit for
+// bit.  A workgroup takes 32 columns x 64 dims: the partials are read 128
+// bytes a row, the context written 256 bytes a column (through LDS).  Bound
+// by the partials' read.
+constexpr int kCombineRowsSlices = 16, kCombineRowsDims = 64;
+// Taken from 2,048 columns (16 rows of 128 heads) on, or 512 with at most two
+// slices: whole calls of 17 rows over 300 positions 40.2 -> 31.4 us, 72 over
+// 72 111 -> 64, 129 over 129 132 -> 52, 8 over 8 17.6 -> 13.0; with less to
+// merge per workgroup k_mla_combine_mfma stays ahead (8 rows over 512
+// positions 27.6 against 29.4 us, one row 13.7 against 18.6).
+static bool mla_combine_rows_ok(int64_t RH, int64_t nslice) {
+    return nslice <= kCombineRowsSlices && (RH >= 2048 || (RH >= 512 && nslice <= 2));
+}
+__global__ __launch_bounds__(256) void k_mla_combine_rows(const float *__restrict__ part_m,
+                                                          const float *__restrict__ part_l,
+                                                          const float *__restrict__ part_o, int RH,
+                                                          int H, int L, PosRef pos,
+                                                          int64_t slice_len,
+                                                          float *__restrict__ clat) {
+    __shared__ float so[32][kCombineRowsDims + 1];
+    const int tid = threadIdx.x, tx = tid & 31, ty = tid >> 5;
+    const int col = blockIdx.x * 32 + tx, d0 = blockIdx.y * kCombineRowsDims;
+    const int64_t n_ctx = pos.get() + col / H + 1;
+    const int64_t slen = slice_len > 0 ? slice_len : mla_mfma_slice(n_ctx);
+    const int ns = (int)((n_ctx + slen - 1) / slen);  // one query row per workgroup
+    float w[kCombineRowsSlices], l[kCombineRowsSlices], M = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < kCombineRowsSlices; j++)
+        if (j < ns) {
+            w[j] = part_m[(int64_t)j * RH + col];
+            l[j] = part_l[(int64_t)j * RH + col];
+        }
+#pragma unroll
+    for (int j = 0; j < kCombineRowsSlices; j++)
+        if (j < ns) M = fmaxf(M, w[j]);
+    float acc[8], t = 0.0f;
+    const float *po = part_o + (int64_t)(d0 + ty) * RH + col;
+#pragma unroll
+    for (int j = 0; j < kCombineRowsSlices; j++)
+        if (j < ns) {
+            float v[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) v[i] = po[((int64_t)j * L + 8 * i) * RH];
+            const float e = __expf(w[j] - M);
+            t = j ? __fadd_rn(t, __fmul_rn(l[j], e)) : __fmul_rn(l[j], e);
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+                acc[i] = j ? __fadd_rn(acc[i], __fmul_rn(v[i], e)) : __fmul_rn(v[i], e);
+        }
+    const float inv = 1.0f / t;
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+        so[tx][ty + 8 * i] = __fmul_rn(__fadd_rn(acc[i], 0.0f), inv);  // the empty parts' zeros
+    __syncthreads();
+    const int c = tid >> 3, q = tid & 7;
+    float *out = clat + (int64_t)(blockIdx.x * 32 + c) * L + d0 + 4 * q;
+#pragma unroll
+    for (int i = 0; i < kCombineRowsDims; i += 32)
+        *(float4 *)(out + i) = make_float4(so[c][4 * q + i], so[c][4 * q + i + 1],
+                                           so[c][4 * q + i + 2], so[c][4 * q + i + 3]);
+}
+
 // Largest slice count over the rows' context lengths n <= T (an upper
 // bound: slices past a row's count exit at once).
 static int64_t mla_mfma_nslice(int64_t T) {
@@ -635,12 +699,17 @@ static int64_t mla_prompt_slice(int64_t R, int64_t H, int64_t T) {
     const int64_t ns = mla_prompt_nslice(R, H, T), tiles = (T + kTile16 - 1) / kTile16;
     return (tiles + ns - 1) / ns * kTile16;
 }
-static bool mla_prompt(int64_t R) { return R > kMlaPromptRows; }
+// Contexts of up to kMlaPromptMinT positions keep the slices of the context
+// length also for many rows, so that a short prompt's rows get the values of
+// its decode steps bit for bit.  The price: 128 rows over 128 positions take
+// 104 us, 129 over 129 without that 52 us.
+constexpr int64_t kMlaPromptMinT = 128;
+static bool mla_prompt(int64_t R, int64_t T) { return R > kMlaPromptRows && T > kMlaPromptMinT; }
 
 static size_t mla_mfma_scratch_bytes(int64_t R, int64_t H, int64_t L, int64_t T) {
-    const size_t ns = (size_t)(mla_prompt(R) ? mla_prompt_nslice(R, H, T) : mla_mfma_nslice(T)),
+    const size_t ns = (size_t)(mla_prompt(R, T) ? mla_prompt_nslice(R, H, T) : mla_mfma_nslice(T)),
                  RH = (size_t)(R * H);
-    if (mla_prompt(R) && ns == 1) return 0;
+    if (mla_prompt(R, T) && ns == 1) return 0;
     return ((ns * RH * 4 + 255) & ~size_t(255)) * 2 + ((ns * L * RH * 4 + 255) & ~size_t(255));
 }
 
@@ -666,11 +735,14 @@ int64_t mla_rows_per_call(int64_t R, int64_t H, int64_t L, int64_t P, int64_t T)
 
 size_t mla_rows_scratch_bytes(int64_t R, int64_t H, int64_t L, int64_t P, int64_t T) {
     const int64_t per = mla_rows_per_call(R, H, L, P, T), n = R < per ? R : per;
+    // (more rows over fewer positions can take more slices in all)
     size_t most = 0;
-    for (int64_t r = 1; r <= n; r++) {
-        const size_t b = mla_scratch_bytes(r, H, L, P, T);
-        if (b > most) most = b;
-    }
+    for (int64_t r = 1; r <= n; r++)
+        for (int64_t t : {T, T < kMlaPromptMinT ? T : kMlaPromptMinT}) {
+            if (r > t) continue;
+            const size_t b = mla_scratch_bytes(r, H, L, P, t);
+            if (b > most) most = b;
+        }
     return most;
 }
 
@@ -698,7 +770,7 @@ int32_t launch_mla_attend_kc(ut_ctx *ctx, const float *qabs, const float *qrope,
                        "16-byte aligned cache and at most %d slices", kMlaMaxSlices);
         return UT_ERR_SHAPE;
     }
-    const bool prompt = mla_prompt(R) && !ctx->step_pos;
+    const bool prompt = mla_prompt(R, T) && !ctx->step_pos;
     MlaMfmaArgs a{};
     a.slen = prompt ? mla_prompt_slice(R, H, T) : 0;
     a.clat = clat;
@@ -728,7 +800,12 @@ int32_t launch_mla_attend_kc(ut_ctx *ctx, const float *qabs, const float *qrope,
     // up to 64 slices: 256-thread workgroups once the grid exceeds one per
     // CU (config-4 verify of four rows: 15.2 -> 7.4 us per combine; at one
     // row the 1,024-thread form is 0.2 us faster)
-    if (a.nslice <= kCombineSmallSlices && (int64_t)cgrid.x * cgrid.y > ctx->multiprocessors)
+    if (mla_combine_rows_ok(RH, a.nslice))
+        hipLaunchKernelGGL(k_mla_combine_rows,
+                           dim3((unsigned)(RH / 32), (unsigned)(L / kCombineRowsDims)), dim3(256), 0,
+                           ctx->stream, a.part_m, a.part_l, a.part_o, (int)RH, (int)H, (int)L,
+                           a.pos, a.slen, clat);
+    else if (a.nslice <= kCombineSmallSlices && (int64_t)cgrid.x * cgrid.y > ctx->multiprocessors)
         hipLaunchKernelGGL((k_mla_combine_mfma<kCombineSmallSlices, UT_MLA_COMBINE_SMALL_NT>), cgrid,
                            dim3(UT_MLA_COMBINE_SMALL_NT), 0, ctx->stream, a.part_m, a.part_l,
                            a.part_o, (int)RH, (int)H, (int)L, a.pos, a.slen, clat);
