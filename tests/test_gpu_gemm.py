@@ -71,3 +71,26 @@ def test_gemm_nonfinite_rows_are_nan(ctx):
     assert np.isnan(got[[2, 5]]).all()
     ok = [r for r in range(9) if r not in (2, 5)]
     assert np.array_equal(got[ok], want[ok])
+
+
+# f32 slices of one to four 64-column steps and none, tails of a step, outputs
+# past a 64-row tile, K % 4 != 0 (the generic kernel), more columns than a
+# slice of the product takes (the GEMV passes)
+@pytest.mark.parametrize("o,i", [(256, 7168), (3, 4), (65, 60), (70, 132), (130, 200), (1000, 1028),
+                                 (2048, 1024), (4096, 1024), (17, 131), (20000, 256)])
+def test_f32_rows_equal_one_row_calls(ctx, o, i):
+    """Each output's products are added in the one-row GEMV's order: bitwise."""
+    import undertow_amd as U
+    rng = np.random.default_rng(o + i)
+    w = rng.standard_normal((o, i)).astype(np.float32)
+    q = U.QTensor(ctx, U.F32, w, None, o, i)
+    x = rng.standard_normal((131, i)).astype(np.float32)
+    rows = [0, 3, 4, 63, 64, 127, 128, 130]
+    one = np.concatenate([run(ctx, q, x[r:r + 1]) for r in rows])
+    for seq in (5, 64, 131):
+        got = run(ctx, q, x[:seq])
+        n = [k for k, r in enumerate(rows) if r < seq]
+        assert np.array_equal(got[[rows[k] for k in n]], one[n]), seq
+    ref = x.astype(np.float64) @ w.astype(np.float64).T
+    err = np.linalg.norm(run(ctx, q, x) - ref) / np.linalg.norm(ref)
+    assert err <= 2.0 ** -23 * max(1.0, np.log2(i))  # tree-wise f32 sums

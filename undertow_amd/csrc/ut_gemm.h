@@ -45,4 +45,15 @@ bool gemm_ok(const ut_qtensor *w, int64_t M);
 int32_t launch_gemm(ut_ctx *ctx, const ut_qtensor *w, const DigitPlanes &x, int64_t M, float *out,
                     int64_t ldo, int accumulate);
 
+// f32 weights (ut_gemm_f32.hip), each output's products added in the order
+// of the GEMV that fewer rows take.  gemv_f32_split: that GEMV's K split, of
+// the weight's shape alone.
+void gemv_f32_split(int64_t O, int64_t K, int *ks, int64_t *kslice);
+bool gemm_f32_ok(const ut_qtensor *w, const float *x, int64_t M);
+int32_t launch_gemm_f32(ut_ctx *ctx, const ut_qtensor *w, const float *x, int64_t M, float *out,
+                        int64_t ldo, int accumulate);
+// launch_rowdot_f32 over any number of rows x [M, K].
+int32_t launch_rowdot_f32_rows(ut_ctx *ctx, const ut_qtensor *w, const float *x, int64_t M,
+                               float *out, int64_t ldo);
+
 }  // namespace ut

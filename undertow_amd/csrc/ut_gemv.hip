@@ -1048,7 +1048,7 @@ __global__ __launch_bounds__(64) void k_gemv_generic(int32_t fmt, const uint8_t 
     const int64_t row = blockIdx.x;
     const int lane = threadIdx.x;
     const uint8_t *wr = w + row * row_bytes;
-    for (int64_t m = 0; m < M; m++) {
+    for (int64_t m = blockIdx.y; m < M; m += gridDim.y) {
         float v;
         if (fmt == UT_FMT_F32) {
             float acc = 0.0f;
@@ -1150,6 +1150,10 @@ static void splitk_plan(int32_t fmt, int64_t O, int64_t K, int rows_per_wg, int6
     kslice = (kslice + step - 1) / step * step;
     *ks_out = (int)((K + kslice - 1) / kslice);
     *kslice_out = kslice;
+}
+
+void gemv_f32_split(int64_t O, int64_t K, int *ks, int64_t *kslice) {
+    splitk_plan(UT_FMT_F32, O, K, 64, 0, ks, kslice);
 }
 
 // Workgroups of k_gemv<FMT, M> resident on the whole chip (occupancy query,
@@ -1553,6 +1557,8 @@ int32_t gemv(ut_ctx *ctx, const GemvArgs &ga) {
                        "columns (a multiple of the step) of an int4/int8 weight, 16-byte aligned");
         return UT_ERR_ARG;
     }
+    if (!ga.w2 && gemm_f32_ok(w, ga.xf, ga.M))
+        return launch_gemm_f32(ctx, w, ga.xf, ga.M, ga.out, ga.ldo, ga.accumulate);
     if (fast_ok(w) && (w->fmt == UT_FMT_F32 ? aligned16(ga.xf) && (w->in_dim % 4 == 0) : true)) {
         for (int64_t m0 = 0; m0 < ga.M; m0 += 4) {
             int mrows = (int)((ga.M - m0) < 4 ? (ga.M - m0) : 4);
@@ -1569,7 +1575,10 @@ int32_t gemv(ut_ctx *ctx, const GemvArgs &ga) {
         return UT_ERR_ARG;
     }
     int tok = timing_begin(ctx, "gemv_generic");
-    hipLaunchKernelGGL(k_gemv_generic, dim3((unsigned)w->out_dim), dim3(64), 0, ctx->stream, w->fmt,
+    // one wave per output and group of rows: enough waves to hide a short
+    // row's chain (K % 4 != 0 f32 rows of a prompt)
+    const unsigned gy = (unsigned)(ga.M < 64 ? ga.M : 64);
+    hipLaunchKernelGGL(k_gemv_generic, dim3((unsigned)w->out_dim, gy), dim3(64), 0, ctx->stream, w->fmt,
                        (const uint8_t *)w->payload, w->scales, w->out_dim, w->in_dim, w->row_bytes,
                        ga.xd.xt, ga.xd.exps, ga.xf, w->in_dim, ga.M, ga.out, ga.ldo, ga.accumulate);
     timing_end(ctx, tok);

@@ -818,13 +818,10 @@ int32_t moe_forward_rows(ut_session *s, const LayerW &L, const float *x, const X
     const ut_model_config &c = m->c;
     Workspace &w = s->ws;
     const int64_t H = c.hidden_size, E = c.n_routed_experts, k = c.num_experts_per_tok;
-    for (int64_t s0 = 0; s0 < rows; s0 += 4) {
-        const int64_t M = rows - s0 < 4 ? rows - s0 : 4;
-        if (rowdot_f32_ok(L.gate, M) && ((uintptr_t)(x + s0 * H) & 15) == 0)
-            UT_TRY(launch_rowdot_f32(ctx, L.gate, x + s0 * H, M, w.rlogits + s0 * E, E));
-        else
-            UT_TRY(mm(s, L.gate, x + s0 * H, M, w.rlogits + s0 * E, E));
-    }
+    if (rowdot_f32_ok(L.gate, 1) && ((uintptr_t)x & 15) == 0)
+        UT_TRY(launch_rowdot_f32_rows(ctx, L.gate, x, rows, w.rlogits, E));
+    else
+        UT_TRY(mm(s, L.gate, x, rows, w.rlogits, E));
     UT_TRY(launch_route(ctx, w.rlogits, L.bias, rows, E, (int)k, (int)c.n_group, (int)c.topk_group,
                         c.norm_topk_prob, c.routed_scaling_factor, w.rids, w.rw));
     if (L.has_shared) UT_TRY(mlp_rows(s, L.shared, x, xd, rows, w.moe_out, 0));
