@@ -168,43 +168,13 @@ struct GemmArgs {
     int64_t *part;  // ks > 1: totals [ks][M][O]
 };
 
-// Up to about 32 rows the weights' read bounds it (int8 7168 x 16384 from
-// memory: 16 rows 47 us, 2.5 TB/s; the four-row GEMV passes took 118 us),
-// beyond that the matrix cores (512 rows 290 us, 1.24 POP/s of digit
-// products against 3,611 us; 129280 x 7168 2,100 against 19,492 us).
-constexpr int kGemmTO = 4;
-template <int FMT, int TM, bool UNAL>
-__global__ __launch_bounds__(kGemmThreads, 2) void k_gemm(GemmArgs a) {
-    __shared__ uint4 lds[gemm_lds_uint4<TM>()];
-    // consecutive workgroups go to the 8 XCDs in turn: the activation tiles
-    // of one weight tile are given to one XCD, so its L2 serves the weights
-    // to all but the first of them
-    const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
-    const int unit = (j / a.tm) * 8 + xcd, mt = j % a.tm;
-    if (unit >= a.to * a.ks) return;
-    const int ot = unit % a.to, z = unit / a.to;
-    const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, q = lane >> 4;
-    const int64_t o0 = (int64_t)ot * (64 * kGemmTO) + (tid >> 6) * (16 * kGemmTO);
-    const int64_t m0 = (int64_t)mt * (16 * TM);
-    GemmRows<kGemmTO> rows;
+// A wave's finished tile: weight rows o0 .. of activation rows m0 ..
+template <int FMT, int TO, int TM>
+__device__ __forceinline__ void gemm_store(const GemmArgs &a, const ut_i32x4 (&acc)[TO][TM][3],
+                                           int64_t o0, int64_t m0, int z) {
+    const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
 #pragma unroll
-    for (int t = 0; t < kGemmTO; t++) {
-        const int64_t o = o0 + 16 * t + r;
-        rows.row[t] = a.w + (o < a.O ? o : a.O - 1) * a.row_bytes;
-    }
-    rows.end = a.end;
-    const int8_t *src[gemm_stage_n<TM>()];
-#pragma unroll
-    for (int i = 0; i < gemm_stage_n<TM>(); i++) {
-        const GemmChunk c = gemm_chunk(tid + i * kGemmThreads);
-        const int64_t m = m0 + c.m < a.M ? m0 + c.m : a.M - 1;
-        src[i] = a.pl + (m * 3 + (c.p < 3 ? c.p : 0)) * a.kp + c.off;
-    }
-    const int64_t kb = z * a.kslice, ke = kb + a.kslice < a.kp ? kb + a.kslice : a.kp;
-    ut_i32x4 acc[kGemmTO][TM][3];
-    gemm_tile<FMT, kGemmTO, TM, UNAL>(rows, a.row_bytes, kb, ke, src, lds, acc);
-#pragma unroll
-    for (int t = 0; t < kGemmTO; t++) {
+    for (int t = 0; t < TO; t++) {
         const int64_t o = o0 + 16 * t + 4 * q;
 #pragma unroll
         for (int n = 0; n < TM; n++) {
@@ -230,6 +200,80 @@ __global__ __launch_bounds__(kGemmThreads, 2) void k_gemm(GemmArgs a) {
                 }
         }
     }
+}
+
+// Up to about 32 rows the weights' read bounds it (int8 7168 x 16384 from
+// memory: 16 rows 47 us, 2.5 TB/s; the four-row GEMV passes took 118 us),
+// beyond that the matrix cores (512 rows 290 us, 1.24 POP/s of digit
+// products against 3,611 us; 129280 x 7168 2,100 against 19,492 us).
+constexpr int kGemmTO = 4;
+template <int FMT, int TM, bool UNAL>
+__global__ __launch_bounds__(kGemmThreads, 2) void k_gemm(GemmArgs a) {
+    __shared__ uint4 lds[gemm_lds_uint4<TM>()];
+    // consecutive workgroups go to the 8 XCDs in turn: the activation tiles
+    // of one weight tile are given to one XCD, so its L2 serves the weights
+    // to all but the first of them
+    const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
+    const int unit = (j / a.tm) * 8 + xcd, mt = j % a.tm;
+    if (unit >= a.to * a.ks) return;
+    const int ot = unit % a.to, z = unit / a.to;
+    const int tid = threadIdx.x, r = tid & 15;
+    const int64_t o0 = (int64_t)ot * (64 * kGemmTO) + (tid >> 6) * (16 * kGemmTO);
+    const int64_t m0 = (int64_t)mt * (16 * TM);
+    GemmRows<kGemmTO> rows;
+#pragma unroll
+    for (int t = 0; t < kGemmTO; t++) {
+        const int64_t o = o0 + 16 * t + r;
+        rows.row[t] = a.w + (o < a.O ? o : a.O - 1) * a.row_bytes;
+    }
+    rows.end = a.end;
+    const int8_t *src[gemm_stage_n<TM>()];
+#pragma unroll
+    for (int i = 0; i < gemm_stage_n<TM>(); i++) {
+        const GemmChunk c = gemm_chunk(tid + i * kGemmThreads);
+        const int64_t m = m0 + c.m < a.M ? m0 + c.m : a.M - 1;
+        src[i] = a.pl + (m * 3 + (c.p < 3 ? c.p : 0)) * a.kp + c.off;
+    }
+    const int64_t kb = z * a.kslice, ke = kb + a.kslice < a.kp ? kb + a.kslice : a.kp;
+    ut_i32x4 acc[kGemmTO][TM][3];
+    gemm_tile<FMT, kGemmTO, TM, UNAL>(rows, a.row_bytes, kb, ke, src, lds, acc);
+    gemm_store<FMT, kGemmTO, TM>(a, acc, o0, m0, z);
+}
+
+// More than kGlMinRows rows of 16-byte aligned weights: 128 weight rows x 64
+// activation rows per workgroup of eight waves, two workgroups (four waves a
+// SIMD) per CU.  Bound by the matrix cores, at nine tenths of what a large
+// int8 library product reaches on this card (2.1 POP/s): 512 rows of int8
+// 7168 x 16384 285 us with the direct tile, 197 us so (1.84 POP/s);
+// 129280 x 7168 1,982 -> 1,545; int4 18432 x 7168 260 -> 226.  Four waves of
+// 4 x 2 tiles: 190 / 1,546 / 245 us; 256 x 64 tiles, one workgroup per CU:
+// 217 / 1,724 / 265; stages of 64 columns, three workgroups: 257 / 1,796 /
+// 269.  At 32 rows and fewer the launch is bound by the weights' read, which
+// the direct tile keeps more of in flight (129280 x 7168 at 16 rows 183
+// against 234 us); at 64 this one leads (7168 x 16384 67 -> 61 us, 18432 x
+// 7168 72 -> 63).
+constexpr int64_t kGlMinRows = 32;
+constexpr int kGlTO = 2, kGlTM = 2, kGlWO = 4, kGlWM = 2, kGlS = 128;
+template <int FMT>
+__global__ __launch_bounds__(64 * kGlWO * kGlWM, 2) void k_gemm_lds(GemmArgs a) {
+    using L = GemmLds<FMT, kGlTO, kGlTM, kGlWO, kGlWM, kGlS>;
+    __shared__ L s0, s1;
+    const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
+    const int unit = (j / a.tm) * 8 + xcd, mt = j % a.tm;
+    if (unit >= a.to * a.ks) return;
+    const int ot = unit % a.to, z = unit / a.to;
+    const int wave = threadIdx.x >> 6;
+    const int64_t ob = (int64_t)ot * L::kARows, mb = (int64_t)mt * (16 * kGlTM * kGlWM);
+    GemmSrc<FMT, kGlTO, kGlTM, kGlWO, kGlWM, kGlS> src;
+    gemm_src<FMT, kGlTO, kGlTM, kGlWO, kGlWM, kGlS>(
+        src,
+        [&](int row) { return a.w + (ob + row < a.O ? ob + row : a.O - 1) * a.row_bytes; },
+        [&](int m, int p) { return a.pl + ((mb + m < a.M ? mb + m : a.M - 1) * 3 + p) * a.kp; });
+    const int64_t kb = z * a.kslice, ke = kb + a.kslice < a.kp ? kb + a.kslice : a.kp;
+    ut_i32x4 acc[kGlTO][kGlTM][3];
+    gemm_tile_lds<FMT, kGlTO, kGlTM, kGlWO, kGlWM, kGlS>(src, a.row_bytes, kb, ke, s0, s1, acc);
+    gemm_store<FMT, kGlTO, kGlTM>(a, acc, ob + (wave % kGlWO) * (16 * kGlTO),
+                                  mb + (wave / kGlWO) * (16 * kGlTM), z);
 }
 
 // The K splits' totals summed and scaled (exact integers: any order).
@@ -272,8 +316,10 @@ int32_t launch_gemm(ut_ctx *ctx, const ut_qtensor *w, const DigitPlanes &x, int6
         a.pl = x.p + s0 * 3 * x.kp;
         a.exps = x.exps + s0;
         a.out = out + s0 * ldo;
-        const int tmr = a.M <= 16 ? 1 : a.M <= 32 ? 2 : 2;
-        a.to = (int)((a.O + 64 * kGemmTO - 1) / (64 * kGemmTO));
+        const bool big = !unal && a.M > kGlMinRows;
+        const int tmr = big ? kGlTM * kGlWM : a.M <= 16 ? 1 : 2;
+        const int tor = big ? 16 * kGlTO * kGlWO : 64 * kGemmTO;
+        a.to = (int)((a.O + tor - 1) / tor);
         a.tm = (int)((a.M + 16 * tmr - 1) / (16 * tmr));
         // split K until the launch has two workgroups per CU, at least two
         // steps each, partials within their buffer
@@ -294,7 +340,11 @@ int32_t launch_gemm(ut_ctx *ctx, const ut_qtensor *w, const DigitPlanes &x, int6
         if (tmr == 1) UT_GM(F, 1, U);   \
         else UT_GM(F, 2, U);            \
     } while (0)
-        if (w->fmt == UT_FMT_INT8) {
+        if (big) {
+            const dim3 bd(64 * kGlWO * kGlWM);
+            if (w->fmt == UT_FMT_INT8) hipLaunchKernelGGL(k_gemm_lds<UT_FMT_INT8>, grid, bd, 0, ctx->stream, a);
+            else hipLaunchKernelGGL(k_gemm_lds<UT_FMT_INT4>, grid, bd, 0, ctx->stream, a);
+        } else if (w->fmt == UT_FMT_INT8) {
             if (unal) UT_GMT(UT_FMT_INT8, true);
             else UT_GMT(UT_FMT_INT8, false);
         } else {

@@ -76,9 +76,20 @@ __device__ __forceinline__ void gemm_load_a(GemmA<FMT, TO> &a, const GemmRows<TO
             a.v[t][i] = gemm_ld16<UNAL>(r.row[t], off, len, r.end);
         }
 }
-// The A operand of matrix instruction s: 16 codes per lane.  int4 codes come
-// out times 16 (a nibble in the byte's high half is its own sign extension),
-// which the epilogue's exponent takes back.
+// 16 int4 codes as bytes, times 16 (a nibble in the byte's high half is its
+// own sign extension), which the epilogue's exponent takes back.
+__device__ __forceinline__ ut_i32x4 gemm_i4_codes(uint32_t u0, uint32_t u1) {
+    ut_i32x4 f;
+    const uint32_t u[2] = {u0, u1};
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const uint32_t lo = (u[j] << 4) & 0xF0F0F0F0u, hi = u[j] & 0xF0F0F0F0u;
+        f[2 * j] = (int)__builtin_amdgcn_perm(hi, lo, 0x05010400u);
+        f[2 * j + 1] = (int)__builtin_amdgcn_perm(hi, lo, 0x07030602u);
+    }
+    return f;
+}
+// The A operand of matrix instruction s: 16 codes per lane.
 template <int FMT, int TO>
 __device__ __forceinline__ ut_i32x4 gemm_frag_a(const GemmA<FMT, TO> &a, int t, int s) {
     ut_i32x4 f;
@@ -87,13 +98,7 @@ __device__ __forceinline__ ut_i32x4 gemm_frag_a(const GemmA<FMT, TO> &a, int t, 
         f[0] = (int)v.x; f[1] = (int)v.y; f[2] = (int)v.z; f[3] = (int)v.w;
     } else {
         const uint4 v = a.v[t][0];
-        const uint32_t u[2] = {s ? v.z : v.x, s ? v.w : v.y};
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const uint32_t lo = (u[j] << 4) & 0xF0F0F0F0u, hi = u[j] & 0xF0F0F0F0u;
-            f[2 * j] = (int)__builtin_amdgcn_perm(hi, lo, 0x05010400u);
-            f[2 * j + 1] = (int)__builtin_amdgcn_perm(hi, lo, 0x07030602u);
-        }
+        f = s ? gemm_i4_codes(v.z, v.w) : gemm_i4_codes(v.x, v.y);
     }
     return f;
 }
@@ -174,6 +179,152 @@ __device__ __forceinline__ void gemm_tile(const GemmRows<TO> &rows, int64_t len,
             }
         }
     }
+}
+
+// ------------------------------------------------ tile through LDS ---
+// The same tile with the weights through LDS too, for launches that the
+// matrix cores bound: a lane's direct weight load takes 16 bytes of its own
+// row, so each 16 lanes touch 16 cache lines, and at 512 rows those lookups
+// held the direct tile at a quarter of the matrix rate.  Here both operands
+// are copied by global_load_lds (no registers) in stages of S columns, one
+// in flight while one is computed on, and WO x WM waves share them: each
+// wave TO tiles of 16 weight rows against 16 TM activation rows.  LDS has
+// 64 banks: a staged row's 16-byte chunks are XOR-swizzled so that the 16
+// rows a lane group reads take 16 different slots of 256 bytes.
+template <int FMT, int TO, int TM, int WO, int WM, int S> struct GemmLds {
+    static constexpr int kThreads = 64 * WO * WM;
+    static constexpr int kARows = 16 * TO * WO, kBRows = 48 * TM * WM;
+    static constexpr int kAC = FMT == UT_FMT_INT8 ? S / 16 : S / 32, kBC = S / 16;  // chunks of a row
+    static constexpr int kA = kARows * kAC, kB = kBRows * kBC;  // chunks of a stage
+    static constexpr int kNA = kA / kThreads, kNB = kB / kThreads;
+    static_assert(kA % kThreads == 0 && kB % kThreads == 0, "whole copies");
+    uint4 a[kA], b[kB];
+};
+// Chunk c of a row of C chunks sits at slot c ^ gemm_swz<C>(row).
+template <int C> __device__ __forceinline__ int gemm_swz(int row) {
+    static_assert(C == 2 || C == 4 || C == 8, "rows of 32, 64 or 128 bytes");
+    return (row / (16 / C)) & (C - 1);
+}
+
+// This thread's copy sources at column 0 (row pointers are the caller's);
+// aoff: the A chunk's byte offset in its row's step.
+template <int FMT, int TO, int TM, int WO, int WM, int S> struct GemmSrc {
+    using L = GemmLds<FMT, TO, TM, WO, WM, S>;
+    const uint8_t *a[L::kNA];
+    const int8_t *b[L::kNB];
+    int aoff;
+};
+template <int FMT, int TO, int TM, int WO, int WM, int S, typename ARow, typename BRow>
+__device__ __forceinline__ void gemm_src(GemmSrc<FMT, TO, TM, WO, WM, S> &s, ARow &&arow,
+                                         BRow &&brow) {
+    using L = GemmLds<FMT, TO, TM, WO, WM, S>;
+    const int tid = threadIdx.x;
+#pragma unroll
+    for (int i = 0; i < L::kNA; i++) {
+        const int c = tid + i * L::kThreads, row = c / L::kAC, ph = c % L::kAC;
+        s.a[i] = arow(row);
+        // a copy covers a multiple of 16 rows, so every copy's chunk offset
+        // is the same
+        if (i == 0) s.aoff = (ph ^ gemm_swz<L::kAC>(row)) * 16;
+    }
+#pragma unroll
+    for (int i = 0; i < L::kNB; i++) {
+        const int c = tid + i * L::kThreads, row = c / L::kBC, n = row / 48, x = row - 48 * n;
+        s.b[i] = brow(16 * n + (x & 15), x >> 4) + ((c % L::kBC) ^ gemm_swz<L::kBC>(row)) * 16;
+    }
+}
+
+// This wave's copies landed, then the workgroup's barrier.  (The builtin and
+// not inline asm: the compiler then knows that the stage has landed, and
+// does not wait for the next stage's copies before reading it.)
+__device__ __forceinline__ void gemm_wait_copies() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(7 << 4);  // vmcnt(0) lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+template <int FMT, int TO, int TM, int WO, int WM, int S>
+__device__ __forceinline__ void gemm_tile_lds(const GemmSrc<FMT, TO, TM, WO, WM, S> &src,
+                                              int64_t len, int64_t kb, int64_t ke,
+                                              GemmLds<FMT, TO, TM, WO, WM, S> &s0,
+                                              GemmLds<FMT, TO, TM, WO, WM, S> &s1,
+                                              ut_i32x4 (&acc)[TO][TM][3]) {
+    using L = GemmLds<FMT, TO, TM, WO, WM, S>;
+    const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, q = lane >> 4, wave = tid >> 6;
+    const int wo = wave % WO, wm = wave / WO;
+#pragma unroll
+    for (int t = 0; t < TO; t++)
+#pragma unroll
+        for (int n = 0; n < TM; n++)
+#pragma unroll
+            for (int p = 0; p < 3; p++) acc[t][n][p] = ut_i32x4{0, 0, 0, 0};
+    const int w64 = __builtin_amdgcn_readfirstlane(wave) * 64;
+    const int n = (int)((ke - kb) / S);  // K slices are whole 128-column steps
+    // (past the last stage: the last one again, into a buffer nothing reads)
+    auto copy = [&](L &s, int i) {
+        const int64_t k = kb + (int64_t)(i < n ? i : n - 1) * S;
+        // columns past K meet zero digits: any in-bounds weight chunk will do
+        int64_t off = (FMT == UT_FMT_INT8 ? k : k / 2) + src.aoff;
+        off = off < len ? off : len - 16;
+#pragma unroll
+        for (int j = 0; j < L::kNA; j++)
+            __builtin_amdgcn_global_load_lds(
+                (const void *)(src.a[j] + off),
+                (__attribute__((address_space(3))) void *)(s.a + j * L::kThreads + w64), 16, 0, 0);
+#pragma unroll
+        for (int j = 0; j < L::kNB; j++)
+            __builtin_amdgcn_global_load_lds(
+                (const void *)(src.b[j] + k),
+                (__attribute__((address_space(3))) void *)(s.b + j * L::kThreads + w64), 16, 0, 0);
+    };
+    auto compute = [&](const L &s) {
+#pragma unroll
+        for (int h = 0; h < S / 64; h++) {
+            const int c = 4 * h + q;  // this lane's 16 columns of the stage
+            ut_i32x4 f[TO], w[TM][3];
+#pragma unroll
+            for (int t = 0; t < TO; t++) {
+                const int row = (wo * TO + t) * 16 + r;
+                if constexpr (FMT == UT_FMT_INT8) {
+                    const uint4 v = s.a[row * L::kAC + (c ^ gemm_swz<L::kAC>(row))];
+                    f[t] = ut_i32x4{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
+                } else {
+                    const uint2 v = ((const uint2 *)&s.a[row * L::kAC + ((c >> 1) ^ gemm_swz<L::kAC>(row))])[c & 1];
+                    f[t] = gemm_i4_codes(v.x, v.y);
+                }
+            }
+#pragma unroll
+            for (int m = 0; m < TM; m++)
+#pragma unroll
+                for (int p = 0; p < 3; p++) {
+                    const int row = ((wm * TM + m) * 3 + p) * 16 + r;
+                    const uint4 v = s.b[row * L::kBC + (c ^ gemm_swz<L::kBC>(row))];
+                    w[m][p] = ut_i32x4{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
+                }
+#pragma unroll
+            for (int m = 0; m < TM; m++)
+#pragma unroll
+                for (int p = 0; p < 3; p++)
+#pragma unroll
+                    for (int t = 0; t < TO; t++)
+                        acc[t][m][p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(f[t], w[m][p], acc[t][m][p], 0, 0, 0);
+        }
+    };
+    // step i: its stage has landed, the other buffer is read and gets the next
+    auto step = [&](L &s, L &other, int i) {
+        gemm_wait_copies();
+        copy(other, i + 1);
+        compute(s);
+    };
+    copy(s0, 0);
+    int i = 0;
+    for (; i + 2 <= n; i += 2) {
+        step(s0, s1, i);
+        step(s1, s0, i + 1);
+    }
+    if (i < n) step(s0, s1, i);
+    gemm_wait_copies();  // no copy outlives the tile
 }
 
 // The exact total of one accumulator element.
