@@ -1,4 +1,4 @@
-"""The grouped expert products (ut_moe_rows.hip: five or more rows) against
+"""The grouped expert products (ut_moe_rows.hip: six or more rows, int8 eight) against
 one-to-four-row calls of the same rows, bit for bit: every total is an exact
 integer and SiLU and the choices' sum run in the same order, so the tolerance
 is zero.  (Four-row calls are checked against the oracle in test_gpu_moe.py.)
@@ -42,7 +42,7 @@ def test_rows_equal_four_row_calls(ctx, fmt, H, I, dtype):
     w = dev(rng.random((rows, k)).astype(np.float32))
     x = dev(rng.standard_normal((rows, H)).astype(np.float32)).to(dtype)
     want = by_fours(tbl, ids, w, x)
-    for n in (5, 8, 41):
+    for n in (5, 6, 8, 41):
         got = tbl.moe_experts(ids[:n].contiguous(), w[:n].contiguous(), x[:n].contiguous())
         assert torch.equal(got, want[:n]), n
 

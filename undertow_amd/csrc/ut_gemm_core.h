@@ -196,8 +196,8 @@ template <int FMT, int TO, int TM, int WO, int WM, int S> struct GemmLds {
     static constexpr int kARows = 16 * TO * WO, kBRows = 48 * TM * WM;
     static constexpr int kAC = FMT == UT_FMT_INT8 ? S / 16 : S / 32, kBC = S / 16;  // chunks of a row
     static constexpr int kA = kARows * kAC, kB = kBRows * kBC;  // chunks of a stage
-    static constexpr int kNA = kA / kThreads, kNB = kB / kThreads;
-    static_assert(kA % kThreads == 0 && kB % kThreads == 0, "whole copies");
+    static constexpr int kNA = kA / kThreads, kNB = (kB + kThreads - 1) / kThreads;
+    static_assert(kA % kThreads == 0 && kB % 64 == 0, "whole copies; a last one of whole waves");
     uint4 a[kA], b[kB];
 };
 // Chunk c of a row of C chunks sits at slot c ^ gemm_swz<C>(row).
@@ -229,7 +229,8 @@ __device__ __forceinline__ void gemm_src(GemmSrc<FMT, TO, TM, WO, WM, S> &s, ARo
     }
 #pragma unroll
     for (int i = 0; i < L::kNB; i++) {
-        const int c = tid + i * L::kThreads, row = c / L::kBC, n = row / 48, x = row - 48 * n;
+        const int t = tid + i * L::kThreads, c = t < L::kB ? t : 0;
+        const int row = c / L::kBC, n = row / 48, x = row - 48 * n;
         s.b[i] = brow(16 * n + (x & 15), x >> 4) + ((c % L::kBC) ^ gemm_swz<L::kBC>(row)) * 16;
     }
 }
@@ -274,9 +275,10 @@ __device__ __forceinline__ void gemm_tile_lds(const GemmSrc<FMT, TO, TM, WO, WM,
                 (__attribute__((address_space(3))) void *)(s.a + j * L::kThreads + w64), 16, 0, 0);
 #pragma unroll
         for (int j = 0; j < L::kNB; j++)
-            __builtin_amdgcn_global_load_lds(
-                (const void *)(src.b[j] + k),
-                (__attribute__((address_space(3))) void *)(s.b + j * L::kThreads + w64), 16, 0, 0);
+            if (L::kB % L::kThreads == 0 || j * L::kThreads + w64 < L::kB)
+                __builtin_amdgcn_global_load_lds(
+                    (const void *)(src.b[j] + k),
+                    (__attribute__((address_space(3))) void *)(s.b + j * L::kThreads + w64), 16, 0, 0);
     };
     auto compute = [&](const L &s) {
 #pragma unroll

@@ -21,9 +21,15 @@ struct MoeTile {
     int32_t expert, pos, n;  // rows pos .. pos + n of the sorted pairs
 };
 
+// The fewest rows: up to five (int4) or seven (int8) most choices name
+// different experts, and the four-row passes' launches are the shorter ones
+// (config 2's block: 5 rows 315 against 328 us, 7 rows 426 against 433, 8
+// rows 489 against 461; int4 5 rows 200 against 205, 6 rows 242 against 228).
+constexpr int64_t kMoeRowsMinI8 = 8, kMoeRowsMinI4 = 6;
+
 bool moe_rows_ok(int fmt, int64_t M, int64_t E, int64_t H, int64_t I) {
-    return M >= kGemmMinRows && (fmt == UT_FMT_INT8 || fmt == UT_FMT_INT4) &&
-           moe_shape_ok(fmt, H, I) && E <= kMoeRowsMaxExperts && H <= 65536 && I <= 65536;
+    return M >= (fmt == UT_FMT_INT8 ? kMoeRowsMinI8 : kMoeRowsMinI4) &&
+           (fmt == UT_FMT_INT8 || fmt == UT_FMT_INT4) && moe_shape_ok(fmt, H, I) && E <= kMoeRowsMaxExperts && H <= 65536 && I <= 65536;
 }
 
 namespace {
@@ -130,38 +136,48 @@ struct MoeRowsArgs {
     float *out;                  // gate/up: h [pairs][I]; down: d [pairs][H]
 };
 
-// The staging chunks' sources for a tile's rows (rowof: tile row -> plane
-// row; rows past the tile repeat its last).
-template <int TM, typename F>
-__device__ __forceinline__ void rows_src(const MoeRowsArgs &a, int n, F &&rowof,
-                                         const int8_t *(&src)[gemm_stage_n<TM>()]) {
-#pragma unroll
-    for (int i = 0; i < gemm_stage_n<TM>(); i++) {
-        const GemmChunk c = gemm_chunk(threadIdx.x + i * kGemmThreads);
-        const int64_t m = rowof(c.m < n ? c.m : n - 1);
-        src[i] = a.pl + (m * 3 + (c.p < 3 ? c.p : 0)) * a.kp + c.off;
-    }
+// Weight tiles of 16 rows per wave, columns per LDS stage.  Four workgroups
+// of 128 weight rows per CU (int4; 40 KB of LDS each): config 2's int4 block
+// at 500 rows 1,315 us with direct weight loads, 1,239 so; at 64 rows 725 ->
+// 669, at 5 rows 235 -> 205.  256-row workgroups, two per CU: 1,279 / 660 /
+// 224; stages of 64 columns: 1,564 / 817 / 270.  Up to 64 rows the weights'
+// read bounds it (222 experts, 4.9 GB, at 64 rows); at 500 the read (0.83 ms)
+// and the padded tiles' matrix work (23 of 32 rows on average) together do.
+constexpr int kMrTO = 2, kMrS = 128;
+constexpr int kMrRows = 64 * kMrTO;
+
+// A workgroup's tile: weight rows wrow(row of the tile) against a tile's
+// activation rows arow(m) (rows past the tile repeat its last).
+template <int FMT, int TM, typename W, typename A>
+__device__ __forceinline__ void rows_tile(const MoeRowsArgs &a, int n, int64_t len, W &&wrow,
+                                          A &&arow, void *s0, void *s1, ut_i32x4 (&acc)[kMrTO][TM][3]) {
+    using L = GemmLds<FMT, kMrTO, TM, 4, 1, kMrS>;
+    GemmSrc<FMT, kMrTO, TM, 4, 1, kMrS> src;
+    gemm_src<FMT, kMrTO, TM, 4, 1, kMrS>(src, wrow, [&](int m, int p) {
+        return a.pl + (arow(m < n ? m : n - 1) * 3 + p) * a.kp;
+    });
+    gemm_tile_lds<FMT, kMrTO, TM, 4, 1, kMrS>(src, len, 0, a.kp, *(L *)s0, *(L *)s1, acc);
 }
 
-// Gate and up of 128 h rows against a tile's rows: wave w's four weight
-// tiles are gate and up rows of the same 32 h rows, so silu(g) * u is formed
-// from one lane's accumulators.
+// Gate and up of kMrRows / 2 h rows against a tile's rows: a wave's weight
+// tiles are gate rows and up rows of the same h rows, so silu(g) * u is
+// formed from one lane's accumulators.
 template <int FMT, int TM>
 __device__ __forceinline__ void rows_gate_up(const MoeRowsArgs &a, const MoeTile &t, int rt,
-                                             uint4 *lds) {
-    const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, q = lane >> 4;
-    const int64_t h0 = (int64_t)rt * 128 + (tid >> 6) * 32;
-    GemmRows<4> rows;
-    rows.end = nullptr;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int64_t h = h0 + 16 * (i & 1) + r;
-        rows.row[i] = (i < 2 ? a.tbl.gate_w : a.tbl.up_w)[t.expert] + (h < a.I ? h : a.I - 1) * a.row_h;
-    }
-    const int8_t *src[gemm_stage_n<TM>()];
-    rows_src<TM>(a, t.n, [&](int m) { return (int64_t)(a.list[t.pos + m] / a.k); }, src);
-    ut_i32x4 acc[4][TM][3];
-    gemm_tile<FMT, 4, TM, false>(rows, a.row_h, 0, a.kp, src, lds, acc);
+                                             void *s0, void *s1) {
+    constexpr int G = kMrTO / 2;  // gate tiles of a wave
+    const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4, wave = threadIdx.x >> 6;
+    const int64_t hb = (int64_t)rt * (kMrRows / 2), h0 = hb + wave * (16 * G);
+    const uint8_t *gw = a.tbl.gate_w[t.expert], *uw = a.tbl.up_w[t.expert];
+    ut_i32x4 acc[kMrTO][TM][3];
+    rows_tile<FMT, TM>(
+        a, t.n, a.row_h,
+        [&](int row) {
+            const int x = row / 16, i = x % kMrTO;  // tile of the workgroup, of its wave
+            const int64_t h = hb + (x / kMrTO * G + i % G) * 16 + row % 16;
+            return (i < G ? gw : uw) + (h < a.I ? h : a.I - 1) * a.row_h;
+        },
+        [&](int m) { return (int64_t)(a.list[t.pos + m] / a.k); }, s0, s1, acc);
     const float *gs = a.tbl.gate_s[t.expert], *us = a.tbl.up_s[t.expert];
 #pragma unroll
     for (int n = 0; n < TM; n++) {
@@ -170,14 +186,14 @@ __device__ __forceinline__ void rows_gate_up(const MoeRowsArgs &a, const MoeTile
         const int32_t e = gemm_exp<FMT>(a.exps[a.list[t.pos + m] / a.k]);
         float *ho = a.out + (int64_t)(t.pos + m) * a.I;
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
+        for (int i = 0; i < G; i++) {
             const int64_t h = h0 + 16 * i + 4 * q;
             if (h >= a.I) continue;  // I % 16 == 0: four columns or none
             float v[4];
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 const float g = int_total_to_f32(gemm_total(acc[i][n], j), e, ld_global_f32(gs + h + j));
-                const float u = int_total_to_f32(gemm_total(acc[i + 2][n], j), e, ld_global_f32(us + h + j));
+                const float u = int_total_to_f32(gemm_total(acc[i + G][n], j), e, ld_global_f32(us + h + j));
                 // silu(g) * u (undertow-quant/src/lib.rs:121; model.rs:241-247)
                 v[j] = __fmul_rn(g / (1.0f + expf(-g)), u);
             }
@@ -187,20 +203,16 @@ __device__ __forceinline__ void rows_gate_up(const MoeRowsArgs &a, const MoeTile
 }
 
 template <int FMT, int TM>
-__device__ __forceinline__ void rows_down(const MoeRowsArgs &a, const MoeTile &t, int rt, uint4 *lds) {
-    const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, q = lane >> 4;
-    const int64_t o0 = (int64_t)rt * 256 + (tid >> 6) * 64;
-    GemmRows<4> rows;
-    rows.end = nullptr;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int64_t o = o0 + 16 * i + r;
-        rows.row[i] = a.tbl.down_w[t.expert] + (o < a.H ? o : a.H - 1) * a.row_i;
-    }
-    const int8_t *src[gemm_stage_n<TM>()];
-    rows_src<TM>(a, t.n, [&](int m) { return (int64_t)(t.pos + m); }, src);
-    ut_i32x4 acc[4][TM][3];
-    gemm_tile<FMT, 4, TM, false>(rows, a.row_i, 0, a.kp, src, lds, acc);
+__device__ __forceinline__ void rows_down(const MoeRowsArgs &a, const MoeTile &t, int rt, void *s0,
+                                          void *s1) {
+    const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4, wave = threadIdx.x >> 6;
+    const int64_t ob = (int64_t)rt * kMrRows, o0 = ob + wave * (16 * kMrTO);
+    const uint8_t *dw = a.tbl.down_w[t.expert];
+    ut_i32x4 acc[kMrTO][TM][3];
+    rows_tile<FMT, TM>(
+        a, t.n, a.row_i,
+        [&](int row) { return dw + (ob + row < a.H ? ob + row : a.H - 1) * a.row_i; },
+        [&](int m) { return (int64_t)(t.pos + m); }, s0, s1, acc);
     const float *ds = a.tbl.down_s[t.expert];
 #pragma unroll
     for (int n = 0; n < TM; n++) {
@@ -209,7 +221,7 @@ __device__ __forceinline__ void rows_down(const MoeRowsArgs &a, const MoeTile &t
         const int32_t e = gemm_exp<FMT>(a.exps[t.pos + m]);
         float *po = a.out + (int64_t)(t.pos + m) * a.H;
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
+        for (int i = 0; i < kMrTO; i++) {
             const int64_t o = o0 + 16 * i + 4 * q;
             if (o >= a.H) continue;  // H % 16 == 0
             float v[4];
@@ -227,17 +239,18 @@ __device__ __forceinline__ void rows_down(const MoeRowsArgs &a, const MoeTile &t
 // rows per expert the weights are read once and at most half of the matrix
 // work is padding.
 template <int FMT, bool DOWN>
-__global__ __launch_bounds__(kGemmThreads, 2) void k_moe_rows(MoeRowsArgs a, int nrt) {
-    __shared__ uint4 lds[gemm_lds_uint4<2>()];
+__global__ __launch_bounds__(kGemmThreads, FMT == UT_FMT_INT4 ? 4 : 2) void k_moe_rows(MoeRowsArgs a, int nrt) {
+    // two objects: the compiler then knows which one a copy in flight fills
+    __shared__ GemmLds<FMT, kMrTO, 2, 4, 1, kMrS> s0, s1;
     const int ti = blockIdx.x / nrt, rt = blockIdx.x - ti * nrt;
     if (ti >= *a.ntiles) return;
     const MoeTile t = a.tiles[ti];
     if constexpr (DOWN) {
-        if (t.n <= 16) rows_down<FMT, 1>(a, t, rt, lds);
-        else rows_down<FMT, 2>(a, t, rt, lds);
+        if (t.n <= 16) rows_down<FMT, 1>(a, t, rt, &s0, &s1);
+        else rows_down<FMT, 2>(a, t, rt, &s0, &s1);
     } else {
-        if (t.n <= 16) rows_gate_up<FMT, 1>(a, t, rt, lds);
-        else rows_gate_up<FMT, 2>(a, t, rt, lds);
+        if (t.n <= 16) rows_gate_up<FMT, 1>(a, t, rt, &s0, &s1);
+        else rows_gate_up<FMT, 2>(a, t, rt, &s0, &s1);
     }
 }
 
@@ -274,7 +287,7 @@ __global__ __launch_bounds__(256) void k_moe_rows_combine(const int32_t *__restr
 
 int32_t launch_moe_rows(ut_ctx *ctx, const MoeRows &c, void *scratch) {
     // (a prompt's last call may hold fewer rows than moe_rows_ok asks)
-    if (c.M < 1 || !moe_rows_ok(c.fmt, kGemmMinRows, c.E, c.H, c.I) || c.M > moe_rows_chunk(c.k) || c.k < 1) {
+    if (c.M < 1 || !moe_rows_ok(c.fmt, kMoeRowsMinI8, c.E, c.H, c.I) || c.M > moe_rows_chunk(c.k) || c.k < 1) {
         set_error(ctx, "moe_rows: %lld rows of format %d not supported", (long long)c.M, c.fmt);
         return UT_ERR_ARG;
     }
@@ -325,10 +338,10 @@ int32_t launch_moe_rows(ut_ctx *ctx, const MoeRows &c, void *scratch) {
         timing_end(ctx, tk);
         return launch_check(ctx, name);
     };
-    UT_TRY(launch("moe_rows_gate_up", xp, h, c.I, 128, false));
+    UT_TRY(launch("moe_rows_gate_up", xp, h, c.I, kMrRows / 2, false));
     const DigitPlanes hp = planes_view(b + L.hp, n, c.I);
     UT_TRY(launch_planes(ctx, h, c.I, n, c.I, hp));
-    UT_TRY(launch("moe_rows_down", hp, d, c.H, 256, true));
+    UT_TRY(launch("moe_rows_down", hp, d, c.H, kMrRows, true));
     tok = timing_begin(ctx, "moe_rows_combine");
     hipLaunchKernelGGL(k_moe_rows_combine, dim3((unsigned)((c.H / 4 + 255) / 256), (unsigned)c.M),
                        dim3(256), 0, ctx->stream, pos, c.weights, d, c.k, c.H, c.shared, c.out,
