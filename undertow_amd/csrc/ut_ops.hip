@@ -382,6 +382,8 @@ int32_t launch_absorb_q(ut_ctx *ctx, const ut_qtensor *kv_b, const float *q, int
         set_error(ctx, "absorb: kv_lora_rank %lld must be a multiple of 4", (long long)L);
         return UT_ERR_SHAPE;
     }
+    if (!ctx->step_pos && absorb_q_rows_ok(kv_b, q, rows, nope, rope, pos_base))
+        return launch_absorb_q_rows(ctx, kv_b, q, rows, heads, rope, vh, qabs, qrope, pos_base, table);
     constexpr int RB = 4;
     const int64_t kvh = nope + vh;
     // LDS-staged kernel: 128- (or 64-) column blocks, 16-byte aligned rows,
@@ -573,6 +575,8 @@ int32_t launch_absorb_v(ut_ctx *ctx, const ut_qtensor *kv_b, const float *clat, 
         set_error(ctx, "absorb: kv_lora_rank %lld must be a multiple of 4", (long long)L);
         return UT_ERR_SHAPE;
     }
+    if (!vmax && absorb_v_rows_ok(kv_b, clat, rows))
+        return launch_absorb_v_rows(ctx, kv_b, clat, rows, heads, nope, vh, out);
     constexpr int RB = 4;
     const uint8_t *w = (const uint8_t *)kv_b->payload;
     if (kv_b->fmt == UT_FMT_INT8 && L == 512 && kv_b->row_bytes % 16 == 0 &&
