@@ -59,6 +59,28 @@ def test_gemm_largest_codes_do_not_overflow(ctx, fmt):
     assert np.array_equal(run(ctx, q, x), gemv_closed_form(fmt, payload, scales, o, i, x))
 
 
+# one-launch GEMV of few outputs: pieces that fill no wave, the widest rows,
+# outputs past a workgroup's four, the largest output counts and the first
+# beyond them
+@pytest.mark.parametrize("fmt", [INT8, INT4])
+@pytest.mark.parametrize("o,i", [(1, 32), (5, 96), (7, 2080), (1024, 1024), (1025, 4096), (2048, 992),
+                                 (2049, 128), (6, 8192), (6, 8224)])
+def test_few_outputs_are_the_closed_form(ctx, fmt, o, i):
+    import undertow_amd as U
+    rng = np.random.default_rng(o + i + fmt)
+    payload, scales = rand_qtensor(rng, fmt, o, i)
+    q = U.QTensor(ctx, fmt, payload, scales, o, i)
+    x = rng.standard_normal((4, i)).astype(np.float32)
+    x[2] *= np.float32(1e-38)  # digits by the general scaling
+    want = gemv_closed_form(fmt, payload, scales, o, i, x)
+    for seq in (1, 2, 3, 4):
+        assert np.array_equal(run(ctx, q, x[:seq]), want[:seq]), seq
+    bad = x[:2].copy()
+    bad[1, i - 1] = np.nan
+    got = run(ctx, q, bad)
+    assert np.isnan(got[1]).all() and np.array_equal(got[0], want[0])
+
+
 def test_gemm_nonfinite_rows_are_nan(ctx):
     import undertow_amd as U
     rng = np.random.default_rng(5)

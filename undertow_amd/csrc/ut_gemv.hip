@@ -883,7 +883,123 @@ __global__ __launch_bounds__(kGemvThreads) void k_gemv_i8_rowsplit(PlainArgs a) 
     }
 }
 
+// One to four f32 rows against an int8 / int4 weight of few output rows in
+// one launch: the rowsplit layout (a workgroup takes 4 output rows, lane
+// group g row g, the four waves interleaved 16-lane runs of 16-byte pieces),
+// with each activation row digitised in registers by the lanes that multiply
+// it, from a maximum that every workgroup takes over the whole row.  The
+// totals are the digit GEMVs', exact integers.
+constexpr int kDirectCols = 128;  // activation columns a lane holds
+template <int FMT>
+__global__ __launch_bounds__(kGemvThreads) void k_gemv_direct(PlainArgs a, int M) {
+    constexpr int LC = FMT == UT_FMT_INT8 ? 16 : 32;  // columns of a 16-byte piece
+    constexpr int NS = kDirectCols / LC;              // pieces a lane may hold
+    constexpr int PL = FMT == UT_FMT_INT8 ? 3 : 6, WC = FMT == UT_FMT_INT8 ? 4 : 8;
+    __shared__ uint32_t red[4];
+    __shared__ int64_t part[4][4];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, s = lane & 15;
+    const int64_t row = (int64_t)blockIdx.x * 4 + g;
+    const uint8_t *wr = plain_row(a, row < a.O ? row : a.O - 1);
+    const int units = (int)(a.K / LC), u0 = 16 * wave + s;  // pieces u0, u0 + 64, ...
+    uint4 w[NS];
+#pragma unroll
+    for (int u = 0; u < NS; u++)
+        if (u0 + 64 * u < units) w[u] = ld_weights(wr + 16 * (u0 + 64 * u));
+    for (int m = 0; m < M; m++) {
+        const float *x = a.x.xf + m * a.x.ldx;
+        float v[NS][LC];
+        uint32_t mx = 0;
+#pragma unroll
+        for (int u = 0; u < NS; u++)
+            if (u0 + 64 * u < units)
+#pragma unroll
+                for (int j = 0; j < LC; j += 4) {
+                    const float4 t = ld_global<float4>(x + (int64_t)(u0 + 64 * u) * LC + j);
+                    v[u][j] = t.x; v[u][j + 1] = t.y; v[u][j + 2] = t.z; v[u][j + 3] = t.w;
+                }
+#pragma unroll
+        for (int u = 0; u < NS; u++)
+            if (u0 + 64 * u < units)
+#pragma unroll
+                for (int j = 0; j < LC; j++) mx = max(mx, __float_as_uint(fabsf(v[u][j])));
+        mx = block_reduce(mx, [](uint32_t p, uint32_t q) { return p > q ? p : q; }, red);
+        const bool bad = mx >= 0x7f800000u;
+        int E = 0;
+        if (!bad && mx != 0) (void)frexpf(__uint_as_float(mx), &E);
+        const int sh = bad ? INT32_MIN : 22 - E;
+        int32_t acc[PL];
+#pragma unroll
+        for (int p = 0; p < PL; p++) acc[p] = 0;
+#pragma unroll
+        for (int u = 0; u < NS; u++) {
+            if (u0 + 64 * u >= units) continue;
+            const uint32_t ww[4] = {w[u].x, w[u].y, w[u].z, w[u].w};
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                uint32_t d[PL];
+                digit_words<FMT>(&v[u][WC * q], WC, sh, d);
+#pragma unroll
+                for (int p = 0; p < PL; p++)
+                    acc[p] = FMT == UT_FMT_INT8
+                                 ? __builtin_amdgcn_sdot4((int)ww[q], (int)d[p], acc[p], false)
+                                 : __builtin_amdgcn_sdot8((int)ww[q], (int)d[p], acc[p], false);
+            }
+        }
+        int64_t t = 0;
+#pragma unroll
+        for (int p = PL - 1; p >= 0; p--) t = t * (FMT == UT_FMT_INT8 ? 256 : 16) + acc[p];
+#pragma unroll
+        for (int off = 8; off >= 1; off >>= 1) t += shfl_xor_i64(t, off);
+        if (s == 0) part[wave][g] = t;
+        __syncthreads();
+        const int64_t r = (int64_t)blockIdx.x * 4 + tid;
+        if (tid < 4 && r < a.O) {
+            const int64_t S = part[0][tid] + part[1][tid] + part[2][tid] + part[3][tid];
+            plain_out(a, m, r)[0] = int_total_to_f32(S, bad ? INT32_MIN : E - 22, plain_scale(a, r));
+        }
+        if (m + 1 < M) __syncthreads();  // part is written again
+    }
+}
+
 static bool fast_ok(const ut_qtensor *w);
+
+// Taken where one launch saves more than digitising in every workgroup
+// costs: the whole weight in one pass of resident workgroups (512 of 4 rows;
+// int4 digits cost twice as much, 256), and rows that follow one another
+// hold few columns.  One row of int8 576 x 7168: 13.3 us with digitise, GEMV
+// and split sum, 7.7 so; 2048 x 8192 16.5 -> 12.9 (4096 x 7168: 16.2 against
+// 20.3); int4 1024 x 7168 12.1 -> 9.7 (1536 x 7168: 12.7 against 14.0); two
+// rows of int8 1024 x 4096 10.7 -> 9.5 (576 x 7168: 13.4 against 12.4 but
+// 1536 x 7168 14.7 against 16.7); four of 1024 x 256 9.7 -> 7.9 (2048 x 2048:
+// 10.8 against 12.6).
+static bool gemv_direct_ok(const ut_qtensor *w, const float *x, int64_t M) {
+    if (w->fmt != UT_FMT_INT8 && w->fmt != UT_FMT_INT4) return false;
+    return M >= 1 && M <= 4 && M * w->in_dim <= (M <= 2 ? 64 : 32) * kDirectCols && fast_ok(w) &&
+           ((uintptr_t)x & 15) == 0 && w->out_dim <= (w->fmt == UT_FMT_INT8 ? 2048 : 1024);
+}
+
+static int32_t launch_gemv_direct(ut_ctx *ctx, const ut_qtensor *w, const float *x, int64_t M,
+                                  float *out, int64_t ldo) {
+    PlainArgs a{};
+    a.w = a.w2 = (const uint8_t *)w->payload;
+    a.scales = a.scales2 = w->scales;
+    a.O = a.O1 = w->out_dim;
+    a.K = w->in_dim;
+    a.row_bytes = w->row_bytes;
+    a.out = a.out2 = out;
+    a.ldo = a.ldo2 = ldo;
+    a.x.xf = x;
+    a.x.ldx = w->in_dim;
+    a.ks = 1;
+    const dim3 grid((unsigned)((a.O + 3) / 4));
+    int tok = timing_begin(ctx, "gemv_direct");
+    if (w->fmt == UT_FMT_INT8)
+        hipLaunchKernelGGL(k_gemv_direct<UT_FMT_INT8>, grid, dim3(kGemvThreads), 0, ctx->stream, a, (int)M);
+    else
+        hipLaunchKernelGGL(k_gemv_direct<UT_FMT_INT4>, grid, dim3(kGemvThreads), 0, ctx->stream, a, (int)M);
+    timing_end(ctx, tok);
+    return launch_check(ctx, "k_gemv_direct");
+}
 
 bool gemv_rowsplit_ok(const GemvArgs &ga) {
     const ut_qtensor *w = ga.w;
@@ -1797,6 +1913,8 @@ extern "C" int32_t ut_qtensor_matmul(ut_ctx *ctx, const ut_qtensor *qt, float *o
     // Int8 { .. } if fast_int8_enabled() (qtensor.rs:385-398)
     if (qt->fmt == UT_FMT_INT8 && ctx->fast_int8)
         return matmul_fast_i8(ctx, qt, out_dev, qt->out_dim, 0, x_dev, seq);
+    if (gemv_direct_ok(qt, x_dev, seq))
+        return launch_gemv_direct(ctx, qt, x_dev, seq, out_dev, qt->out_dim);
     if (gemm_ok(qt, seq)) {
         ScratchPlan plan;
         plan.add(planes_bytes(seq, qt->in_dim));
