@@ -42,8 +42,12 @@ constexpr int64_t kGemmMinRows = 5;
 bool gemm_ok(const ut_qtensor *w, int64_t M);
 // out[m, o] (+)= x[m] . w[o] for M digitised rows; the values are the
 // GEMVs', bit for bit.
+// (w2: a second weight of the same format and width, gemm_pair_ok, into out2
+// in the same launch.)
+bool gemm_pair_ok(const ut_qtensor *w, const ut_qtensor *w2, int64_t M);
 int32_t launch_gemm(ut_ctx *ctx, const ut_qtensor *w, const DigitPlanes &x, int64_t M, float *out,
-                    int64_t ldo, int accumulate);
+                    int64_t ldo, int accumulate, const ut_qtensor *w2 = nullptr,
+                    float *out2 = nullptr, int64_t ldo2 = 0);
 
 // f32 weights (ut_gemm_f32.hip), each output's products added in the order
 // of the GEMV that fewer rows take.  gemv_f32_split: that GEMV's K split, of

@@ -150,28 +150,36 @@ int32_t launch_silu_planes(ut_ctx *ctx, const float *g, const float *u, int64_t 
 }
 
 // --------------------------------------------------------------- GEMM ---
-struct GemmArgs {
-    const uint8_t *w;
+// One or two weights of one format and width against the same rows.
+struct GemmWeight {
+    const uint8_t *w, *end;
     const float *scales;
-    int64_t O, row_bytes;  // weight rows, bytes from one to the next (all of them read)
-    const uint8_t *end;
+    int64_t O;  // weight rows
+    float *out;
+    int64_t ldo;
+};
+struct GemmArgs {
+    GemmWeight w[2];
+    int64_t row_bytes;  // from one weight row to the next (all of them read)
+    int to0;            // weight tiles of w[0]; the launch's others are w[1]'s
     const int8_t *pl;
     int64_t kp;
     const int32_t *exps;
     int64_t M;
-    float *out;
-    int64_t ldo;
     int accumulate;
     // units = weight tiles x K splits; a unit's activation tiles run on one XCD
     int to, tm, ks;
     int64_t kslice;
-    int64_t *part;  // ks > 1: totals [ks][M][O]
+    int64_t *part;  // ks > 1: totals [ks][M][O], w[1]'s rows after w[0]'s
 };
 
-// A wave's finished tile: weight rows o0 .. of activation rows m0 ..
+// A wave's finished tile: rows o0 .. of weight wi, activation rows m0 ..
 template <int FMT, int TO, int TM>
-__device__ __forceinline__ void gemm_store(const GemmArgs &a, const ut_i32x4 (&acc)[TO][TM][3],
-                                           int64_t o0, int64_t m0, int z) {
+__device__ __forceinline__ void gemm_store(const GemmArgs &a, int wi,
+                                           const ut_i32x4 (&acc)[TO][TM][3], int64_t o0, int64_t m0,
+                                           int z) {
+    const GemmWeight &W = a.w[wi];
+    const int64_t po0 = wi ? a.w[0].O : 0, OT = a.w[0].O + a.w[1].O;
     const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
 #pragma unroll
     for (int t = 0; t < TO; t++) {
@@ -179,23 +187,23 @@ __device__ __forceinline__ void gemm_store(const GemmArgs &a, const ut_i32x4 (&a
 #pragma unroll
         for (int n = 0; n < TM; n++) {
             const int64_t m = m0 + 16 * n + r;
-            if (m >= a.M || o >= a.O) continue;
+            if (m >= a.M || o >= W.O) continue;
             int64_t S[4];
 #pragma unroll
             for (int i = 0; i < 4; i++) S[i] = gemm_total(acc[t][n], i);
             if (a.ks > 1) {
-                int64_t *p = a.part + ((int64_t)z * a.M + m) * a.O + o;
+                int64_t *p = a.part + ((int64_t)z * a.M + m) * OT + po0 + o;
 #pragma unroll
                 for (int i = 0; i < 4; i++)
-                    if (o + i < a.O) p[i] = S[i];
+                    if (o + i < W.O) p[i] = S[i];
                 continue;
             }
             const int32_t e = gemm_exp<FMT>(a.exps[m]);
-            float *po = a.out + m * a.ldo + o;
+            float *po = W.out + m * W.ldo + o;
 #pragma unroll
             for (int i = 0; i < 4; i++)
-                if (o + i < a.O) {
-                    const float v = int_total_to_f32(S[i], e, ld_global_f32(a.scales + o + i));
+                if (o + i < W.O) {
+                    const float v = int_total_to_f32(S[i], e, ld_global_f32(W.scales + o + i));
                     po[i] = a.accumulate ? __fadd_rn(po[i], v) : v;
                 }
         }
@@ -216,7 +224,8 @@ __global__ __launch_bounds__(kGemmThreads, 2) void k_gemm(GemmArgs a) {
     const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
     const int unit = (j / a.tm) * 8 + xcd, mt = j % a.tm;
     if (unit >= a.to * a.ks) return;
-    const int ot = unit % a.to, z = unit / a.to;
+    const int ut = unit % a.to, z = unit / a.to, wi = ut >= a.to0, ot = wi ? ut - a.to0 : ut;
+    const GemmWeight &W = a.w[wi];
     const int tid = threadIdx.x, r = tid & 15;
     const int64_t o0 = (int64_t)ot * (64 * kGemmTO) + (tid >> 6) * (16 * kGemmTO);
     const int64_t m0 = (int64_t)mt * (16 * TM);
@@ -224,9 +233,9 @@ __global__ __launch_bounds__(kGemmThreads, 2) void k_gemm(GemmArgs a) {
 #pragma unroll
     for (int t = 0; t < kGemmTO; t++) {
         const int64_t o = o0 + 16 * t + r;
-        rows.row[t] = a.w + (o < a.O ? o : a.O - 1) * a.row_bytes;
+        rows.row[t] = W.w + (o < W.O ? o : W.O - 1) * a.row_bytes;
     }
-    rows.end = a.end;
+    rows.end = W.end;
     const int8_t *src[gemm_stage_n<TM>()];
 #pragma unroll
     for (int i = 0; i < gemm_stage_n<TM>(); i++) {
@@ -237,7 +246,7 @@ __global__ __launch_bounds__(kGemmThreads, 2) void k_gemm(GemmArgs a) {
     const int64_t kb = z * a.kslice, ke = kb + a.kslice < a.kp ? kb + a.kslice : a.kp;
     ut_i32x4 acc[kGemmTO][TM][3];
     gemm_tile<FMT, kGemmTO, TM, UNAL>(rows, a.row_bytes, kb, ke, src, lds, acc);
-    gemm_store<FMT, kGemmTO, TM>(a, acc, o0, m0, z);
+    gemm_store<FMT, kGemmTO, TM>(a, wi, acc, o0, m0, z);
 }
 
 // More than kGlMinRows rows of 16-byte aligned weights: 128 weight rows x 64
@@ -261,31 +270,35 @@ __global__ __launch_bounds__(64 * kGlWO * kGlWM, 2) void k_gemm_lds(GemmArgs a) 
     const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
     const int unit = (j / a.tm) * 8 + xcd, mt = j % a.tm;
     if (unit >= a.to * a.ks) return;
-    const int ot = unit % a.to, z = unit / a.to;
+    const int ut = unit % a.to, z = unit / a.to, wi = ut >= a.to0, ot = wi ? ut - a.to0 : ut;
+    const GemmWeight &W = a.w[wi];
     const int wave = threadIdx.x >> 6;
     const int64_t ob = (int64_t)ot * L::kARows, mb = (int64_t)mt * (16 * kGlTM * kGlWM);
     GemmSrc<FMT, kGlTO, kGlTM, kGlWO, kGlWM, kGlS> src;
     gemm_src<FMT, kGlTO, kGlTM, kGlWO, kGlWM, kGlS>(
         src,
-        [&](int row) { return a.w + (ob + row < a.O ? ob + row : a.O - 1) * a.row_bytes; },
+        [&](int row) { return W.w + (ob + row < W.O ? ob + row : W.O - 1) * a.row_bytes; },
         [&](int m, int p) { return a.pl + ((mb + m < a.M ? mb + m : a.M - 1) * 3 + p) * a.kp; });
     const int64_t kb = z * a.kslice, ke = kb + a.kslice < a.kp ? kb + a.kslice : a.kp;
     ut_i32x4 acc[kGlTO][kGlTM][3];
     gemm_tile_lds<FMT, kGlTO, kGlTM, kGlWO, kGlWM, kGlS>(src, a.row_bytes, kb, ke, s0, s1, acc);
-    gemm_store<FMT, kGlTO, kGlTM>(a, acc, ob + (wave % kGlWO) * (16 * kGlTO),
+    gemm_store<FMT, kGlTO, kGlTM>(a, wi, acc, ob + (wave % kGlWO) * (16 * kGlTO),
                                   mb + (wave / kGlWO) * (16 * kGlTM), z);
 }
 
 // The K splits' totals summed and scaled (exact integers: any order).
 template <int FMT>
 __global__ __launch_bounds__(256) void k_gemm_sum(GemmArgs a) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x, n = a.M * a.O;
+    const int64_t OT = a.w[0].O + a.w[1].O, i = (int64_t)blockIdx.x * 256 + threadIdx.x, n = a.M * OT;
     if (i >= n) return;
-    const int64_t m = i / a.O, o = i - m * a.O;
+    const int64_t m = i / OT, x = i - m * OT;
+    const int wi = x >= a.w[0].O;
+    const int64_t o = wi ? x - a.w[0].O : x;
+    const GemmWeight &W = a.w[wi];
     int64_t S = 0;
     for (int z = 0; z < a.ks; z++) S += a.part[z * n + i];
-    const float v = int_total_to_f32(S, gemm_exp<FMT>(a.exps[m]), a.scales[o]);
-    float *po = a.out + m * a.ldo + o;
+    const float v = int_total_to_f32(S, gemm_exp<FMT>(a.exps[m]), W.scales[o]);
+    float *po = W.out + m * W.ldo + o;
     *po = a.accumulate ? __fadd_rn(*po, v) : v;
 }
 
@@ -295,38 +308,47 @@ bool gemm_ok(const ut_qtensor *w, int64_t M) {
            w->in_dim >= 1 && w->in_dim <= 65536;
 }
 
+bool gemm_pair_ok(const ut_qtensor *w, const ut_qtensor *w2, int64_t M) {
+    return gemm_ok(w, M) && gemm_ok(w2, M) && w->fmt == w2->fmt && w->in_dim == w2->in_dim &&
+           w->row_bytes == w2->row_bytes &&
+           ((((uintptr_t)w->payload ^ (uintptr_t)w2->payload) & 15) == 0);
+}
+
 int32_t launch_gemm(ut_ctx *ctx, const ut_qtensor *w, const DigitPlanes &x, int64_t M, float *out,
-                    int64_t ldo, int accumulate) {
+                    int64_t ldo, int accumulate, const ut_qtensor *w2, float *out2, int64_t ldo2) {
+    if (w2 && !gemm_pair_ok(w, w2, M)) {
+        set_error(ctx, "gemm: the two weights must share format, width and alignment");
+        return UT_ERR_ARG;
+    }
     GemmArgs a{};
-    a.w = (const uint8_t *)w->payload;
-    a.scales = w->scales;
-    a.O = w->out_dim;
+    auto weight = [](const ut_qtensor *t, float *o, int64_t ld) {
+        const uint8_t *p = (const uint8_t *)t->payload;
+        return GemmWeight{p, p + t->out_dim * t->row_bytes, t->scales, t->out_dim, o, ld};
+    };
     a.row_bytes = w->row_bytes;
-    a.end = a.w + w->out_dim * w->row_bytes;
-    a.pl = x.p;
     a.kp = x.kp;
-    a.exps = x.exps;
-    a.out = out;
-    a.ldo = ldo;
     a.accumulate = accumulate;
     const bool unal = ((uintptr_t)w->payload & 15) != 0 || w->row_bytes % 16 != 0;
     const int64_t cap = unal ? 1 << 20 : 1 << 24;  // rows per launch: grids stay in 31 bits
+    const int64_t O2 = w2 ? w2->out_dim : 0, OT = w->out_dim + O2;
     for (int64_t s0 = 0; s0 < M; s0 += cap) {
         a.M = M - s0 < cap ? M - s0 : cap;
         a.pl = x.p + s0 * 3 * x.kp;
         a.exps = x.exps + s0;
-        a.out = out + s0 * ldo;
+        a.w[0] = weight(w, out + s0 * ldo, ldo);
+        if (w2) a.w[1] = weight(w2, out2 + s0 * ldo2, ldo2);
         const bool big = !unal && a.M > kGlMinRows;
         const int tmr = big ? kGlTM * kGlWM : a.M <= 16 ? 1 : 2;
         const int tor = big ? 16 * kGlTO * kGlWO : 64 * kGemmTO;
-        a.to = (int)((a.O + tor - 1) / tor);
+        a.to0 = (int)((w->out_dim + tor - 1) / tor);
+        a.to = a.to0 + (int)((O2 + tor - 1) / tor);
         a.tm = (int)((a.M + 16 * tmr - 1) / (16 * tmr));
         // split K until the launch has two workgroups per CU, at least two
         // steps each, partials within their buffer
         int64_t ks = (2 * ctx->multiprocessors) / ((int64_t)a.to * a.tm);
         const int64_t steps = a.kp / kGemmStep;
         if (ks > steps / 2) ks = steps / 2;
-        while (ks > 1 && ks * a.M * a.O * 8 > kSplitKPartBytes) ks--;
+        while (ks > 1 && ks * a.M * OT * 8 > kSplitKPartBytes) ks--;
         if (ks < 1) ks = 1;
         a.kslice = (steps + ks - 1) / ks * kGemmStep;
         a.ks = (int)((a.kp + a.kslice - 1) / a.kslice);
@@ -355,7 +377,7 @@ int32_t launch_gemm(ut_ctx *ctx, const ut_qtensor *w, const DigitPlanes &x, int6
 #undef UT_GM
         UT_TRY(launch_check(ctx, "k_gemm"));
         if (a.ks > 1) {
-            const dim3 sg((unsigned)((a.M * a.O + 255) / 256));
+            const dim3 sg((unsigned)((a.M * OT + 255) / 256));
             if (w->fmt == UT_FMT_INT8)
                 hipLaunchKernelGGL(k_gemm_sum<UT_FMT_INT8>, sg, dim3(256), 0, ctx->stream, a);
             else

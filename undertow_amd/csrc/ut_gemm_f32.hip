@@ -197,19 +197,21 @@ int32_t launch_gemm_f32(ut_ctx *ctx, const ut_qtensor *w, const float *x, int64_
 // ------------------------------------------- k_rowdot_f32's order ---
 // The router gate over a prompt: k_rowdot_f32's chains (thread t: columns
 // 4 t + 1024 j in j order), wave sums and wave order, with a workgroup's EPW
-// weight rows held in registers while kRowsPerWG activation rows pass (the
-// next row's loads in flight).  Bound by x's passes through L2 (O / EPW of
-// them).
+// weight rows held in registers while up to kRowsPerWG activation rows pass
+// (the next row's loads in flight).  Bound by x's passes through L2 (O / EPW
+// of them); few weight or activation rows take fewer rows per workgroup, so
+// that their loads' round trips run side by side (48 rows of 8 x 256: 12.8 us
+// at 16 rows a workgroup, 2.7 at one).
 constexpr int kRowsPerWG = 16;
 template <int NJ, int EPW>
 __global__ __launch_bounds__(256) void k_rowdot_f32_rows(const float *__restrict__ w, int64_t K,
                                                          const float *__restrict__ x, int64_t M,
                                                          float *__restrict__ out, int64_t ldo,
-                                                         int64_t O) {
+                                                         int64_t O, int per) {
     __shared__ float red[kRowsPerWG][EPW][4];
     const int tid = threadIdx.x;
-    const int64_t o0 = (int64_t)blockIdx.x * EPW, m0 = (int64_t)blockIdx.y * kRowsPerWG;
-    const int rows = (int)(M - m0 < kRowsPerWG ? M - m0 : kRowsPerWG);
+    const int64_t o0 = (int64_t)blockIdx.x * EPW, m0 = (int64_t)blockIdx.y * per;
+    const int rows = (int)(M - m0 < per ? M - m0 : per);
     float4 wv[EPW][NJ], xv[NJ], xn[NJ];
     auto ld = [&](const float *p, float4 (&v)[NJ]) {
 #pragma unroll
@@ -258,11 +260,13 @@ int32_t launch_rowdot_f32_rows(ut_ctx *ctx, const ut_qtensor *w, const float *x,
     constexpr int EPW = 4;
     const int64_t K = w->in_dim, O = w->out_dim;
     const int nj = (int)((K + 1023) / 1024);
-    const dim3 grid((unsigned)((O + EPW - 1) / EPW), (unsigned)((M + kRowsPerWG - 1) / kRowsPerWG));
+    const int64_t og = (O + EPW - 1) / EPW, want = M * og / (2 * ctx->multiprocessors);
+    const int per = (int)(want < 1 ? 1 : want > kRowsPerWG ? kRowsPerWG : want);
+    const dim3 grid((unsigned)og, (unsigned)((M + per - 1) / per));
     int tok = timing_begin(ctx, "rowdot_f32_rows");
     const float *wp = (const float *)w->payload;
 #define UT_RR(NJ) \
-    hipLaunchKernelGGL((k_rowdot_f32_rows<NJ, EPW>), grid, dim3(256), 0, ctx->stream, wp, K, x, M, out, ldo, O)
+    hipLaunchKernelGGL((k_rowdot_f32_rows<NJ, EPW>), grid, dim3(256), 0, ctx->stream, wp, K, x, M, out, ldo, O, per)
     if (nj <= 1) UT_RR(1);
     else if (nj <= 2) UT_RR(2);
     else if (nj <= 4) UT_RR(4);

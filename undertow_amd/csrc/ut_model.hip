@@ -604,8 +604,12 @@ int32_t mlp_rows(ut_session *s, const MlpW &w, const float *x, const XDigits &xd
         pl = planes_view(s->ws.digits, rows, H);
         UT_TRY(launch_planes(ctx, x, H, rows, H, pl));
     }
-    UT_TRY(launch_gemm(ctx, w.gate, pl, rows, s->ws.mlp_g, I, 0));
-    UT_TRY(launch_gemm(ctx, w.up, pl, rows, s->ws.mlp_u, I, 0));
+    if (gemm_pair_ok(w.gate, w.up, rows)) {
+        UT_TRY(launch_gemm(ctx, w.gate, pl, rows, s->ws.mlp_g, I, 0, w.up, s->ws.mlp_u, I));
+    } else {
+        UT_TRY(launch_gemm(ctx, w.gate, pl, rows, s->ws.mlp_g, I, 0));
+        UT_TRY(launch_gemm(ctx, w.up, pl, rows, s->ws.mlp_u, I, 0));
+    }
     const DigitPlanes hp = planes_view(s->ws.digits, rows, I);
     UT_TRY(launch_silu_planes(ctx, s->ws.mlp_g, s->ws.mlp_u, rows, I, hp));
     return launch_gemm(ctx, w.down, hp, rows, out, H, accumulate);
@@ -932,6 +936,8 @@ int32_t mla_forward(ut_session *s, const LayerW &L, const float *x, const XDigit
     const bool pair = !fast8(s) && L.lora && !gemm_ok(L.kv_a, rows) && L.kv_a->fmt == L.q_a->fmt && L.kv_a->fmt != UT_FMT_F32 &&
                       L.kv_a->in_dim == L.q_a->in_dim && L.kv_a->row_bytes == L.q_a->row_bytes &&
                       gemv_fast_ok(L.kv_a) && gemv_fast_ok(L.q_a);
+    // more rows: both in one product
+    const bool gemm_pair = !fast8(s) && L.lora && gemm_pair_ok(L.kv_a, L.q_a, rows);
     // with the pair's split-K partials deferred, one launch finishes both
     // outputs: q_a's norm + digits and kv_a's cache append
     const bool fused = pair && mla_pre_ok(rows, c.q_lora_rank, Lr, rope);
@@ -988,6 +994,13 @@ int32_t mla_forward(ut_session *s, const LayerW &L, const float *x, const XDigit
         ga.ldo2 = c.q_lora_rank;
         if (fused) ga.defer = &pp;
         UT_TRY(gemv(ctx, ga));
+    } else if (gemm_pair) {
+        DigitPlanes pl;
+        if (!xdigits_planes(xd, c.hidden_size, &pl)) {
+            pl = planes_view(w.digits, rows, c.hidden_size);
+            UT_TRY(launch_planes(ctx, x, c.hidden_size, rows, c.hidden_size, pl));
+        }
+        UT_TRY(launch_gemm(ctx, L.kv_a, pl, rows, w.comp, Lr + rope, 0, L.q_a, w.qa, c.q_lora_rank));
     } else {
         UT_TRY(proj(s, L.kv_a, x, xd, rows, w.comp, Lr + rope));
     }
@@ -1021,7 +1034,7 @@ int32_t mla_forward(ut_session *s, const LayerW &L, const float *x, const XDigit
         UT_TRY(matmul_digits(ctx, L.q_b, w.qa_n, qd, rows, w.q, heads * qh, 0));
     } else {
         if (L.lora) {
-            if (!pair) UT_TRY(proj(s, L.q_a, x, xd, rows, w.qa, c.q_lora_rank));
+            if (!pair && !gemm_pair) UT_TRY(proj(s, L.q_a, x, xd, rows, w.qa, c.q_lora_rank));
             XDigits qd;
             UT_TRY(norm_dig(s, w.qa, c.q_lora_rank, L.q_a_norm, c.q_lora_rank, rows, w.qa_n,
                             c.q_lora_rank, w.digB, dig_flags({L.q_b}, rows), &qd));
