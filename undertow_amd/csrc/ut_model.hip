@@ -1154,18 +1154,6 @@ int32_t run_layer(ut_session *s, const LayerW &L, float *x, int64_t rows, KvCach
     return mlp_add(s, L.shared, w.normed, xd, rows, x, w.moe_out, next);
 }
 
-int32_t check_flags(ut_session *s) {
-    // called after a stream sync: the sticky expert-id error flag
-    ut_ctx *ctx = s->ctx;
-    int32_t f = 0;
-    UT_CHECK_HIP(ctx, hipMemcpy(&f, s->ws.err, 4, hipMemcpyDeviceToHost));
-    if (f) {
-        set_error(ctx, "a routed expert id was out of range or not loaded");
-        return UT_ERR_BAD_EXPERT;
-    }
-    return UT_OK;
-}
-
 int32_t upload_ids(ut_session *s, const int32_t *ids, int64_t n) {
     ut_ctx *ctx = s->ctx;
     void *pin = nullptr;
@@ -1262,13 +1250,28 @@ int32_t prefill_dev(ut_session *s, const int32_t *ids, int64_t n, const int32_t 
     return launch_argmax(ctx, w.logits, n, V, V, w.am, w.argm, w.err, tail, ntail);
 }
 
-int32_t read_argmax(ut_session *s, int64_t n, int32_t *out) {
+// A prefill's argmax rows and the sticky error word behind them (prefill_dev
+// leaves it at am[n]) in one copy and one wait.  logits (optional, host):
+// the rows' logits too, through the pinned buffer where they are few (the
+// runtime stages a copy to pageable memory with a wait of its own).
+constexpr size_t kPinLogits = size_t(256) << 10;
+int32_t read_argmax(ut_session *s, int64_t n, int32_t *out, float *logits = nullptr) {
     ut_ctx *ctx = s->ctx;
+    const size_t ab = ((size_t)(n + 1) * 4 + 63) & ~size_t(63);
+    const size_t lb = logits ? (size_t)n * s->m->c.vocab_size * 4 : 0;
+    const bool staged = lb > 0 && lb <= kPinLogits;
     void *pin = nullptr;
-    UT_TRY(pinned_acquire(ctx, (size_t)n * 4, &pin));
-    UT_CHECK_HIP(ctx, hipMemcpyAsync(pin, s->ws.am, (size_t)n * 4, hipMemcpyDeviceToHost, ctx->stream));
+    UT_TRY(pinned_acquire(ctx, ab + (staged ? lb : 0), &pin));
+    UT_CHECK_HIP(ctx, hipMemcpyAsync(pin, s->ws.am, (size_t)(n + 1) * 4, hipMemcpyDeviceToHost, ctx->stream));
+    if (lb)
+        UT_CHECK_HIP(ctx, hipMemcpyAsync(staged ? (char *)pin + ab : (char *)logits, s->ws.logits, lb,
+                                         hipMemcpyDeviceToHost, ctx->stream));
     UT_CHECK_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    UT_TRY(check_flags(s));
+    if (staged) memcpy(logits, (char *)pin + ab, lb);
+    if (((const int32_t *)pin)[n]) {
+        set_error(ctx, "a routed expert id was out of range or not loaded");
+        return UT_ERR_BAD_EXPERT;
+    }
     memcpy(out, pin, (size_t)n * 4);
     return UT_OK;
 }
@@ -2700,15 +2703,9 @@ void ut_session_free(ut_session *s) {
 int32_t ut_session_prefill(ut_session *s, const int32_t *ids, int64_t n, float *logits_host,
                            int32_t *argmax_host) {
     if (!s || (!ids && n > 0)) return UT_ERR_ARG;
-    ut_ctx *ctx = s->ctx;
     UT_TRY(prefill_dev(s, ids, n));
-    if (logits_host) {
-        UT_CHECK_HIP(ctx, hipMemcpyAsync(logits_host, s->ws.logits,
-                                         (size_t)n * s->m->c.vocab_size * 4,
-                                         hipMemcpyDeviceToHost, ctx->stream));
-    }
     std::vector<int32_t> am((size_t)n);
-    UT_TRY(read_argmax(s, n, am.data()));
+    UT_TRY(read_argmax(s, n, am.data(), logits_host));
     if (argmax_host) memcpy(argmax_host, am.data(), (size_t)n * 4);
     return UT_OK;
 }
