@@ -3,6 +3,8 @@
 // activations and the matrix-core product (ut_gemm_core.h).
 #include "ut_gemm.h"
 
+#include <cmath>
+
 #include "ut_gemm_core.h"
 
 namespace ut {
@@ -296,6 +298,7 @@ __global__ __launch_bounds__(256) void k_gemm_sum(GemmArgs a) {
     const int64_t o = wi ? x - a.w[0].O : x;
     const GemmWeight &W = a.w[wi];
     int64_t S = 0;
+#pragma unroll 8
     for (int z = 0; z < a.ks; z++) S += a.part[z * n + i];
     const float v = int_total_to_f32(S, gemm_exp<FMT>(a.exps[m]), W.scales[o]);
     float *po = W.out + m * W.ldo + o;
@@ -344,10 +347,21 @@ int32_t launch_gemm(ut_ctx *ctx, const ut_qtensor *w, const DigitPlanes &x, int6
         a.to = a.to0 + (int)((O2 + tor - 1) / tor);
         a.tm = (int)((a.M + 16 * tmr - 1) / (16 * tmr));
         // split K until the launch has two workgroups per CU, at least two
-        // steps each, partials within their buffer
+        // steps each, partials within their buffer, and not beyond where a
+        // split's partials (16 bytes a total written and read, at 4 MB a us)
+        // cost more than it takes off the steps (0.8 us each, unaligned rows
+        // 2.5): the sum of both is least at sqrt(steps * step / split)
+        // splits.  37 rows of int4 2048 x 7168 31.0 -> 22.6 us (28 splits were
+        // 17 MB of partials beside an 8 MB weight), 77 rows of int8 1536 x 7168
+        // 31.1 -> 25.1, 128 of 576 x 7168 32.1 -> 25.9; 0.3 and 2 us a step:
+        // 22.9 / 28.7, 27.6 / 29.9, 25.6 / 28.0; 200 unaligned rows of
+        // 1003 x 1537 29.3 us at 2.5, 31.9 at 0.8.
         int64_t ks = (2 * ctx->multiprocessors) / ((int64_t)a.to * a.tm);
         const int64_t steps = a.kp / kGemmStep;
         if (ks > steps / 2) ks = steps / 2;
+        const double split_us = (double)a.M * (double)OT * 16.0 / 4.0e6;
+        const int64_t best = (int64_t)(sqrt((double)steps * (unal ? 2.5 : 0.8) / split_us) + 0.5);
+        if (ks > best) ks = best;
         while (ks > 1 && ks * a.M * OT * 8 > kSplitKPartBytes) ks--;
         if (ks < 1) ks = 1;
         a.kslice = (steps + ks - 1) / ks * kGemmStep;
