@@ -81,6 +81,21 @@ def test_few_outputs_are_the_closed_form(ctx, fmt, o, i):
     assert np.isnan(got[1]).all() and np.array_equal(got[0], want[0])
 
 
+@pytest.mark.parametrize("seq", [1, 4, 9])
+@pytest.mark.parametrize("fmt", [INT8, INT4])
+def test_product_over_its_own_input(ctx, fmt, seq):
+    # x is digitised before anything is written: the output may replace it
+    import undertow_amd as U
+    rng = np.random.default_rng(seq)
+    payload, scales = rand_qtensor(rng, fmt, 256, 256)
+    q = U.QTensor(ctx, fmt, payload, scales, 256, 256)
+    x = rng.standard_normal((seq, 256)).astype(np.float32)
+    buf = dev(x)
+    q.matmul(buf, buf, seq)
+    np.testing.assert_array_equal(host(buf), gemv_closed_form(fmt, payload, scales, 256, 256, x))
+
+
+
 def test_gemm_nonfinite_rows_are_nan(ctx):
     import undertow_amd as U
     rng = np.random.default_rng(5)

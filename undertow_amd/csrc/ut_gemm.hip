@@ -212,10 +212,10 @@ __device__ __forceinline__ void gemm_store(const GemmArgs &a, int wi,
     }
 }
 
-// Up to about 32 rows the weights' read bounds it (int8 7168 x 16384 from
-// memory: 16 rows 47 us, 2.5 TB/s; the four-row GEMV passes took 118 us),
-// beyond that the matrix cores (512 rows 290 us, 1.24 POP/s of digit
-// products against 3,611 us; 129280 x 7168 2,100 against 19,492 us).
+// Up to kGlMinRows rows, and any number of rows of unaligned weights.  The
+// weights' read bounds the few rows (int8 7168 x 16384 from memory: 16 rows
+// 47 us, 2.5 TB/s; the four-row GEMV passes took 118 us), the unaligned loads
+// the others (200 rows of 1003 x 1537: 29 us).
 constexpr int kGemmTO = 4;
 template <int FMT, int TM, bool UNAL>
 __global__ __launch_bounds__(kGemmThreads, 2) void k_gemm(GemmArgs a) {
@@ -332,7 +332,7 @@ int32_t launch_gemm(ut_ctx *ctx, const ut_qtensor *w, const DigitPlanes &x, int6
     a.kp = x.kp;
     a.accumulate = accumulate;
     const bool unal = ((uintptr_t)w->payload & 15) != 0 || w->row_bytes % 16 != 0;
-    const int64_t cap = unal ? 1 << 20 : 1 << 24;  // rows per launch: grids stay in 31 bits
+    const int64_t cap = 1 << 16;  // rows per launch: grids stay within 2^32 threads
     const int64_t O2 = w2 ? w2->out_dim : 0, OT = w->out_dim + O2;
     for (int64_t s0 = 0; s0 < M; s0 += cap) {
         a.M = M - s0 < cap ? M - s0 : cap;
@@ -363,7 +363,8 @@ int32_t launch_gemm(ut_ctx *ctx, const ut_qtensor *w, const DigitPlanes &x, int6
         const int64_t best = (int64_t)(sqrt((double)steps * (unal ? 2.5 : 0.8) / split_us) + 0.5);
         if (ks > best) ks = best;
         while (ks > 1 && ks * a.M * OT * 8 > kSplitKPartBytes) ks--;
-        if (ks < 1) ks = 1;
+        // (a first call under capture has no buffer for the partials)
+        if (ks < 1 || (!ctx->splitk && ks > 1 && stream_capturing(ctx))) ks = 1;
         a.kslice = (steps + ks - 1) / ks * kGemmStep;
         a.ks = (int)((a.kp + a.kslice - 1) / a.kslice);
         if (a.ks > 1) UT_TRY(splitk_buffer(ctx, &a.part));

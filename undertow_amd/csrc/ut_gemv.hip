@@ -972,8 +972,10 @@ static bool fast_ok(const ut_qtensor *w);
 // rows of int8 1024 x 4096 10.7 -> 9.5 (576 x 7168: 13.4 against 12.4 but
 // 1536 x 7168 14.7 against 16.7); four of 1024 x 256 9.7 -> 7.9 (2048 x 2048:
 // 10.8 against 12.6).
-static bool gemv_direct_ok(const ut_qtensor *w, const float *x, int64_t M) {
+// (Its workgroups read x while others write out: not where the two overlap.)
+static bool gemv_direct_ok(const ut_qtensor *w, const float *x, int64_t M, const float *out) {
     if (w->fmt != UT_FMT_INT8 && w->fmt != UT_FMT_INT4) return false;
+    if (out < x + M * w->in_dim && x < out + M * w->out_dim) return false;
     return M >= 1 && M <= 4 && M * w->in_dim <= (M <= 2 ? 64 : 32) * kDirectCols && fast_ok(w) &&
            ((uintptr_t)x & 15) == 0 && w->out_dim <= (w->fmt == UT_FMT_INT8 ? 2048 : 1024);
 }
@@ -1913,8 +1915,19 @@ extern "C" int32_t ut_qtensor_matmul(ut_ctx *ctx, const ut_qtensor *qt, float *o
     // Int8 { .. } if fast_int8_enabled() (qtensor.rs:385-398)
     if (qt->fmt == UT_FMT_INT8 && ctx->fast_int8)
         return matmul_fast_i8(ctx, qt, out_dev, qt->out_dim, 0, x_dev, seq);
-    if (gemv_direct_ok(qt, x_dev, seq))
+    if (gemv_direct_ok(qt, x_dev, seq, out_dev)) {
+        // the buffers that other row counts of this weight need are there
+        // after a first call of any, so that those can be captured
+        if ((ctx->scratch.bytes == 0 || !ctx->splitk) && !stream_capturing(ctx)) {
+            ScratchPlan plan;
+            plan.add(planes_bytes(seq, qt->in_dim));
+            std::vector<void *> ptrs;
+            int64_t *part = nullptr;
+            UT_TRY(scratch_acquire(ctx, plan, ptrs));
+            UT_TRY(splitk_buffer(ctx, &part));
+        }
         return launch_gemv_direct(ctx, qt, x_dev, seq, out_dev, qt->out_dim);
+    }
     if (gemm_ok(qt, seq)) {
         ScratchPlan plan;
         plan.add(planes_bytes(seq, qt->in_dim));

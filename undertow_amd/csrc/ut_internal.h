@@ -138,6 +138,8 @@ struct ScratchPlan {
     }
 };
 int32_t scratch_acquire(ut_ctx *ctx, const ScratchPlan &plan, std::vector<void *> &ptrs);
+// Whether the context's stream is being captured (nothing may be allocated).
+bool stream_capturing(ut_ctx *ctx);
 int32_t pinned_acquire(ut_ctx *ctx, size_t bytes, void **ptr);
 
 // Kernel timing hooks: call timing_begin before a launch and timing_end

@@ -709,8 +709,12 @@ static bool mla_prompt(int64_t R, int64_t T) { return R > kMlaPromptRows && T > 
 static size_t mla_mfma_scratch_bytes(int64_t R, int64_t H, int64_t L, int64_t T) {
     const size_t ns = (size_t)(mla_prompt(R, T) ? mla_prompt_nslice(R, H, T) : mla_mfma_nslice(T)),
                  RH = (size_t)(R * H);
-    if (mla_prompt(R, T) && ns == 1) return 0;
-    return ((ns * RH * 4 + 255) & ~size_t(255)) * 2 + ((ns * L * RH * 4 + 255) & ~size_t(255));
+    const size_t b = ((ns * RH * 4 + 255) & ~size_t(255)) * 2 + ((ns * L * RH * 4 + 255) & ~size_t(255));
+    if (!mla_prompt(R, T)) return b;
+    // at least a few rows' over the same context: scratch that a prompt left
+    // serves the calls after it
+    const size_t few = mla_mfma_scratch_bytes(kMlaPromptRows, H, L, T);
+    return ns > 1 && b > few ? b : few;
 }
 
 static size_t mla_split_scratch_bytes(int64_t R, int64_t H, int64_t L, int64_t T) {

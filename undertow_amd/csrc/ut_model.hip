@@ -398,12 +398,16 @@ int32_t ws_reserve(ut_session *s, int64_t rows) {
     // up, h [4][max inter], the choices' outputs [4][k][H] and a shared
     // MLP's [4][H]
     size_t ifast = F(3 * 4 * max_inter(m) + 4 * (k > 0 ? k : 1) * H + 4 * H);
-    size_t img = 0, imu = 0, imr = 0;
+    // a prompt's products (last, left out when the device has no room for
+    // them: the four-row passes need none)
+    size_t img = 0, imu = 0, imr = 0, products = 0;
     if (R > 4) {
+        const size_t before = plan.sizes.size();
         img = F(R * max_inter(m));
         imu = F(R * max_inter(m));
         const int64_t kk = k > 0 ? k : 1, ch = moe_rows_chunk(kk);
-        imr = plan.add(moe_rows_bytes(R < ch ? R : ch, kk, E > 0 ? E : 1, H, c.moe_intermediate_size, true));
+        imr = plan.add(m->store ? 0 : moe_rows_bytes(R < ch ? R : ch, kk, E > 0 ? E : 1, H, c.moe_intermediate_size, true));
+        for (size_t i = before; i < plan.sizes.size(); i++) products += plan.sizes[i];
     }
     size_t total = 0;
     for (size_t b : plan.sizes) total += b;
@@ -426,7 +430,14 @@ int32_t ws_reserve(ut_session *s, int64_t rows) {
         (void)hipGraphExecDestroy(s->g1);
         s->g1 = nullptr;
     }
-    if (hipMalloc(&w.base, total) != hipSuccess) {
+    hipError_t got = hipMalloc(&w.base, total);
+    if (got != hipSuccess && products > 0) {
+        (void)hipGetLastError();
+        total -= products;
+        products = 0;
+        got = hipMalloc(&w.base, total);
+    }
+    if (got != hipSuccess) {
         (void)hipGetLastError();
         set_error(ctx, "workspace allocation of %zu bytes failed", total);
         w.rows = 0;
@@ -448,11 +459,9 @@ int32_t ws_reserve(ut_session *s, int64_t rows) {
     w.digits = p[idig]; w.moe = p[imoes]; w.mla = p[imla]; w.argm = p[iarg];
     w.digA = p[idA]; w.digB = p[idB];
     w.fast = (float *)p[ifast];
-    if (R > 4) {
-        w.mlp_g = (float *)p[img];
-        w.mlp_u = (float *)p[imu];
-        w.moe_rows = p[imr];
-    }
+    w.mlp_g = products ? (float *)p[img] : nullptr;
+    w.mlp_u = products ? (float *)p[imu] : nullptr;
+    w.moe_rows = products ? p[imr] : nullptr;
     w.rows = R;
     UT_CHECK_HIP(ctx, hipMemsetAsync(w.err, 0, 4, ctx->stream));
     return UT_OK;
@@ -589,7 +598,7 @@ int32_t norm_dig(ut_session *s, const float *x, int64_t ldx, const float *w, int
 
 // Whether an MLP's rows run as three products over all rows (mlp_rows).
 bool mlp_gemm_ok(const ut_session *s, const MlpW &w, int64_t rows) {
-    return !fast8(s) && gemm_ok(w.gate, rows) && gemm_ok(w.up, rows) && gemm_ok(w.down, rows);
+    return !fast8(s) && s->ws.mlp_g && gemm_ok(w.gate, rows) && gemm_ok(w.up, rows) && gemm_ok(w.down, rows);
 }
 
 // An MLP over rows of normed x (digits xd made for it where they need no
@@ -806,7 +815,7 @@ int32_t moe_forward(ut_session *s, const LayerW &L, const float *x, const XDigit
 // Whether a MoE layer's rows run as grouped products (moe_forward_rows).
 bool moe_gemm_ok(const ut_session *s, const LayerW &L, int64_t rows) {
     const ut_model_config &c = s->m->c;
-    return !fast8(s) && !s->m->store &&
+    return !fast8(s) && !s->m->store && s->ws.moe_rows &&
            moe_rows_ok(L.expert_fmt, rows, c.n_routed_experts, c.hidden_size,
                        c.moe_intermediate_size) &&
            (!L.has_shared || mlp_gemm_ok(s, L.shared, rows));

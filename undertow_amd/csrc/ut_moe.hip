@@ -2362,14 +2362,7 @@ int32_t moe_experts_grouped(ut_ctx *ctx, const ut_expert_table *tbl, const int32
     if (!moe_rows_ok(tbl->fmt, rows, tbl->n, H, tbl->inter)) return UT_OK;
     ScratchPlan plan;
     plan.add(moe_rows_bytes(rows < chunk ? rows : chunk, top_k, tbl->n, H, tbl->inter, true));
-    if (plan.sizes[0] > ctx->scratch.bytes) {
-        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(ctx->stream, &st) != hipSuccess) {
-            (void)hipGetLastError();
-            return UT_OK;
-        }
-        if (st != hipStreamCaptureStatusNone) return UT_OK;
-    }
+    if (plan.sizes[0] > ctx->scratch.bytes && stream_capturing(ctx)) return UT_OK;
     std::vector<void *> ptrs;
     const int32_t rc = scratch_acquire(ctx, plan, ptrs);
     if (rc == UT_ERR_OOM) return UT_OK;

@@ -52,6 +52,16 @@ int32_t scratch_acquire(ut_ctx *ctx, const ScratchPlan &plan, std::vector<void *
     return UT_OK;
 }
 
+bool stream_capturing(ut_ctx *ctx) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &st) != hipSuccess) {
+        // (the null stream while another stream is captured)
+        (void)hipGetLastError();
+        return true;
+    }
+    return st != hipStreamCaptureStatusNone;
+}
+
 int32_t pinned_acquire(ut_ctx *ctx, size_t bytes, void **ptr) {
     if (bytes > ctx->pinned_bytes) {
         UT_CHECK_HIP(ctx, hipStreamSynchronize(ctx->stream));
