@@ -60,3 +60,15 @@ def test_rows_merge_equals_single_rows(ctx, R, H, T):
     one = torch.cat([U.mla_attend_split(ctx, qabs[r:r + 1].contiguous(), qr[r:r + 1].contiguous(),
                                         kc, T - R + r, scale) for r in range(R)])
     assert torch.equal(got, one)
+
+
+@pytest.mark.parametrize("R,T", [(20, 100), (40, 700), (257, 257)])
+def test_output_aligned_to_one_float(ctx, R, T):
+    import undertow_amd as U
+    g = torch.Generator(device="cuda").manual_seed(R)
+    rnd = lambda *s: torch.randn(s, device="cuda", generator=g)
+    qabs, qr, lat, kr = rnd(R, 128, 512), rnd(R, 128, 64), rnd(T, 512), rnd(T, 64)
+    kc, scale = U.mla_cache_split(ctx, lat, kr), float(1 / np.sqrt(192.0))
+    out = torch.empty(R * 128 * 512 + 1, device="cuda")[1:].view(R, 128, 512)
+    U.mla_attend_split(ctx, qabs, qr, kc, T - R, scale, out=out)
+    assert torch.equal(out, U.mla_attend_split(ctx, qabs, qr, kc, T - R, scale))

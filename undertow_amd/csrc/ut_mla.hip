@@ -267,6 +267,9 @@ __device__ __forceinline__ float pair_sum(float v) {
 constexpr int kTile16 = 16;
 constexpr int kTile16Bytes = kTile16 * kRowChunks * 16;  // 36864
 
+// Four outputs in one store: the caller's output is aligned to one float.
+typedef float mla_f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
 // PROMPT: the rows of a prompt (mla_prompt_slice's slice length), longest
 // contexts first so that the launch ends on short ones; with one slice per
 // row the workgroup writes the finished context (no partials, no combine).
@@ -426,9 +429,9 @@ __global__ __launch_bounds__(256, 2) void k_mla_mfma16(MlaMfmaArgs a) {
         for (int mt = 0; mt < MT; mt++)
 #pragma unroll
             for (int i = 0; i < 4; i++)
-                *(float4 *)(po + 32 * mt + 8 * i) =
-                    make_float4(__fmul_rn(o[mt][4 * i], inv), __fmul_rn(o[mt][4 * i + 1], inv),
-                                __fmul_rn(o[mt][4 * i + 2], inv), __fmul_rn(o[mt][4 * i + 3], inv));
+                *(mla_f32x4u *)(po + 32 * mt + 8 * i) =
+                    mla_f32x4u{__fmul_rn(o[mt][4 * i], inv), __fmul_rn(o[mt][4 * i + 1], inv),
+                               __fmul_rn(o[mt][4 * i + 2], inv), __fmul_rn(o[mt][4 * i + 3], inv)};
         return;
     }
     const int64_t RH = a.RH;
@@ -662,8 +665,8 @@ __global__ __launch_bounds__(256) void k_mla_combine_rows(const float *__restric
     float *out = clat + (int64_t)(blockIdx.x * 32 + c) * L + d0 + 4 * q;
 #pragma unroll
     for (int i = 0; i < kCombineRowsDims; i += 32)
-        *(float4 *)(out + i) = make_float4(so[c][4 * q + i], so[c][4 * q + i + 1],
-                                           so[c][4 * q + i + 2], so[c][4 * q + i + 3]);
+        *(mla_f32x4u *)(out + i) = mla_f32x4u{so[c][4 * q + i], so[c][4 * q + i + 1],
+                                              so[c][4 * q + i + 2], so[c][4 * q + i + 3]};
 }
 
 // Largest slice count over the rows' context lengths n <= T (an upper
