@@ -95,7 +95,6 @@ def test_product_over_its_own_input(ctx, fmt, seq):
     np.testing.assert_array_equal(host(buf), gemv_closed_form(fmt, payload, scales, 256, 256, x))
 
 
-
 def test_gemm_nonfinite_rows_are_nan(ctx):
     import undertow_amd as U
     rng = np.random.default_rng(5)
@@ -131,3 +130,23 @@ def test_f32_rows_equal_one_row_calls(ctx, o, i):
     ref = x.astype(np.float64) @ w.astype(np.float64).T
     err = np.linalg.norm(run(ctx, q, x) - ref) / np.linalg.norm(ref)
     assert err <= 2.0 ** -23 * max(1.0, np.log2(i))  # tree-wise f32 sums
+
+
+# unsplit slices either side of the line between the two LDS tiles (16 stages
+# of 128 columns; one odd, one even count past it), rows past both tile edges
+@pytest.mark.parametrize("i", [2048, 2176, 2304])
+@pytest.mark.parametrize("fmt", [INT8, INT4])
+def test_long_slices_equal_few_rows(ctx, fmt, i):
+    import torch
+    import undertow_amd as U
+    rng = np.random.default_rng(i)
+    o, seq = 128 * 130 + 16, 65  # 262 tiles: no K split
+    payload, scales = rand_qtensor(rng, fmt, o, i)
+    q = U.QTensor(ctx, fmt, payload, scales, o, i)
+    x = dev(rng.standard_normal((seq, i)).astype(np.float32))
+    got, few = (torch.empty((seq, o), device="cuda") for _ in range(2))
+    q.matmul(got, x, seq)
+    for r in range(0, seq, 4):
+        n = min(4, seq - r)
+        q.matmul(few[r:r + n], x[r:r + n], n)
+    assert torch.equal(got, few)

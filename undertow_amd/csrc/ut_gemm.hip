@@ -252,22 +252,38 @@ __global__ __launch_bounds__(kGemmThreads, 2) void k_gemm(GemmArgs a) {
 }
 
 // More than kGlMinRows rows of 16-byte aligned weights: 128 weight rows x 64
-// activation rows per workgroup of eight waves, two workgroups (four waves a
-// SIMD) per CU.  Bound by the matrix cores, at nine tenths of what a large
-// int8 library product reaches on this card (2.1 POP/s): 512 rows of int8
-// 7168 x 16384 285 us with the direct tile, 197 us so (1.84 POP/s);
-// 129280 x 7168 1,982 -> 1,545; int4 18432 x 7168 260 -> 226.  Four waves of
-// 4 x 2 tiles: 190 / 1,546 / 245 us; 256 x 64 tiles, one workgroup per CU:
-// 217 / 1,724 / 265; stages of 64 columns, three workgroups: 257 / 1,796 /
-// 269.  At 32 rows and fewer the launch is bound by the weights' read, which
-// the direct tile keeps more of in flight (129280 x 7168 at 16 rows 183
-// against 234 us); at 64 this one leads (7168 x 16384 67 -> 61 us, 18432 x
-// 7168 72 -> 63).
+// activation rows per workgroup, two workgroups per CU.  Bound by the matrix
+// cores (from registers alone the instruction reaches 3.55 POP/s on random
+// data; a large int8 library product 2.1): 512 rows of int8 7168 x 16384
+// 285 us with the direct tile, 197 us with eight waves of 2 x 2 tiles;
+// 129280 x 7168 1,982 -> 1,545; int4 18432 x 7168 260 -> 226 (without the
+// digitising).  256 x 64 tiles, one workgroup per CU: 217 / 1,724 / 265;
+// stages of 64 columns, three workgroups: 257 / 1,796 / 269.  At 32 rows and
+// fewer the launch is bound by the weights' read, which the direct tile keeps
+// more of in flight (129280 x 7168 at 16 rows 183 against 234 us); at 64 this
+// one leads (7168 x 16384 67 -> 61 us, 18432 x 7168 72 -> 63).
 constexpr int64_t kGlMinRows = 32;
-constexpr int kGlTO = 2, kGlTM = 2, kGlWO = 4, kGlWM = 2, kGlS = 128;
-template <int FMT>
-__global__ __launch_bounds__(64 * kGlWO * kGlWM, 2) void k_gemm_lds(GemmArgs a) {
-    using L = GemmLds<FMT, kGlTO, kGlTM, kGlWO, kGlWM, kGlS>;
+//
+// LONG (slices of more than kGlLong stages): four waves of 4 x 2 tiles, which
+// read 10 fragments for 24 matrix instructions instead of 8 for 12, each
+// half stage's beside the matrix instructions of the half before (PIPE).  A
+// wave's reads used to stand before its products: the matrix cores were 40%
+// busy, with a third of the wave cycles waiting.  512 rows of 129280 x 7168
+// 1,472 -> 1,375 us (2.07 POP/s), 18432 x 7168 251 -> 227, int4 234 -> 212,
+// 7168 x 16384 214 -> 204 and at 64 rows 65.1 -> 63.1, with the digitising.
+// The short slices' eight waves fill the pipeline sooner: 509 rows of
+// 24576 x 1536 92.3 us, 94.7 with LONG; 200 of int4 7168 x 2048 27.9 / 29.4.
+// Four buffers of 64-column stages, three in flight: 250 us
+// at 7168 x 16384, 1,686 at 129280 x 7168 (half lines of 128 bytes).
+constexpr int kGlTM = 2, kGlWM = 2, kGlS = 128;
+constexpr int kGlRows = 128;  // weight rows per workgroup
+constexpr int64_t kGlLong = 16;
+template <bool LONG> constexpr int gl_to() { return LONG ? 4 : 2; }
+template <bool LONG> constexpr int gl_threads() { return 64 * kGlRows / (16 * gl_to<LONG>()) * kGlWM; }
+template <int FMT, bool LONG>
+__global__ __launch_bounds__(gl_threads<LONG>(), 2) void k_gemm_lds(GemmArgs a) {
+    constexpr int TO = gl_to<LONG>(), WO = kGlRows / (16 * TO);
+    using L = GemmLds<FMT, TO, kGlTM, WO, kGlWM, kGlS>;
     __shared__ L s0, s1;
     const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
     const int unit = (j / a.tm) * 8 + xcd, mt = j % a.tm;
@@ -276,16 +292,16 @@ __global__ __launch_bounds__(64 * kGlWO * kGlWM, 2) void k_gemm_lds(GemmArgs a) 
     const GemmWeight &W = a.w[wi];
     const int wave = threadIdx.x >> 6;
     const int64_t ob = (int64_t)ot * L::kARows, mb = (int64_t)mt * (16 * kGlTM * kGlWM);
-    GemmSrc<FMT, kGlTO, kGlTM, kGlWO, kGlWM, kGlS> src;
-    gemm_src<FMT, kGlTO, kGlTM, kGlWO, kGlWM, kGlS>(
+    GemmSrc<FMT, TO, kGlTM, WO, kGlWM, kGlS> src;
+    gemm_src<FMT, TO, kGlTM, WO, kGlWM, kGlS>(
         src,
         [&](int row) { return W.w + (ob + row < W.O ? ob + row : W.O - 1) * a.row_bytes; },
         [&](int m, int p) { return a.pl + ((mb + m < a.M ? mb + m : a.M - 1) * 3 + p) * a.kp; });
     const int64_t kb = z * a.kslice, ke = kb + a.kslice < a.kp ? kb + a.kslice : a.kp;
-    ut_i32x4 acc[kGlTO][kGlTM][3];
-    gemm_tile_lds<FMT, kGlTO, kGlTM, kGlWO, kGlWM, kGlS>(src, a.row_bytes, kb, ke, s0, s1, acc);
-    gemm_store<FMT, kGlTO, kGlTM>(a, wi, acc, ob + (wave % kGlWO) * (16 * kGlTO),
-                                  mb + (wave / kGlWO) * (16 * kGlTM), z);
+    ut_i32x4 acc[TO][kGlTM][3];
+    gemm_tile_lds<LONG, FMT, TO, kGlTM, WO, kGlWM, kGlS>(src, a.row_bytes, kb, ke, s0, s1, acc);
+    gemm_store<FMT, TO, kGlTM>(a, wi, acc, ob + (wave % WO) * (16 * TO),
+                               mb + (wave / WO) * (16 * kGlTM), z);
 }
 
 // The K splits' totals summed and scaled (exact integers: any order).
@@ -342,7 +358,7 @@ int32_t launch_gemm(ut_ctx *ctx, const ut_qtensor *w, const DigitPlanes &x, int6
         if (w2) a.w[1] = weight(w2, out2 + s0 * ldo2, ldo2);
         const bool big = !unal && a.M > kGlMinRows;
         const int tmr = big ? kGlTM * kGlWM : a.M <= 16 ? 1 : 2;
-        const int tor = big ? 16 * kGlTO * kGlWO : 64 * kGemmTO;
+        const int tor = big ? kGlRows : 64 * kGemmTO;
         a.to0 = (int)((w->out_dim + tor - 1) / tor);
         a.to = a.to0 + (int)((O2 + tor - 1) / tor);
         a.tm = (int)((a.M + 16 * tmr - 1) / (16 * tmr));
@@ -378,9 +394,16 @@ int32_t launch_gemm(ut_ctx *ctx, const ut_qtensor *w, const DigitPlanes &x, int6
         else UT_GM(F, 2, U);            \
     } while (0)
         if (big) {
-            const dim3 bd(64 * kGlWO * kGlWM);
-            if (w->fmt == UT_FMT_INT8) hipLaunchKernelGGL(k_gemm_lds<UT_FMT_INT8>, grid, bd, 0, ctx->stream, a);
-            else hipLaunchKernelGGL(k_gemm_lds<UT_FMT_INT4>, grid, bd, 0, ctx->stream, a);
+            const bool lng = a.kslice > kGlLong * kGlS;
+#define UT_GL(F, LG) hipLaunchKernelGGL((k_gemm_lds<F, LG>), grid, dim3(gl_threads<LG>()), 0, ctx->stream, a)
+            if (w->fmt == UT_FMT_INT8) {
+                if (lng) UT_GL(UT_FMT_INT8, true);
+                else UT_GL(UT_FMT_INT8, false);
+            } else {
+                if (lng) UT_GL(UT_FMT_INT4, true);
+                else UT_GL(UT_FMT_INT4, false);
+            }
+#undef UT_GL
         } else if (w->fmt == UT_FMT_INT8) {
             if (unal) UT_GMT(UT_FMT_INT8, true);
             else UT_GMT(UT_FMT_INT8, false);

@@ -245,7 +245,10 @@ __device__ __forceinline__ void gemm_wait_copies() {
     asm volatile("" ::: "memory");
 }
 
-template <int FMT, int TO, int TM, int WO, int WM, int S>
+// PIPE: a stage's second half is multiplied after the next stage's first half
+// has been read, so a wave's LDS reads run beside its matrix instructions
+// instead of before them (twice the fragments in registers).
+template <bool PIPE, int FMT, int TO, int TM, int WO, int WM, int S>
 __device__ __forceinline__ void gemm_tile_lds(const GemmSrc<FMT, TO, TM, WO, WM, S> &src,
                                               int64_t len, int64_t kb, int64_t ke,
                                               GemmLds<FMT, TO, TM, WO, WM, S> &s0,
@@ -313,11 +316,63 @@ __device__ __forceinline__ void gemm_tile_lds(const GemmSrc<FMT, TO, TM, WO, WM,
                         acc[t][m][p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(f[t], w[m][p], acc[t][m][p], 0, 0, 0);
         }
     };
+    struct Frag {
+        ut_i32x4 a[TO], b[TM][3];  // a: int4 codes still packed
+    };
+    auto read = [&](const L &s, int h, Frag &x) {
+        const int c = 4 * h + q;  // this lane's 16 columns of the stage
+#pragma unroll
+        for (int t = 0; t < TO; t++) {
+            const int row = (wo * TO + t) * 16 + r;
+            if constexpr (FMT == UT_FMT_INT8) {
+                const uint4 v = s.a[row * L::kAC + (c ^ gemm_swz<L::kAC>(row))];
+                x.a[t] = ut_i32x4{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
+            } else {
+                const uint2 v = ((const uint2 *)&s.a[row * L::kAC + ((c >> 1) ^ gemm_swz<L::kAC>(row))])[c & 1];
+                x.a[t][0] = (int)v.x;
+                x.a[t][1] = (int)v.y;
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < TM; m++)
+#pragma unroll
+            for (int p = 0; p < 3; p++) {
+                const int row = ((wm * TM + m) * 3 + p) * 16 + r;
+                const uint4 v = s.b[row * L::kBC + (c ^ gemm_swz<L::kBC>(row))];
+                x.b[m][p] = ut_i32x4{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
+            }
+    };
+    auto multiply = [&](const Frag &x) {
+        ut_i32x4 f[TO];
+#pragma unroll
+        for (int t = 0; t < TO; t++) {
+            if constexpr (FMT == UT_FMT_INT8) f[t] = x.a[t];
+            else f[t] = gemm_i4_codes((uint32_t)x.a[t][0], (uint32_t)x.a[t][1]);
+        }
+#pragma unroll
+        for (int m = 0; m < TM; m++)
+#pragma unroll
+            for (int p = 0; p < 3; p++)
+#pragma unroll
+                for (int t = 0; t < TO; t++)
+                    acc[t][m][p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(f[t], x.b[m][p], acc[t][m][p], 0, 0, 0);
+    };
+    Frag f0, f1;
     // step i: its stage has landed, the other buffer is read and gets the next
     auto step = [&](L &s, L &other, int i) {
         gemm_wait_copies();
         copy(other, i + 1);
-        compute(s);
+        if constexpr (PIPE) {
+            static_assert(S == 128, "two halves");
+            read(s, 0, f0);
+            __builtin_amdgcn_sched_barrier(0);
+            if (i) multiply(f1);
+            read(s, 1, f1);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(f0);
+        } else {
+            compute(s);
+        }
     };
     copy(s0, 0);
     int i = 0;
@@ -326,6 +381,7 @@ __device__ __forceinline__ void gemm_tile_lds(const GemmSrc<FMT, TO, TM, WO, WM,
         step(s1, s0, i + 1);
     }
     if (i < n) step(s0, s1, i);
+    if constexpr (PIPE) multiply(f1);
     gemm_wait_copies();  // no copy outlives the tile
 }
 

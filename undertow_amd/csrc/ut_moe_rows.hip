@@ -156,7 +156,7 @@ __device__ __forceinline__ void rows_tile(const MoeRowsArgs &a, int n, int64_t l
     gemm_src<FMT, kMrTO, TM, 4, 1, kMrS>(src, wrow, [&](int m, int p) {
         return a.pl + (arow(m < n ? m : n - 1) * 3 + p) * a.kp;
     });
-    gemm_tile_lds<FMT, kMrTO, TM, 4, 1, kMrS>(src, len, 0, a.kp, *(L *)s0, *(L *)s1, acc);
+    gemm_tile_lds<false, FMT, kMrTO, TM, 4, 1, kMrS>(src, len, 0, a.kp, *(L *)s0, *(L *)s1, acc);
 }
 
 // Gate and up of kMrRows / 2 h rows against a tile's rows: a wave's weight
