@@ -266,15 +266,17 @@ constexpr int64_t kGlMinRows = 32;
 //
 // LONG (slices of more than kGlLong stages): four waves of 4 x 2 tiles, which
 // read 10 fragments for 24 matrix instructions instead of 8 for 12, each
-// half stage's beside the matrix instructions of the half before (PIPE).  A
-// wave's reads used to stand before its products: the matrix cores were 40%
-// busy, with a third of the wave cycles waiting.  512 rows of 129280 x 7168
+// half stage's beside the matrix instructions of the half before (PIPE): a
+// wave's reads otherwise stand before its products.  (Counters of the trial
+// of four buffers below, which reads so too: matrix cores 40% busy, 39% of
+// the wave cycles waiting.)  512 rows of 129280 x 7168
 // 1,472 -> 1,375 us (2.07 POP/s), 18432 x 7168 251 -> 227, int4 234 -> 212,
 // 7168 x 16384 214 -> 204 and at 64 rows 65.1 -> 63.1, with the digitising.
 // The short slices' eight waves fill the pipeline sooner: 509 rows of
 // 24576 x 1536 92.3 us, 94.7 with LONG; 200 of int4 7168 x 2048 27.9 / 29.4.
-// Four buffers of 64-column stages, three in flight: 250 us
-// at 7168 x 16384, 1,686 at 129280 x 7168 (half lines of 128 bytes).
+// Four buffers of 64-column stages, three in flight, copy half lines of 128
+// bytes: 243 us at 7168 x 16384 and 1,637 at 129280 x 7168, with PIPE reads
+// 250 and 1,686.
 constexpr int kGlTM = 2, kGlWM = 2, kGlS = 128;
 constexpr int kGlRows = 128;  // weight rows per workgroup
 constexpr int64_t kGlLong = 16;
