@@ -61,7 +61,11 @@ typedef struct ut_session ut_session;
 
 /* --------------------------------------------------------------- context */
 /* No reference counterpart (the reference has no device): owns one HIP
- * stream on `device` and a scratch arena reused across calls. */
+ * stream on `device` and a scratch arena reused across calls.  The arena
+ * grows to the largest call (after a wait for the stream); growing it under
+ * a stream capture fails, so a call to be captured is run once before, at
+ * its size or a larger one.  Memory that a captured call uses stays where it
+ * is until the context is destroyed, whatever calls follow the capture. */
 int32_t     ut_ctx_create(int32_t device, ut_ctx **out);
 void        ut_ctx_destroy(ut_ctx *ctx);
 const char *ut_last_error(const ut_ctx *ctx);

@@ -1,0 +1,69 @@
+"""Calls captured into graphs beside eager calls of other sizes on the same
+context: what a capture needs is there after an eager call of its size or a
+larger one, and what it recorded stays valid when later calls need more."""
+import numpy as np
+import pytest
+import torch
+
+from conftest import dev
+from qgen import INT4, rand_qtensor
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def side():
+    """A stream of its own with a fresh context bound to it."""
+    import undertow_amd as U
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        c = U.Context(0)
+        yield s, c
+        s.synchronize()
+
+
+def expert_table(c, rng, fmt, E, H, I):
+    import undertow_amd as U
+    tbl = U.ExpertTable(c, E, H, I)
+    for e in range(E):
+        tbl.set(e, *[U.QTensor(c, fmt, *rand_qtensor(rng, fmt, o, i), o, i)
+                     for o, i in ((I, H), (I, H), (H, I))])
+    return tbl
+
+
+def expert_rows(rng, E, H, k, rows):
+    ids = dev(np.stack([rng.permutation(E)[:k] for _ in range(rows)]).astype(np.int32))
+    return ids, dev(rng.random((rows, k)).astype(np.float32)), dev(rng.standard_normal((rows, H)).astype(np.float32))
+
+
+def capture(s, f):
+    s.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        out = f()
+    return g, out
+
+
+def test_captured_experts_outlive_a_longer_prompt(side):
+    """A decode call's graph keeps its arena block when a prompt grows the
+    arena past it (600 rows: 2.6 MB and more of scratch, the four rows'
+    block is under 1.7 MB)."""
+    s, c = side
+    rng = np.random.default_rng(8)
+    E, H, I, k = 6, 256, 128, 2
+    assert 600 * k * (H + I) * 4 > 1.7e6
+    tbl = expert_table(c, rng, INT4, E, H, I)
+    ids, w, x = expert_rows(rng, E, H, k, 600)
+    few = [t[:4].contiguous() for t in (ids, w, x)]
+    want = tbl.moe_experts(*few)
+    g, got = capture(s, lambda: tbl.moe_experts(*few))
+    every = tbl.moe_experts(ids, w, x)
+    spill = torch.zeros(64 << 20, dtype=torch.uint8, device="cuda")  # what a freed block would hold
+    for _ in range(3):
+        got.zero_()
+        spill.fill_(255)
+        g.replay()
+        s.synchronize()
+        assert torch.equal(got, want)
+        assert torch.equal(tbl.moe_experts(ids, w, x), every)
+    assert torch.equal(every[:4], want)

@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "../../include/undertow_hip.h"
+#include "ut_arena.h"
 
 namespace ut {
 
@@ -44,11 +45,6 @@ struct PendingTiming {
     hipEvent_t start, stop;
 };
 
-struct DeviceBuffer {
-    void *ptr = nullptr;
-    size_t bytes = 0;
-};
-
 }  // namespace ut
 
 struct ut_ctx {
@@ -58,7 +54,7 @@ struct ut_ctx {
     std::string err;
     // Scratch arena: one device allocation, carved per call.  All work runs
     // on one stream, so a later call may reuse what an earlier one used.
-    ut::DeviceBuffer scratch;
+    ut::Arena scratch;
     // Pinned host staging for small device->host results.
     void *pinned = nullptr;
     size_t pinned_bytes = 0;
@@ -129,7 +125,8 @@ struct ut_qtensor {
 namespace ut {
 
 // Scratch carving: returns device pointers into ctx->scratch, growing it
-// (after a stream sync) when needed.  Each carve is 256-byte aligned.
+// (after a stream sync) when needed; a block that a captured call uses stays
+// alive.  Each carve is 256-byte aligned.
 struct ScratchPlan {
     std::vector<size_t> sizes;
     size_t add(size_t bytes) {

@@ -27,21 +27,32 @@ int64_t payload_bytes(int32_t fmt, int64_t out_dim, int64_t in_dim) {
     }
 }
 
+struct DeviceMem {
+    ut_ctx *ctx;
+    void *alloc(size_t bytes) {
+        void *p = nullptr;
+        if (hipMalloc(&p, bytes) == hipSuccess) return p;
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    bool wait() { return ok(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize"); }
+    bool free(void *p) { return ok(hipFree(p), "hipFree"); }
+    bool ok(hipError_t e, const char *what) {
+        if (e != hipSuccess) set_error(ctx, "scratch: %s failed: %s", what, hipGetErrorString(e));
+        return e == hipSuccess;
+    }
+};
+
 int32_t scratch_acquire(ut_ctx *ctx, const ScratchPlan &plan, std::vector<void *> &ptrs) {
     size_t total = 0;
     for (size_t s : plan.sizes) total += s;
-    if (total > ctx->scratch.bytes) {
-        UT_CHECK_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        if (ctx->scratch.ptr) UT_CHECK_HIP(ctx, hipFree(ctx->scratch.ptr));
-        ctx->scratch.ptr = nullptr;
-        ctx->scratch.bytes = 0;
-        size_t want = total + total / 4 + (1 << 20);
-        if (hipMalloc(&ctx->scratch.ptr, want) != hipSuccess) {
-            (void)hipGetLastError();
-            set_error(ctx, "scratch allocation of %zu bytes failed", want);
-            return UT_ERR_OOM;
-        }
-        ctx->scratch.bytes = want;
+    const bool capturing = !ctx->scratch.captured && stream_capturing(ctx);
+    switch (arena_reserve(ctx->scratch, total, capturing, DeviceMem{ctx})) {
+    case ARENA_OK: break;
+    case ARENA_OOM:
+        set_error(ctx, "scratch allocation for %zu bytes failed", total);
+        return UT_ERR_OOM;
+    default: return UT_ERR_HIP;
     }
     ptrs.clear();
     char *p = (char *)ctx->scratch.ptr;
@@ -329,7 +340,7 @@ void ut::ctx_release(ut_ctx *ctx) {
         (void)hipEventDestroy(p.start);
         (void)hipEventDestroy(p.stop);
     }
-    if (ctx->scratch.ptr) (void)hipFree(ctx->scratch.ptr);
+    arena_release(ctx->scratch, DeviceMem{ctx});
     if (ctx->dev_err) (void)hipFree(ctx->dev_err);
     if (ctx->splitk) (void)hipFree(ctx->splitk);
     if (ctx->pinned) (void)hipHostFree(ctx->pinned);
