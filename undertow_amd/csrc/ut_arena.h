@@ -23,20 +23,29 @@ struct Arena {
 
 enum ArenaStatus { ARENA_OK, ARENA_OOM, ARENA_ERROR };
 
-// At least `total` bytes in a.ptr.
+// At least `total` bytes in a.ptr.  optional: for a caller that has another
+// way without so much; the old block then stays until the new one is there,
+// so that a call that gets none costs no wait and leaves the arena as it was.
 template <typename Mem>
-ArenaStatus arena_reserve(Arena &a, size_t total, bool capturing, Mem &&mem) {
+ArenaStatus arena_reserve(Arena &a, size_t total, bool capturing, bool optional, Mem &&mem) {
     if (total > a.bytes) {
-        if (!mem.wait()) return ARENA_ERROR;
+        const size_t want = total + total / 4 + (1 << 20);
+        void *early = optional ? mem.alloc(want) : nullptr;
+        if (optional && !early) return ARENA_OOM;
+        if (!mem.wait()) {
+            if (early) (void)mem.free(early);
+            return ARENA_ERROR;
+        }
         if (a.ptr) {
             if (a.captured) a.kept.push_back(a.ptr);
-            else if (!mem.free(a.ptr)) return ARENA_ERROR;
+            else if (!mem.free(a.ptr)) {
+                if (early) (void)mem.free(early);
+                return ARENA_ERROR;
+            }
         }
-        a.ptr = nullptr;
         a.bytes = 0;
         a.captured = false;
-        const size_t want = total + total / 4 + (1 << 20);
-        a.ptr = mem.alloc(want);
+        a.ptr = early ? early : mem.alloc(want);
         if (!a.ptr) return ARENA_OOM;
         a.bytes = want;
     }

@@ -134,7 +134,9 @@ struct ScratchPlan {
         return sizes.size() - 1;
     }
 };
-int32_t scratch_acquire(ut_ctx *ctx, const ScratchPlan &plan, std::vector<void *> &ptrs);
+// optional: UT_ERR_OOM leaves the arena as it was (the caller goes another way).
+int32_t scratch_acquire(ut_ctx *ctx, const ScratchPlan &plan, std::vector<void *> &ptrs,
+                        bool optional = false);
 // Whether the context's stream is being captured (nothing may be allocated).
 bool stream_capturing(ut_ctx *ctx);
 int32_t pinned_acquire(ut_ctx *ctx, size_t bytes, void **ptr);

@@ -2364,7 +2364,7 @@ int32_t moe_experts_grouped(ut_ctx *ctx, const ut_expert_table *tbl, const int32
     plan.add(moe_rows_bytes(rows < chunk ? rows : chunk, top_k, tbl->n, H, tbl->inter, true));
     if (plan.sizes[0] > ctx->scratch.bytes && stream_capturing(ctx)) return UT_OK;
     std::vector<void *> ptrs;
-    const int32_t rc = scratch_acquire(ctx, plan, ptrs);
+    const int32_t rc = scratch_acquire(ctx, plan, ptrs, true);
     if (rc == UT_ERR_OOM) return UT_OK;
     UT_TRY(rc);
     for (int64_t s0 = 0; rows - s0 >= kGemmMinRows; s0 = *done) {

@@ -43,11 +43,12 @@ struct DeviceMem {
     }
 };
 
-int32_t scratch_acquire(ut_ctx *ctx, const ScratchPlan &plan, std::vector<void *> &ptrs) {
+int32_t scratch_acquire(ut_ctx *ctx, const ScratchPlan &plan, std::vector<void *> &ptrs,
+                        bool optional) {
     size_t total = 0;
     for (size_t s : plan.sizes) total += s;
     const bool capturing = !ctx->scratch.captured && stream_capturing(ctx);
-    switch (arena_reserve(ctx->scratch, total, capturing, DeviceMem{ctx})) {
+    switch (arena_reserve(ctx->scratch, total, capturing, optional, DeviceMem{ctx})) {
     case ARENA_OK: break;
     case ARENA_OOM:
         set_error(ctx, "scratch allocation for %zu bytes failed", total);
