@@ -67,3 +67,23 @@ def test_captured_experts_outlive_a_longer_prompt(side):
         assert torch.equal(got, want)
         assert torch.equal(tbl.moe_experts(ids, w, x), every)
     assert torch.equal(every[:4], want)
+
+
+def test_few_experts_rows_captured_after_a_prompt(side):
+    """The scratch of a four-row pass is there after a call of six rows, whose
+    own grouped scratch is smaller (64 slots of four rows against 96 pairs:
+    4.2 MB, more than an arena of 1.17 MB * 1.25 + 1 MiB)."""
+    s, c = side
+    rng = np.random.default_rng(9)
+    E, H, I, k = 64, 2048, 512, 16
+    tbl = expert_table(c, rng, INT4, E, H, I)
+    ids, w, x = expert_rows(rng, E, H, k, 6)
+    want = tbl.moe_experts(ids, w, x)
+    few = [t[:4].contiguous() for t in (ids, w, x)]
+    g, got = capture(s, lambda: tbl.moe_experts(*few))
+    for _ in range(3):
+        got.zero_()
+        g.replay()
+        s.synchronize()
+        assert torch.equal(got, want[:4])
+        assert torch.equal(tbl.moe_experts(ids, w, x), want)

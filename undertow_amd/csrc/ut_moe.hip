@@ -2352,16 +2352,19 @@ namespace {
 // each); *done: the rows finished so.  Nothing is done where the path does
 // not take the shape, where its scratch cannot be had, or where it would
 // have to grow while the stream is captured: the four-row passes then run,
-// with the same results.
+// with the same results.  few: the scratch of a four-row pass, reserved with
+// the products' own: the last rows may need it, and a later call of few rows
+// can be captured after this one.
 int32_t moe_experts_grouped(ut_ctx *ctx, const ut_expert_table *tbl, const int32_t *ids_dev,
                             const float *weights_dev, int64_t rows, int32_t top_k,
                             const float *x_dev, const uint16_t *xh_dev, float *out_dev,
-                            int32_t *flag, int64_t *done) {
+                            int32_t *flag, size_t few, int64_t *done) {
     *done = 0;
     const int64_t H = tbl->hidden, chunk = moe_rows_chunk(top_k);
     if (!moe_rows_ok(tbl->fmt, rows, tbl->n, H, tbl->inter)) return UT_OK;
+    const size_t bytes = moe_rows_bytes(rows < chunk ? rows : chunk, top_k, tbl->n, H, tbl->inter, true);
     ScratchPlan plan;
-    plan.add(moe_rows_bytes(rows < chunk ? rows : chunk, top_k, tbl->n, H, tbl->inter, true));
+    plan.add(bytes > few ? bytes : few);
     if (plan.sizes[0] > ctx->scratch.bytes && stream_capturing(ctx)) return UT_OK;
     std::vector<void *> ptrs;
     const int32_t rc = scratch_acquire(ctx, plan, ptrs, true);
@@ -2425,14 +2428,15 @@ int32_t moe_experts_any(ut_ctx *ctx, const ut_expert_table *tbl, const int32_t *
                         const uint16_t *xh_dev, float *out_dev) {
     int32_t *flag = nullptr;
     UT_TRY(device_error_flag(ctx, &flag));
-    int64_t done = 0;
-    UT_TRY(moe_experts_grouped(ctx, tbl, ids_dev, weights_dev, rows, top_k, x_dev, xh_dev, out_dev,
-                               flag, &done));
-    if (done == rows) return UT_OK;
     const int64_t maxM = 4;
     const int64_t slots = moe_slots((int)maxM, top_k, tbl->n, -1);
+    const size_t few = moe_layout(maxM, top_k, slots, tbl->hidden, tbl->inter, tbl->fmt).total;
+    int64_t done = 0;
+    UT_TRY(moe_experts_grouped(ctx, tbl, ids_dev, weights_dev, rows, top_k, x_dev, xh_dev, out_dev,
+                               flag, few, &done));
+    if (done == rows) return UT_OK;
     ScratchPlan plan;
-    plan.add(moe_layout(maxM, top_k, slots, tbl->hidden, tbl->inter, tbl->fmt).total);
+    plan.add(few);
     std::vector<void *> ptrs;
     UT_TRY(scratch_acquire(ctx, plan, ptrs));
     return moe_experts_rows(ctx, tbl, ids_dev, weights_dev, rows, top_k, x_dev, out_dev, ptrs[0],
