@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from conftest import dev
-from qgen import INT4, rand_qtensor
+from qgen import INT4, INT8, rand_qtensor
 
 pytestmark = pytest.mark.gpu
 
@@ -87,3 +87,22 @@ def test_few_experts_rows_captured_after_a_prompt(side):
         s.synchronize()
         assert torch.equal(got, want[:4])
         assert torch.equal(tbl.moe_experts(ids, w, x), want)
+
+
+@pytest.mark.parametrize("fmt", [INT8, INT4])
+def test_few_matmul_rows_captured_after_a_prompt(side, fmt):
+    """A 512-row product of 7168 x 2048 is 448 workgroups and splits no
+    columns; four rows split them: the partials' buffer is there all the same."""
+    import undertow_amd as U
+    s, c = side
+    rng = np.random.default_rng(fmt)
+    q = U.QTensor(c, fmt, *rand_qtensor(rng, fmt, 7168, 2048), 7168, 2048)
+    x = dev(rng.standard_normal((512, 2048)).astype(np.float32))
+    every, few = (torch.empty((n, 7168), device="cuda") for n in (512, 4))
+    q.matmul(every, x, 512)
+    g, _ = capture(s, lambda: q.matmul(few, x[:4], 4))
+    for _ in range(3):
+        few.zero_()
+        g.replay()
+        s.synchronize()
+        assert torch.equal(few, every[:4])

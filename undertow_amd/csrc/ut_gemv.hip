@@ -1933,6 +1933,8 @@ extern "C" int32_t ut_qtensor_matmul(ut_ctx *ctx, const ut_qtensor *qt, float *o
         plan.add(planes_bytes(seq, qt->in_dim));
         std::vector<void *> ptrs;
         UT_TRY(scratch_acquire(ctx, plan, ptrs));
+        // (an unsplit product takes no partials; one to four rows may)
+        splitk_reserve(ctx);
         return matmul_dev(ctx, qt, x_dev, seq, out_dev, qt->out_dim, 0, ptrs[0]);
     }
     GemvArgs ga;

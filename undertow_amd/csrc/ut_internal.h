@@ -160,6 +160,9 @@ void moe_noalloc_release(const ut_ctx *ctx);
 // first use: four rows of the LM head's logits (129,280) over four splits.
 constexpr int64_t kSplitKPartBytes = int64_t(32) << 20;
 int32_t splitk_buffer(ut_ctx *ctx, int64_t **part);
+// The buffer for later calls, from one that does without it: not while the
+// stream is captured, and not an error where there is no room.
+void splitk_reserve(ut_ctx *ctx);
 int32_t check_device_error(ut_ctx *ctx);
 
 int64_t payload_bytes(int32_t fmt, int64_t out_dim, int64_t in_dim);

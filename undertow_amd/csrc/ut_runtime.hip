@@ -168,6 +168,11 @@ int32_t splitk_buffer(ut_ctx *ctx, int64_t **part) {
     return UT_OK;
 }
 
+void splitk_reserve(ut_ctx *ctx) {
+    int64_t *part = nullptr;
+    if (!ctx->splitk && !stream_capturing(ctx)) (void)splitk_buffer(ctx, &part);
+}
+
 int32_t check_device_error(ut_ctx *ctx) {
     if (!ctx->dev_err) return UT_OK;
     int32_t f = 0;
