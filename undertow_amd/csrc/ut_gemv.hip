@@ -1916,15 +1916,15 @@ extern "C" int32_t ut_qtensor_matmul(ut_ctx *ctx, const ut_qtensor *qt, float *o
     if (qt->fmt == UT_FMT_INT8 && ctx->fast_int8)
         return matmul_fast_i8(ctx, qt, out_dev, qt->out_dim, 0, x_dev, seq);
     if (gemv_direct_ok(qt, x_dev, seq, out_dev)) {
-        // the buffers that other row counts of this weight need are there
-        // after a first call of any, so that those can be captured
+        // this launch needs no memory, other row counts of the weight do: it is
+        // there after a first call of any, so that those can be captured
         if ((ctx->scratch.bytes == 0 || !ctx->splitk) && !stream_capturing(ctx)) {
             ScratchPlan plan;
             plan.add(planes_bytes(seq, qt->in_dim));
             std::vector<void *> ptrs;
-            int64_t *part = nullptr;
-            UT_TRY(scratch_acquire(ctx, plan, ptrs));
-            UT_TRY(splitk_buffer(ctx, &part));
+            const int32_t rc = scratch_acquire(ctx, plan, ptrs, true);
+            if (rc != UT_OK && rc != UT_ERR_OOM) return rc;
+            splitk_reserve(ctx);
         }
         return launch_gemv_direct(ctx, qt, x_dev, seq, out_dev, qt->out_dim);
     }
