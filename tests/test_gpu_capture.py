@@ -106,3 +106,27 @@ def test_few_matmul_rows_captured_after_a_prompt(side, fmt):
         g.replay()
         s.synchronize()
         assert torch.equal(few, every[:4])
+
+
+# a prompt unsplit (1,200 column groups), then fewer rows that split; the same
+# rows over at most 128 positions, whose slices are the context length's
+@pytest.mark.parametrize("first,then", [((300, 300), (129, 300)), ((300, 300), (128, 128)),
+                                        ((128, 129), (128, 128)), ((200, 9000), (20, 9000))])
+def test_shorter_attention_captured_after_a_prompt(side, first, then):
+    import undertow_amd as U
+    s, c = side
+    g = torch.Generator(device="cuda").manual_seed(3)
+    rnd = lambda *d: torch.randn(d, device="cuda", generator=g)
+    T = first[1]
+    kc = U.mla_cache_split(c, rnd(T, 512), rnd(T, 64))
+    q, p = rnd(first[0], 128, 512), rnd(first[0], 128, 64)
+    out = torch.empty_like(q)
+    call = lambda R, T: U.mla_attend_split(c, q[:R], p[:R], kc, T - R, 0.07, out=out[:R])
+    call(*first)
+    gr, _ = capture(s, lambda: call(*then))
+    out.zero_()
+    gr.replay()
+    s.synchronize()
+    got = out[:then[0]].clone()
+    call(*then)
+    assert torch.equal(got, out[:then[0]])

@@ -709,15 +709,22 @@ static int64_t mla_prompt_slice(int64_t R, int64_t H, int64_t T) {
 constexpr int64_t kMlaPromptMinT = 128;
 static bool mla_prompt(int64_t R, int64_t T) { return R > kMlaPromptRows && T > kMlaPromptMinT; }
 
+// Slice partials of any call of up to R rows over up to T positions: scratch
+// that one call left serves every smaller one (a captured one among them).
+// More rows or positions can take fewer slices, so it is the largest of the
+// rules' cases: few rows, short contexts, a prompt's splits (two and more:
+// under 2 kMlaPromptWGs workgroups of 32 columns).
 static size_t mla_mfma_scratch_bytes(int64_t R, int64_t H, int64_t L, int64_t T) {
-    const size_t ns = (size_t)(mla_prompt(R, T) ? mla_prompt_nslice(R, H, T) : mla_mfma_nslice(T)),
-                 RH = (size_t)(R * H);
-    const size_t b = ((ns * RH * 4 + 255) & ~size_t(255)) * 2 + ((ns * L * RH * 4 + 255) & ~size_t(255));
-    if (!mla_prompt(R, T)) return b;
-    // at least a few rows' over the same context: scratch that a prompt left
-    // serves the calls after it
-    const size_t few = mla_mfma_scratch_bytes(kMlaPromptRows, H, L, T);
-    return ns > 1 && b > few ? b : few;
+    auto cols = [&](int64_t r, int64_t t) { return (size_t)((r < R ? r : R) * H * mla_mfma_nslice(t < T ? t : T)); };
+    size_t n = cols(kMlaPromptRows, T);
+    const size_t low = cols(kMlaPromptMinT, kMlaPromptMinT);
+    if (low > n) n = low;
+    if (mla_prompt(R, T)) {
+        const int64_t most = mla_prompt_nslice(1, 32, T), groups = R * H / 32;  // one column group
+        const int64_t wgs = most * groups < 2 * kMlaPromptWGs ? most * groups : 2 * kMlaPromptWGs;
+        if (most > 1 && (size_t)wgs * 32 > n) n = (size_t)wgs * 32;
+    }
+    return ((n * 4 + 255) & ~size_t(255)) * 2 + ((n * L * 4 + 255) & ~size_t(255));
 }
 
 static size_t mla_split_scratch_bytes(int64_t R, int64_t H, int64_t L, int64_t T) {
@@ -741,16 +748,8 @@ int64_t mla_rows_per_call(int64_t R, int64_t H, int64_t L, int64_t P, int64_t T)
 }
 
 size_t mla_rows_scratch_bytes(int64_t R, int64_t H, int64_t L, int64_t P, int64_t T) {
-    const int64_t per = mla_rows_per_call(R, H, L, P, T), n = R < per ? R : per;
-    // (more rows over fewer positions can take more slices in all)
-    size_t most = 0;
-    for (int64_t r = 1; r <= n; r++)
-        for (int64_t t : {T, T < kMlaPromptMinT ? T : kMlaPromptMinT}) {
-            if (r > t) continue;
-            const size_t b = mla_scratch_bytes(r, H, L, P, t);
-            if (b > most) most = b;
-        }
-    return most;
+    const int64_t per = mla_rows_per_call(R, H, L, P, T);
+    return mla_scratch_bytes(R < per ? R : per, H, L, P, T);
 }
 
 size_t mla_kc_scratch_bytes(int64_t R, int64_t H, int64_t L, int64_t T) {
