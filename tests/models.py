@@ -31,6 +31,9 @@ C1_MLA = dict(C1, hidden_size=1024, num_attention_heads=128, kv_lora_rank=512, q
 # each head holds rows past the head (tails of its two 8-row passes).
 C1_MLA_V40 = dict(C1_MLA, v_head_dim=40)
 
+# A value head of 42: the heads' scales start at any even float.
+C1_MLA_V42 = dict(C1_MLA, v_head_dim=42)
+
 # Config 1 with DeepSeek-V3's router shape: 256 routed experts in 8 groups,
 # top-4 groups, top-8 experts (the wave router with four keys per lane,
 # which the gate/up launch runs itself on the decode path).

@@ -10,7 +10,7 @@ tests' 1e-3 / 1e-4 on the logits.
 import numpy as np
 import pytest
 
-from models import C1_MLA, C1_MLA_V40, checkpoint, gpu_model, prompt_ids
+from models import C1_MLA, C1_MLA_V40, C1_MLA_V42, checkpoint, gpu_model, prompt_ids
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -45,3 +45,20 @@ def test_long_prompt_matches_oracle(ctx):
     s.prefill(ids[:90])
     e = np.abs(s.prefill(ids[90:]) - want[90:])
     assert e.max() <= 1e-3 and e.mean() <= 1e-4
+
+
+@pytest.mark.parametrize("cfg,taken", [(C1_MLA_V40, True), (C1_MLA_V42, False)])
+def test_value_heads_of_whole_float4s(ctx, cfg, taken):
+    """absorb_q's matrix-core kernel loads each head's scales 16 bytes at a
+    time, so it leaves a value head that is no multiple of four floats."""
+    ck = checkpoint(cfg, fmt="int4")
+    m = gpu_model(ctx, ck)
+    ids = prompt_ids(150, cfg["vocab_size"], seed=4)
+    ctx.enable_timing(True)
+    before = ctx.kernel_time("absorb_q_rows")[0]
+    got = m.forward(ids)
+    launches = ctx.kernel_time("absorb_q_rows")[0] - before
+    ctx.enable_timing(False)
+    assert (launches > 0) == taken
+    e = np.abs(got - O.Model(ck).forward(ids))
+    assert e.max() <= 1e-3 and e.mean() <= 1e-4, (e.max(), e.mean())

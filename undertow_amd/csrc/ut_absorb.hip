@@ -124,11 +124,13 @@ __global__ __launch_bounds__(256, 2) void k_absorb_q_rows(const uint8_t *__restr
 }
 
 bool absorb_q_rows_ok(const ut_qtensor *kv_b, const float *q, int64_t rows, int64_t nope,
-                      int64_t rope, int64_t pos_base) {
-    // contexts of up to 128 positions keep the vector kernel's rounding, so a
-    // short prompt's rows equal its decode steps' bit for bit
+                      int64_t rope, int64_t vh, int64_t pos_base) {
+    // 16-byte loads of each head's query and scales: rows of 128 + rope and
+    // 128 + vh floats.  Contexts of up to 128 positions keep the vector
+    // kernel's rounding, so a short prompt's rows equal its decode steps' bit
+    // for bit
     return kv_b->fmt == UT_FMT_INT8 && kv_b->in_dim == kAbqCols && nope == 128 && rows > 16 &&
-           pos_base + rows > 128 && rope % 4 == 0 && kv_b->row_bytes % 4 == 0 &&
+           pos_base + rows > 128 && rope % 4 == 0 && vh % 4 == 0 && kv_b->row_bytes % 4 == 0 &&
            ((uintptr_t)kv_b->payload & 3) == 0 && (((uintptr_t)q | (uintptr_t)kv_b->scales) & 15) == 0;
 }
 

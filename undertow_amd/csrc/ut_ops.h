@@ -97,19 +97,16 @@ int32_t launch_pos_add(ut_ctx *ctx, int64_t *p, int64_t n);
 // Absorbed query (attention.rs:204-213): for each (s, h)
 //   qabs[s,h,:] = sum_d (q[s,h,d]*scale[h*kvh+d]) * W[h*kvh+d, :]  (d < nope,
 //   adds in d order) and q_rope[s,h,:] = rope_interleave(q[s,h,nope:], pos_base+s).
-// The same products over more than 16 rows on the f32 matrix cores
-// (ut_absorb.hip): int8 kv_b of latent width 512 (q: nope 128).
-bool absorb_q_rows_ok(const ut_qtensor *kv_b, const float *q, int64_t rows, int64_t nope,
-                      int64_t rope, int64_t pos_base);
-int32_t launch_absorb_q_rows(ut_ctx *ctx, const ut_qtensor *kv_b, const float *q, int64_t rows,
-                             int64_t heads, int64_t rope, int64_t vh, float *qabs, float *qrope,
-                             int64_t pos_base, const float2 *table);
-bool absorb_v_rows_ok(const ut_qtensor *kv_b, const float *clat, int64_t rows);
-int32_t launch_absorb_v_rows(ut_ctx *ctx, const ut_qtensor *kv_b, const float *clat, int64_t rows,
-                             int64_t heads, int64_t nope, int64_t vh, float *out);
 int32_t launch_absorb_q(ut_ctx *ctx, const ut_qtensor *kv_b, const float *q, int64_t rows,
                         int64_t heads, int64_t nope, int64_t rope, int64_t vh, float *qabs,
                         float *qrope, int64_t pos_base, const float2 *table);
+// The same products over more than 16 rows on the f32 matrix cores
+// (ut_absorb.hip): int8 kv_b of latent width 512 (q: nope 128).
+bool absorb_q_rows_ok(const ut_qtensor *kv_b, const float *q, int64_t rows, int64_t nope,
+                      int64_t rope, int64_t vh, int64_t pos_base);
+int32_t launch_absorb_q_rows(ut_ctx *ctx, const ut_qtensor *kv_b, const float *q, int64_t rows,
+                             int64_t heads, int64_t rope, int64_t vh, float *qabs, float *qrope,
+                             int64_t pos_base, const float2 *table);
 // Cache append (attention.rs:168-186) for rows at positions pos_base..:
 // latent = rmsnorm(comp[:L], w), krot = rope_interleave(comp[L:L+P], pos),
 // stored as f32 (latent, krot) or, with kc, in the MFMA attention's split
@@ -127,5 +124,10 @@ int64_t absorb_v_parts(int64_t heads, int64_t vh);
 int32_t launch_absorb_v(ut_ctx *ctx, const ut_qtensor *kv_b, const float *clat, int64_t rows,
                         int64_t heads, int64_t nope, int64_t vh, float *out,
                         uint32_t *vmax = nullptr);
+// The same sums over more than 16 rows on the f32 matrix cores
+// (ut_absorb.hip): weights that absorb_v_max_ok takes.
+bool absorb_v_rows_ok(const ut_qtensor *kv_b, const float *clat, int64_t rows);
+int32_t launch_absorb_v_rows(ut_ctx *ctx, const ut_qtensor *kv_b, const float *clat, int64_t rows,
+                             int64_t heads, int64_t nope, int64_t vh, float *out);
 
 }  // namespace ut

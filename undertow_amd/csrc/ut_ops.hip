@@ -382,7 +382,7 @@ int32_t launch_absorb_q(ut_ctx *ctx, const ut_qtensor *kv_b, const float *q, int
         set_error(ctx, "absorb: kv_lora_rank %lld must be a multiple of 4", (long long)L);
         return UT_ERR_SHAPE;
     }
-    if (!ctx->step_pos && absorb_q_rows_ok(kv_b, q, rows, nope, rope, pos_base))
+    if (!ctx->step_pos && absorb_q_rows_ok(kv_b, q, rows, nope, rope, vh, pos_base))
         return launch_absorb_q_rows(ctx, kv_b, q, rows, heads, rope, vh, qabs, qrope, pos_base, table);
     constexpr int RB = 4;
     const int64_t kvh = nope + vh;
