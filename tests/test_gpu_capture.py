@@ -108,10 +108,12 @@ def test_few_matmul_rows_captured_after_a_prompt(side, fmt):
         assert torch.equal(few, every[:4])
 
 
-# a prompt unsplit (1,200 column groups), then fewer rows that split; the same
-# rows over at most 128 positions, whose slices are the context length's
-@pytest.mark.parametrize("first,then", [((300, 300), (129, 300)), ((300, 300), (128, 128)),
-                                        ((128, 129), (128, 128)), ((200, 9000), (20, 9000))])
+# a prompt unsplit (1,600 column groups), then fewer rows that split; the same
+# rows over at most 128 positions, whose slices are the context length's; few
+# rows whose slices are
+@pytest.mark.parametrize("first,then", [((400, 400), (24, 400)), ((300, 300), (128, 128)),
+                                        ((128, 129), (128, 128)), ((200, 9000), (20, 9000)),
+                                        ((200, 9000), (16, 9000))])
 def test_shorter_attention_captured_after_a_prompt(side, first, then):
     import undertow_amd as U
     s, c = side

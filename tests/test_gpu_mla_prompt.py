@@ -23,10 +23,12 @@ def f64(qabs, qr, lat, kr, base, scale):
     return torch.einsum("rht,tl->rhl", torch.softmax(s, -1), lat.double())
 
 
-# one slice a row (1,024 column groups), several, a tail tile of one
-# position, contexts that end inside the first slice, fewer heads
+# one slice a row, several (an uneven split's last one is short or empty), a
+# tail tile of one position, contexts that end inside the first slice, fewer
+# heads, few column groups either side of the longest context they split
 @pytest.mark.parametrize("R,H,T", [(17, 128, 17), (17, 128, 700), (33, 32, 33), (40, 64, 2049),
-                                   (100, 128, 100), (257, 128, 257), (260, 128, 900)])
+                                   (100, 128, 100), (257, 128, 257), (260, 128, 900), (37, 96, 1500),
+                                   (24, 32, 16384), (24, 32, 16385), (25, 32, 16385)])
 def test_prompt_rows(ctx, R, H, T):
     import undertow_amd as U
     g = torch.Generator(device="cuda").manual_seed(R * T)

@@ -684,19 +684,36 @@ static bool mla_mfma_ok(int64_t H, int64_t L, int64_t P, int64_t T) {
 
 bool mla_kc_ok(int64_t H, int64_t L, int64_t P, int64_t T) { return mla_mfma_ok(H, L, P, T); }
 
-// A call of more than kMlaPromptRows rows: its R*H/32 column groups fill the
-// chip by themselves, so positions are split only as far as that needs
-// (kMlaPromptWGs workgroups; 512 are resident at once) instead of by the
-// context length, and not at all from 1,024 groups on.  512 rows over 512
-// positions: 168 us, and 1,004 us with the slices of the context length (16 a row,
-// whose partials alone are 2.1 GB).
-constexpr int64_t kMlaPromptRows = 16, kMlaPromptWGs = 1024;
+// A call of more than kMlaPromptRows rows: its R*H/32 column groups go far
+// in filling the chip by themselves, so positions are split only as far as
+// that needs instead of by the context length.  512 rows over 512 positions:
+// 168 us unsplit, and 1,004 us with the slices of the context length (16 a
+// row, whose partials alone are 2.1 GB).
+//
+// The split is the one of least time in units of a 16-position tile (1.8 us
+// with two workgroups on a CU): the fullest CU's workgroups pair by pair, a
+// single one at 0.75 of a pair's time, two tiles to start, and the partials'
+// way to memory and back.  Rounding groups up to 1,024 workgroups left a
+// third wave nearly empty: 24 rows of 128 heads over 32,768 positions took
+// 937 us (872 with the context length's slices) and 774 so, 17 over 512
+// 42.5 -> 31.2, 240 over 512 177 -> 111, 64 over 1,024 98 -> 85.
+constexpr int64_t kMlaPromptRows = 16, kMlaPromptWGs = 1536;
 static int64_t mla_prompt_nslice(int64_t R, int64_t H, int64_t T) {  // at most
-    const int64_t groups = R * H / 32;
-    int64_t ns = (kMlaPromptWGs + groups - 1) / groups;
-    const int64_t tiles = (T + kTile16 - 1) / kTile16;
-    if (ns > (tiles + 1) / 2) ns = (tiles + 1) / 2;  // two tiles a slice at least
-    return ns < kCombineSmallSlices ? ns : kCombineSmallSlices;
+    const int64_t groups = R * H / 32, tiles = (T + kTile16 - 1) / kTile16;
+    int64_t best = 1;
+    double least = INFINITY;
+    // two tiles a slice at least
+    for (int64_t ns = 1; ns <= kCombineSmallSlices && ns <= (tiles + 1) / 2; ns++) {
+        const int64_t wgs = ns * groups, per = (wgs + 255) / 256;
+        if (ns > 1 && wgs > kMlaPromptWGs) break;
+        const double t = ((double)(per / 2) + 0.75 * (double)(per % 2)) * (double)((tiles + ns - 1) / ns + 2) +
+                         (ns > 1 ? 0.015 * (double)wgs : 0.0);
+        if (t < least) {
+            least = t;
+            best = ns;
+        }
+    }
+    return best;
 }
 static int64_t mla_prompt_slice(int64_t R, int64_t H, int64_t T) {
     const int64_t ns = mla_prompt_nslice(R, H, T), tiles = (T + kTile16 - 1) / kTile16;
@@ -705,24 +722,33 @@ static int64_t mla_prompt_slice(int64_t R, int64_t H, int64_t T) {
 // Contexts of up to kMlaPromptMinT positions keep the slices of the context
 // length also for many rows, so that a short prompt's rows get the values of
 // its decode steps bit for bit.  The price: 128 rows over 128 positions take
-// 104 us, 129 over 129 without that 52 us.
+// 102 us, 129 over 129 without that 50 us.
+// So do a few column groups over a very long context, where k_mla_mfma16's
+// order of workgroups keeps a slice's positions in one XCD's L2: 24 rows of
+// 32 heads over 32,768 positions 210 us against 235, 20 rows 183 against 205
+// (17 rows 178 / 175; over 16,384 the prompt's slices lead: 24 rows 118
+// against 124, 17 rows 90 against 105).
 constexpr int64_t kMlaPromptMinT = 128;
-static bool mla_prompt(int64_t R, int64_t T) { return R > kMlaPromptRows && T > kMlaPromptMinT; }
+constexpr int64_t kMlaFewGroups = 24, kMlaLongT = 16384;
+static bool mla_prompt(int64_t R, int64_t H, int64_t T) {
+    return R > kMlaPromptRows && T > kMlaPromptMinT && !(R * H / 32 <= kMlaFewGroups && T > kMlaLongT);
+}
 
 // Slice partials of any call of up to R rows over up to T positions: scratch
 // that one call left serves every smaller one (a captured one among them).
 // More rows or positions can take fewer slices, so it is the largest of the
-// rules' cases: few rows, short contexts, a prompt's splits (two and more:
-// under 2 kMlaPromptWGs workgroups of 32 columns).
+// rules' cases: few rows or few column groups, short contexts, a prompt's
+// splits (two and more: up to kMlaPromptWGs workgroups of 32 columns).
 static size_t mla_mfma_scratch_bytes(int64_t R, int64_t H, int64_t L, int64_t T) {
     auto cols = [&](int64_t r, int64_t t) { return (size_t)((r < R ? r : R) * H * mla_mfma_nslice(t < T ? t : T)); };
-    size_t n = cols(kMlaPromptRows, T);
+    const int64_t few = T > kMlaLongT ? kMlaFewGroups * 32 / H : 0;
+    size_t n = cols(few > kMlaPromptRows ? few : kMlaPromptRows, T);
     const size_t low = cols(kMlaPromptMinT, kMlaPromptMinT);
     if (low > n) n = low;
-    if (mla_prompt(R, T)) {
-        const int64_t most = mla_prompt_nslice(1, 32, T), groups = R * H / 32;  // one column group
-        const int64_t wgs = most * groups < 2 * kMlaPromptWGs ? most * groups : 2 * kMlaPromptWGs;
-        if (most > 1 && (size_t)wgs * 32 > n) n = (size_t)wgs * 32;
+    if (mla_prompt(R, H, T)) {
+        const int64_t groups = R * H / 32;
+        const int64_t wgs = kCombineSmallSlices * groups < kMlaPromptWGs ? kCombineSmallSlices * groups : kMlaPromptWGs;
+        if ((size_t)wgs * 32 > n) n = (size_t)wgs * 32;
     }
     return ((n * 4 + 255) & ~size_t(255)) * 2 + ((n * L * 4 + 255) & ~size_t(255));
 }
@@ -776,7 +802,7 @@ int32_t launch_mla_attend_kc(ut_ctx *ctx, const float *qabs, const float *qrope,
                        "16-byte aligned cache and at most %d slices", kMlaMaxSlices);
         return UT_ERR_SHAPE;
     }
-    const bool prompt = mla_prompt(R, T) && !ctx->step_pos;
+    const bool prompt = mla_prompt(R, H, T) && !ctx->step_pos;
     MlaMfmaArgs a{};
     a.slen = prompt ? mla_prompt_slice(R, H, T) : 0;
     a.clat = clat;
