@@ -144,13 +144,35 @@ def test_f32_rows_equal_one_row_calls(ctx, o, i):
     x = rng.standard_normal((131, i)).astype(np.float32)
     rows = [0, 3, 4, 63, 64, 127, 128, 130]
     one = np.concatenate([run(ctx, q, x[r:r + 1]) for r in rows])
-    for seq in (5, 64, 131):
+    for seq in (5, 9, 64, 131):
         got = run(ctx, q, x[:seq])
         n = [k for k, r in enumerate(rows) if r < seq]
         assert np.array_equal(got[[rows[k] for k in n]], one[n]), seq
     ref = x.astype(np.float64) @ w.astype(np.float64).T
     err = np.linalg.norm(run(ctx, q, x) - ref) / np.linalg.norm(ref)
     assert err <= 2.0 ** -23 * max(1.0, np.log2(i))  # tree-wise f32 sums
+
+
+# the lines of gemm_f32_min_rows: split and unsplit slices of one to four
+# steps, more tiles than one wave; (rows in passes, rows in the product)
+@pytest.mark.parametrize("o,i,few,more", [(64, 64, 4, 5), (65, 128, 8, 9), (65, 132, 12, 13), (65, 252, 13, 14),
+                                          (16500, 252, 24, 25), (130, 1028, 8, 9), (256, 1024, 4, 5),
+                                          (1024, 7168, 8, 9), (3000, 1500, 12, 13),
+                                          (2048, 7168, 16, 17)])
+def test_f32_rows_take_the_faster_way(ctx, o, i, few, more):
+    import undertow_amd as U
+    rng = np.random.default_rng(o + i)
+    q = U.QTensor(ctx, U.F32, rng.standard_normal((o, i)).astype(np.float32), None, o, i)
+    x = rng.standard_normal((more, i)).astype(np.float32)
+    got, launches = {}, {}
+    ctx.enable_timing(True)
+    for n in (few, more):
+        before = ctx.kernel_time("gemm_f32")[0]
+        got[n] = run(ctx, q, x[:n])
+        launches[n] = ctx.kernel_time("gemm_f32")[0] - before
+    ctx.enable_timing(False)
+    assert launches == {few: 0, more: 1}
+    assert np.array_equal(got[more][:few], got[few])
 
 
 # unsplit slices either side of the line between the two LDS tiles (16 stages
