@@ -266,7 +266,10 @@ int32_t ut_argmax_rows(ut_ctx *ctx, const float *logits_dev, int64_t rows, int64
  * rows x H heads: row s sees n_ctx = pos_base + s + 1 cache positions,
  * score_t = (qabs.latent_t + q_rope.krot_t) * scale, fp32 softmax,
  * clat = sum_t p_t latent_t.  qabs [R,H,L], q_rope [R,H,P], latent [T,L],
- * krot [T,P] (T >= pos_base + R), clat [R,H,L]; all f32. */
+ * krot [T,P] (T >= pos_base + R), clat [R,H,L]; all f32.  A row's bits do not
+ * depend on the other rows of the call; for the shapes of
+ * ut_mla_attend_split that holds where R <= 16 or pos_base + R <= 128, and
+ * larger calls agree with smaller ones to 1e-4 of the largest output. */
 int32_t ut_mla_attend(ut_ctx *ctx, const float *qabs_dev, const float *q_rope_dev,
                       const float *latent_dev, const float *krot_dev, int64_t R, int64_t H,
                       int64_t L, int64_t P, int64_t pos_base, float scale, float *clat_dev);

@@ -128,6 +128,26 @@ def test_c4_decode_rows_equal_verify_rows(c4, rows):
     assert np.array_equal(one, many)
 
 
+def test_c4_prompt_rows_equal_decode_steps(c4):
+    """A prompt's products at full width (the LM head, the grouped experts of
+    256, the gate's seven steps of 1,024 columns): 40 rows in one call are
+    their decode steps, bit for bit.  150 rows round differently from
+    their 16-row calls in attention and absorbed query, past 128 positions:
+    the attention's contract is 1e-4 of its largest output, and four layers
+    hand theirs on, so 4e-4 of the largest logit (and the oracle tests' mean;
+    measured 1e-4 of it at one row, 5e-6 at the median row, as far as the
+    16-row calls are from the oracle)."""
+    ck, m, om, prompt, stream = c4
+    ids = prompt_ids(150, C4["vocab_size"], seed=23)
+    s = m.session()
+    one = np.stack([s.decode(t) for t in ids[:40]])
+    assert np.array_equal(m.session().prefill(ids[:40]), one)
+    s = m.session()
+    few = np.concatenate([s.prefill(ids[i:i + 16]) for i in range(0, 150, 16)])
+    err = np.abs(m.session().prefill(ids) - few)
+    assert err.max() <= 4e-4 * np.abs(few).max() and err.mean() <= 1e-4, (err.max(), err.mean())
+
+
 LONG = 72  # three 32-position attention slices per row at the end
 
 
@@ -143,8 +163,8 @@ def c4_long(c4):
 
 def test_c4_long_prompt_logits_match_oracle(c4, c4_long):
     """Multi-slice attention in the model path (rows past 32 positions take
-    two and three slices, merged by the slice combine), prefill chunks of
-    four rows over a 72-token prompt."""
+    two and three slices, merged by the slice combine), one prefill call of
+    72 rows."""
     ck, m, om, prompt, stream = c4
     long_prompt, want, lstream = c4_long
     got = m.forward(long_prompt)

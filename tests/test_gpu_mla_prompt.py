@@ -26,7 +26,7 @@ def f64(qabs, qr, lat, kr, base, scale):
 # one slice a row, several (an uneven split's last one is short or empty), a
 # tail tile of one position, contexts that end inside the first slice, fewer
 # heads, few column groups either side of the longest context they split
-@pytest.mark.parametrize("R,H,T", [(17, 128, 17), (17, 128, 700), (33, 32, 33), (40, 64, 2049),
+@pytest.mark.parametrize("R,H,T", [(17, 128, 17), (17, 128, 129), (17, 128, 700), (33, 32, 33), (40, 64, 2049),
                                    (100, 128, 100), (257, 128, 257), (260, 128, 900), (37, 96, 1500),
                                    (24, 32, 16384), (24, 32, 16385), (25, 32, 16385)])
 def test_prompt_rows(ctx, R, H, T):
@@ -48,8 +48,8 @@ def test_prompt_rows(ctx, R, H, T):
     assert float((got - want).norm()) <= 1.05 * float((few - want).norm())
 
 
-@pytest.mark.parametrize("R,H,T", [(16, 128, 16), (16, 128, 513), (20, 128, 100), (17, 128, 128),
-                                   (128, 32, 128), (4, 128, 33)])
+@pytest.mark.parametrize("R,H,T", [(16, 128, 16), (16, 128, 129), (16, 128, 513), (20, 128, 100),
+                                   (17, 128, 128), (128, 32, 128), (4, 128, 33), (24, 32, 16400)])
 def test_rows_merge_equals_single_rows(ctx, R, H, T):
     """Calls that keep the slices of the context length merge them with the
     same sums whatever kernel merges: rows equal their own one-row calls."""

@@ -8,8 +8,9 @@
 //                  slice's max / sum / unnormalised context are written out.
 //   k_mla_combine  merges the slices: M = max m_j, L = sum l_j e^(m_j-M),
 //                  clat = sum o_j e^(m_j-M) / L.
-// Row s sees n_ctx = pos_base + s + 1 positions.  Slice boundaries depend
-// only on the position index, so a row's result does not depend on R.
+// Row s sees n_ctx = pos_base + s + 1 positions.  These kernels' slice
+// boundaries depend only on the position index, so a row's result does not
+// depend on R (the matrix-core kernel's rules stand below).
 // Scores accumulate as the reference does: sum_i q_i*lat_i then
 // sum_i qr_i*krot_i, sequential f32 adds without contraction.
 #include "ut_internal.h"
@@ -183,7 +184,8 @@ __global__ __launch_bounds__(256) void k_mla_combine(const float *__restrict__ p
 // 77 KiB of LDS and < 256 registers per lane let two workgroups share a CU.
 // The slice writes (m, l, O) to the partial buffers, k_mla_combine_mfma
 // merges the slices.  The slice length depends only on the row's context
-// length, so a row's result is the same whichever rows share the call.
+// length, so a row's result is the same whichever rows share the call -- but
+// for a prompt's rows (mla_prompt), whose slices follow the rows at hand.
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
@@ -192,7 +194,7 @@ typedef float f32x16_t __attribute__((ext_vector_type(16)));
 // 16-position tiles, at least 32 and at most UT_MLA_SLICE_CAP = 512 (so at
 // most 64 slices up to 32768 positions, n_ctx/512 beyond).  A function of
 // n_ctx alone, so a row's result does not depend on which rows share the
-// call; no power-of-two steps, so neighbouring context lengths get similar
+// call (a prompt's slices: mla_prompt_slice); no power-of-two steps, so neighbouring context lengths get similar
 // slice counts.  The cap of 512 against 256 halves the slice partials past
 // 16384 positions: at T = 32768 two- and four-row calls went from 97.2 to
 // 88.0 us and from 179.3 to 154.6 us, one-row calls from 56.6 to 61.1 us
