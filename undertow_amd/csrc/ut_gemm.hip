@@ -277,7 +277,7 @@ constexpr int64_t kGlMinRows = 32;
 // Four buffers of 64-column stages, three in flight, copy half lines of 128
 // bytes: 243 us at 7168 x 16384 and 1,637 at 129280 x 7168, with PIPE reads
 // 250 and 1,686.
-constexpr int kGlTM = 2, kGlWM = 2, kGlS = 128;
+constexpr int kGlTM = 2, kGlWM = 2;
 constexpr int kGlRows = 128;  // weight rows per workgroup
 constexpr int64_t kGlLong = 16;
 template <bool LONG> constexpr int gl_to() { return LONG ? 4 : 2; }
@@ -285,7 +285,7 @@ template <bool LONG> constexpr int gl_threads() { return 64 * kGlRows / (16 * gl
 template <int FMT, bool LONG>
 __global__ __launch_bounds__(gl_threads<LONG>(), 2) void k_gemm_lds(GemmArgs a) {
     constexpr int TO = gl_to<LONG>(), WO = kGlRows / (16 * TO);
-    using L = GemmLds<FMT, TO, kGlTM, WO, kGlWM, kGlS>;
+    using L = GemmLds<FMT, TO, kGlTM, WO, kGlWM>;
     __shared__ L s0, s1;
     const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
     const int unit = (j / a.tm) * 8 + xcd, mt = j % a.tm;
@@ -294,14 +294,14 @@ __global__ __launch_bounds__(gl_threads<LONG>(), 2) void k_gemm_lds(GemmArgs a) 
     const GemmWeight &W = a.w[wi];
     const int wave = threadIdx.x >> 6;
     const int64_t ob = (int64_t)ot * L::kARows, mb = (int64_t)mt * (16 * kGlTM * kGlWM);
-    GemmSrc<FMT, TO, kGlTM, WO, kGlWM, kGlS> src;
-    gemm_src<FMT, TO, kGlTM, WO, kGlWM, kGlS>(
+    GemmSrc<FMT, TO, kGlTM, WO, kGlWM> src;
+    gemm_src<FMT, TO, kGlTM, WO, kGlWM>(
         src,
         [&](int row) { return W.w + (ob + row < W.O ? ob + row : W.O - 1) * a.row_bytes; },
         [&](int m, int p) { return a.pl + ((mb + m < a.M ? mb + m : a.M - 1) * 3 + p) * a.kp; });
     const int64_t kb = z * a.kslice, ke = kb + a.kslice < a.kp ? kb + a.kslice : a.kp;
     ut_i32x4 acc[TO][kGlTM][3];
-    gemm_tile_lds<LONG, FMT, TO, kGlTM, WO, kGlWM, kGlS>(src, a.row_bytes, kb, ke, s0, s1, acc);
+    gemm_tile_lds<LONG, FMT, TO, kGlTM, WO, kGlWM>(src, a.row_bytes, kb, ke, s0, s1, acc);
     gemm_store<FMT, TO, kGlTM>(a, wi, acc, ob + (wave % WO) * (16 * TO),
                                mb + (wave / WO) * (16 * kGlTM), z);
 }
@@ -396,7 +396,7 @@ int32_t launch_gemm(ut_ctx *ctx, const ut_qtensor *w, const DigitPlanes &x, int6
         else UT_GM(F, 2, U);            \
     } while (0)
         if (big) {
-            const bool lng = a.kslice > kGlLong * kGlS;
+            const bool lng = a.kslice > kGlLong * kGemmStep;
 #define UT_GL(F, LG) hipLaunchKernelGGL((k_gemm_lds<F, LG>), grid, dim3(gl_threads<LG>()), 0, ctx->stream, a)
             if (w->fmt == UT_FMT_INT8) {
                 if (lng) UT_GL(UT_FMT_INT8, true);

@@ -16,7 +16,8 @@
 // fetched a step of 128 columns ahead; the barrier waits for LDS only, so the
 // loads stay in flight across it.  LDS rows of 128 bytes keep
 // their 16-byte chunks XOR-swizzled by the row's low three bits: eight lanes
-// that read one chunk of eight rows use all 32 banks.
+// that read one chunk of eight rows read eight different slots of the 256
+// bytes that the 64 banks hold.
 #pragma once
 
 #include "ut_gemv_mfma.h"
@@ -108,16 +109,15 @@ template <int FMT> __device__ __forceinline__ int32_t gemm_exp(int32_t e) {
 
 // acc[t][n][p] = tile over columns [kb, ke) (kb a multiple of 128, columns
 // past K zero in the planes).  src[i]: the digit bytes of this thread's
-// staging chunk i at column 0 (its chunk offset included).  D (even): steps
-// held in registers, D - 1 of them in flight while one computes.  Four
-// measured no better than two at 5 to 64 rows (int8 7168 x 16384 at 5 rows
-// 44.2 against 43.7 us) and worse at 512 (int4 18432 x 7168 272 against
-// 260 us).
-template <int FMT, int TO, int TM, bool UNAL, int D = 2>
+// staging chunk i at column 0 (its chunk offset included).  Two steps are held
+// in registers, one in flight while the other computes.  Four measured no
+// better at 5 to 64 rows (int8 7168 x 16384 at 5 rows 44.2 against 43.7 us)
+// and worse at 512 (int4 18432 x 7168 272 against 260 us).
+template <int FMT, int TO, int TM, bool UNAL>
 __device__ __forceinline__ void gemm_tile(const GemmRows<TO> &rows, int64_t len, int64_t kb,
                                           int64_t ke, const int8_t *const (&src)[gemm_stage_n<TM>()],
                                           uint4 *lds, ut_i32x4 (&acc)[TO][TM][3]) {
-    static_assert(D % 2 == 0, "the LDS buffer of a step is its slot's parity");
+    constexpr int D = 2;  // (the LDS buffer of a step is its slot's parity)
     constexpr int NB = gemm_stage_n<TM>(), CH = TM * 48 * 8;
     const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, q = lane >> 4;
 #pragma unroll
@@ -186,12 +186,13 @@ __device__ __forceinline__ void gemm_tile(const GemmRows<TO> &rows, int64_t len,
 // matrix cores bound: a lane's direct weight load takes 16 bytes of its own
 // row, so each 16 lanes touch 16 cache lines, and at 512 rows those lookups
 // held the direct tile at a quarter of the matrix rate.  Here both operands
-// are copied by global_load_lds (no registers) in stages of S columns, one
+// are copied by global_load_lds (no registers) in stages of 128 columns, one
 // in flight while one is computed on, and WO x WM waves share them: each
 // wave TO tiles of 16 weight rows against 16 TM activation rows.  LDS has
 // 64 banks: a staged row's 16-byte chunks are XOR-swizzled so that the 16
 // rows a lane group reads take 16 different slots of 256 bytes.
-template <int FMT, int TO, int TM, int WO, int WM, int S> struct GemmLds {
+template <int FMT, int TO, int TM, int WO, int WM> struct GemmLds {
+    static constexpr int S = kGemmStep;
     static constexpr int kThreads = 64 * WO * WM;
     static constexpr int kARows = 16 * TO * WO, kBRows = 48 * TM * WM;
     static constexpr int kAC = FMT == UT_FMT_INT8 ? S / 16 : S / 32, kBC = S / 16;  // chunks of a row
@@ -202,22 +203,22 @@ template <int FMT, int TO, int TM, int WO, int WM, int S> struct GemmLds {
 };
 // Chunk c of a row of C chunks sits at slot c ^ gemm_swz<C>(row).
 template <int C> __device__ __forceinline__ int gemm_swz(int row) {
-    static_assert(C == 2 || C == 4 || C == 8, "rows of 32, 64 or 128 bytes");
+    static_assert(C == 4 || C == 8, "rows of 64 or 128 bytes");
     return (row / (16 / C)) & (C - 1);
 }
 
 // This thread's copy sources at column 0 (row pointers are the caller's);
 // aoff: the A chunk's byte offset in its row's step.
-template <int FMT, int TO, int TM, int WO, int WM, int S> struct GemmSrc {
-    using L = GemmLds<FMT, TO, TM, WO, WM, S>;
+template <int FMT, int TO, int TM, int WO, int WM> struct GemmSrc {
+    using L = GemmLds<FMT, TO, TM, WO, WM>;
     const uint8_t *a[L::kNA];
     const int8_t *b[L::kNB];
     int aoff;
 };
-template <int FMT, int TO, int TM, int WO, int WM, int S, typename ARow, typename BRow>
-__device__ __forceinline__ void gemm_src(GemmSrc<FMT, TO, TM, WO, WM, S> &s, ARow &&arow,
+template <int FMT, int TO, int TM, int WO, int WM, typename ARow, typename BRow>
+__device__ __forceinline__ void gemm_src(GemmSrc<FMT, TO, TM, WO, WM> &s, ARow &&arow,
                                          BRow &&brow) {
-    using L = GemmLds<FMT, TO, TM, WO, WM, S>;
+    using L = GemmLds<FMT, TO, TM, WO, WM>;
     const int tid = threadIdx.x;
 #pragma unroll
     for (int i = 0; i < L::kNA; i++) {
@@ -248,13 +249,13 @@ __device__ __forceinline__ void gemm_wait_copies() {
 // PIPE: a stage's second half is multiplied after the next stage's first half
 // has been read, so a wave's LDS reads run beside its matrix instructions
 // instead of before them (twice the fragments in registers).
-template <bool PIPE, int FMT, int TO, int TM, int WO, int WM, int S>
-__device__ __forceinline__ void gemm_tile_lds(const GemmSrc<FMT, TO, TM, WO, WM, S> &src,
-                                              int64_t len, int64_t kb, int64_t ke,
-                                              GemmLds<FMT, TO, TM, WO, WM, S> &s0,
-                                              GemmLds<FMT, TO, TM, WO, WM, S> &s1,
+template <bool PIPE, int FMT, int TO, int TM, int WO, int WM>
+__device__ __forceinline__ void gemm_tile_lds(const GemmSrc<FMT, TO, TM, WO, WM> &src, int64_t len,
+                                              int64_t kb, int64_t ke, GemmLds<FMT, TO, TM, WO, WM> &s0,
+                                              GemmLds<FMT, TO, TM, WO, WM> &s1,
                                               ut_i32x4 (&acc)[TO][TM][3]) {
-    using L = GemmLds<FMT, TO, TM, WO, WM, S>;
+    constexpr int S = kGemmStep;
+    using L = GemmLds<FMT, TO, TM, WO, WM>;
     const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, q = lane >> 4, wave = tid >> 6;
     const int wo = wave % WO, wm = wave / WO;
 #pragma unroll
@@ -283,79 +284,56 @@ __device__ __forceinline__ void gemm_tile_lds(const GemmSrc<FMT, TO, TM, WO, WM,
                     (const void *)(src.b[j] + k),
                     (__attribute__((address_space(3))) void *)(s.b + j * L::kThreads + w64), 16, 0, 0);
     };
-    auto compute = [&](const L &s) {
-#pragma unroll
-        for (int h = 0; h < S / 64; h++) {
-            const int c = 4 * h + q;  // this lane's 16 columns of the stage
-            ut_i32x4 f[TO], w[TM][3];
-#pragma unroll
-            for (int t = 0; t < TO; t++) {
-                const int row = (wo * TO + t) * 16 + r;
-                if constexpr (FMT == UT_FMT_INT8) {
-                    const uint4 v = s.a[row * L::kAC + (c ^ gemm_swz<L::kAC>(row))];
-                    f[t] = ut_i32x4{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
-                } else {
-                    const uint2 v = ((const uint2 *)&s.a[row * L::kAC + ((c >> 1) ^ gemm_swz<L::kAC>(row))])[c & 1];
-                    f[t] = gemm_i4_codes(v.x, v.y);
-                }
-            }
-#pragma unroll
-            for (int m = 0; m < TM; m++)
-#pragma unroll
-                for (int p = 0; p < 3; p++) {
-                    const int row = ((wm * TM + m) * 3 + p) * 16 + r;
-                    const uint4 v = s.b[row * L::kBC + (c ^ gemm_swz<L::kBC>(row))];
-                    w[m][p] = ut_i32x4{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
-                }
-#pragma unroll
-            for (int m = 0; m < TM; m++)
-#pragma unroll
-                for (int p = 0; p < 3; p++)
-#pragma unroll
-                    for (int t = 0; t < TO; t++)
-                        acc[t][m][p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(f[t], w[m][p], acc[t][m][p], 0, 0, 0);
+    // the operands of half stage h: weights (int4 codes still packed), digits
+    auto frag_a = [&](const L &s, int h, int t) {
+        const int c = 4 * h + q, row = (wo * TO + t) * 16 + r;  // c: this lane's 16 columns
+        ut_i32x4 x;
+        if constexpr (FMT == UT_FMT_INT8) {
+            const uint4 v = s.a[row * L::kAC + (c ^ gemm_swz<L::kAC>(row))];
+            x = ut_i32x4{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
+        } else {
+            const uint2 v = ((const uint2 *)&s.a[row * L::kAC + ((c >> 1) ^ gemm_swz<L::kAC>(row))])[c & 1];
+            x[0] = (int)v.x;
+            x[1] = (int)v.y;
         }
+        return x;
     };
-    struct Frag {
-        ut_i32x4 a[TO], b[TM][3];  // a: int4 codes still packed
-    };
-    auto read = [&](const L &s, int h, Frag &x) {
-        const int c = 4 * h + q;  // this lane's 16 columns of the stage
-#pragma unroll
-        for (int t = 0; t < TO; t++) {
-            const int row = (wo * TO + t) * 16 + r;
-            if constexpr (FMT == UT_FMT_INT8) {
-                const uint4 v = s.a[row * L::kAC + (c ^ gemm_swz<L::kAC>(row))];
-                x.a[t] = ut_i32x4{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
-            } else {
-                const uint2 v = ((const uint2 *)&s.a[row * L::kAC + ((c >> 1) ^ gemm_swz<L::kAC>(row))])[c & 1];
-                x.a[t][0] = (int)v.x;
-                x.a[t][1] = (int)v.y;
-            }
-        }
+    auto frag_b = [&](const L &s, int h, ut_i32x4 (&x)[TM][3]) {
 #pragma unroll
         for (int m = 0; m < TM; m++)
 #pragma unroll
             for (int p = 0; p < 3; p++) {
                 const int row = ((wm * TM + m) * 3 + p) * 16 + r;
-                const uint4 v = s.b[row * L::kBC + (c ^ gemm_swz<L::kBC>(row))];
-                x.b[m][p] = ut_i32x4{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
+                const uint4 v = s.b[row * L::kBC + ((4 * h + q) ^ gemm_swz<L::kBC>(row))];
+                x[m][p] = ut_i32x4{(int)v.x, (int)v.y, (int)v.z, (int)v.w};
             }
     };
-    auto multiply = [&](const Frag &x) {
-        ut_i32x4 f[TO];
-#pragma unroll
-        for (int t = 0; t < TO; t++) {
-            if constexpr (FMT == UT_FMT_INT8) f[t] = x.a[t];
-            else f[t] = gemm_i4_codes((uint32_t)x.a[t][0], (uint32_t)x.a[t][1]);
-        }
+    auto codes = [](const ut_i32x4 &x) {
+        if constexpr (FMT == UT_FMT_INT8) return x;
+        else return gemm_i4_codes((uint32_t)x[0], (uint32_t)x[1]);
+    };
+    auto products = [&](const ut_i32x4 (&f)[TO], const ut_i32x4 (&x)[TM][3]) {
 #pragma unroll
         for (int m = 0; m < TM; m++)
 #pragma unroll
             for (int p = 0; p < 3; p++)
 #pragma unroll
                 for (int t = 0; t < TO; t++)
-                    acc[t][m][p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(f[t], x.b[m][p], acc[t][m][p], 0, 0, 0);
+                    acc[t][m][p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(f[t], x[m][p], acc[t][m][p], 0, 0, 0);
+    };
+    struct Frag {
+        ut_i32x4 a[TO], b[TM][3];
+    };
+    auto read = [&](const L &s, int h, Frag &x) {
+#pragma unroll
+        for (int t = 0; t < TO; t++) x.a[t] = frag_a(s, h, t);
+        frag_b(s, h, x.b);
+    };
+    auto multiply = [&](const Frag &x) {
+        ut_i32x4 f[TO];
+#pragma unroll
+        for (int t = 0; t < TO; t++) f[t] = codes(x.a[t]);
+        products(f, x.b);
     };
     Frag f0, f1;
     // step i: its stage has landed, the other buffer is read and gets the next
@@ -363,7 +341,6 @@ __device__ __forceinline__ void gemm_tile_lds(const GemmSrc<FMT, TO, TM, WO, WM,
         gemm_wait_copies();
         copy(other, i + 1);
         if constexpr (PIPE) {
-            static_assert(S == 128, "two halves");
             read(s, 0, f0);
             __builtin_amdgcn_sched_barrier(0);
             if (i) multiply(f1);
@@ -371,7 +348,16 @@ __device__ __forceinline__ void gemm_tile_lds(const GemmSrc<FMT, TO, TM, WO, WM,
             __builtin_amdgcn_sched_barrier(0);
             multiply(f0);
         } else {
-            compute(s);
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                // (unpacked as they are read: after the digits' reads int4
+                // 24576 x 1536 at 509 rows took 112 us, 79 so)
+                ut_i32x4 f[TO], x[TM][3];
+#pragma unroll
+                for (int t = 0; t < TO; t++) f[t] = codes(frag_a(s, h, t));
+                frag_b(s, h, x);
+                products(f, x);
+            }
         }
     };
     copy(s0, 0);

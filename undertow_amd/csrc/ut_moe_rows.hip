@@ -136,14 +136,14 @@ struct MoeRowsArgs {
     float *out;                  // gate/up: h [pairs][I]; down: d [pairs][H]
 };
 
-// Weight tiles of 16 rows per wave, columns per LDS stage.  Four workgroups
+// Weight tiles of 16 rows per wave.  Four workgroups
 // of 128 weight rows per CU (int4; 40 KB of LDS each): config 2's int4 block
 // at 500 rows 1,315 us with direct weight loads, 1,239 so; at 64 rows 725 ->
 // 669, at 5 rows 235 -> 205.  256-row workgroups, two per CU: 1,279 / 660 /
 // 224; stages of 64 columns: 1,564 / 817 / 270.  Up to 64 rows the weights'
 // read bounds it (222 experts, 4.9 GB, at 64 rows); at 500 the read (0.83 ms)
 // and the padded tiles' matrix work (23 of 32 rows on average) together do.
-constexpr int kMrTO = 2, kMrS = 128;
+constexpr int kMrTO = 2;
 constexpr int kMrRows = 64 * kMrTO;
 
 // A workgroup's tile: weight rows wrow(row of the tile) against a tile's
@@ -151,12 +151,12 @@ constexpr int kMrRows = 64 * kMrTO;
 template <int FMT, int TM, typename W, typename A>
 __device__ __forceinline__ void rows_tile(const MoeRowsArgs &a, int n, int64_t len, W &&wrow,
                                           A &&arow, void *s0, void *s1, ut_i32x4 (&acc)[kMrTO][TM][3]) {
-    using L = GemmLds<FMT, kMrTO, TM, 4, 1, kMrS>;
-    GemmSrc<FMT, kMrTO, TM, 4, 1, kMrS> src;
-    gemm_src<FMT, kMrTO, TM, 4, 1, kMrS>(src, wrow, [&](int m, int p) {
+    using L = GemmLds<FMT, kMrTO, TM, 4, 1>;
+    GemmSrc<FMT, kMrTO, TM, 4, 1> src;
+    gemm_src<FMT, kMrTO, TM, 4, 1>(src, wrow, [&](int m, int p) {
         return a.pl + (arow(m < n ? m : n - 1) * 3 + p) * a.kp;
     });
-    gemm_tile_lds<false, FMT, kMrTO, TM, 4, 1, kMrS>(src, len, 0, a.kp, *(L *)s0, *(L *)s1, acc);
+    gemm_tile_lds<false, FMT, kMrTO, TM, 4, 1>(src, len, 0, a.kp, *(L *)s0, *(L *)s1, acc);
 }
 
 // Gate and up of kMrRows / 2 h rows against a tile's rows: a wave's weight
@@ -241,7 +241,7 @@ __device__ __forceinline__ void rows_down(const MoeRowsArgs &a, const MoeTile &t
 template <int FMT, bool DOWN>
 __global__ __launch_bounds__(kGemmThreads, FMT == UT_FMT_INT4 ? 4 : 2) void k_moe_rows(MoeRowsArgs a, int nrt) {
     // two objects: the compiler then knows which one a copy in flight fills
-    __shared__ GemmLds<FMT, kMrTO, 2, 4, 1, kMrS> s0, s1;
+    __shared__ GemmLds<FMT, kMrTO, 2, 4, 1> s0, s1;
     const int ti = blockIdx.x / nrt, rt = blockIdx.x - ti * nrt;
     if (ti >= *a.ntiles) return;
     const MoeTile t = a.tiles[ti];
