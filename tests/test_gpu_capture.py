@@ -108,6 +108,28 @@ def test_few_matmul_rows_captured_after_a_prompt(side, fmt):
         assert torch.equal(few, every[:4])
 
 
+def test_product_captured_without_partials(side):
+    """A first product under capture has no buffer for the partials of a K
+    split and runs unsplit; the arena is there from a call of another kind."""
+    import undertow_amd as U
+    s, c = side
+    rng = np.random.default_rng(4)
+    q = U.QTensor(c, INT4, *rand_qtensor(rng, INT4, 1024, 7168), 1024, 7168)
+    x = dev(rng.standard_normal((37, 7168)).astype(np.float32))
+    y = torch.empty((37, 1024), device="cuda")
+    qa = torch.randn((16, 128, 576), device="cuda")  # 67 MB of slice partials, no split-K buffer
+    kc = U.mla_cache_split(c, torch.randn((512, 512), device="cuda"), torch.randn((512, 64), device="cuda"))
+    U.mla_attend_split(c, qa[..., :512].contiguous(), qa[..., 512:].contiguous(), kc, 496, 0.07)
+    g, _ = capture(s, lambda: q.matmul(y, x, 37))
+    for _ in range(3):
+        y.zero_()
+        g.replay()
+        s.synchronize()
+        got = y.clone()
+        q.matmul(y, x, 37)  # split, from the first eager call on
+        assert torch.equal(got, y)
+
+
 # a prompt unsplit (1,600 column groups), then fewer rows that split; the same
 # rows over at most 128 positions, whose slices are the context length's; few
 # rows whose slices are

@@ -24,12 +24,20 @@ def table(ctx, rng, fmt, E, H, I, skip=()):
     return tbl
 
 
+def graph_nodes(g):
+    import ctypes as C
+    import undertow_amd as U
+    n = C.c_size_t(0)  # (through the library: the HIP runtime that it is linked to)
+    assert U.lib().hipGraphGetNodes(C.c_void_p(g.raw_cuda_graph()), None, C.byref(n)) == 0
+    return n.value
+
+
 def by_fours(tbl, ids, w, x):
     return torch.cat([tbl.moe_experts(ids[r:r + 4].contiguous(), w[r:r + 4].contiguous(),
                                       x[r:r + 4].contiguous()) for r in range(0, len(x), 4)])
 
 
-# h rows of a 128-row tile and remainders, down rows of a 256-row tile and
+# h rows of a 64-row tile and remainders, down rows of a 128-row tile and
 # remainders, widths with and without padded planes
 @pytest.mark.parametrize("fmt,H,I", [(INT4, 512, 256), (INT4, 288, 160), (INT8, 272, 144),
                                      (INT8, 256, 128), (INT4, 7168, 2048)])
@@ -100,11 +108,16 @@ def test_routed_rows_equal_route_then_experts(ctx, E, k, ng, tg):
 
 
 def test_rows_under_capture_without_scratch_fall_back(ctx):
-    """A captured call whose grouped scratch is not there yet takes the
-    four-row passes (which one earlier call of four rows sized)."""
+    """A captured call whose grouped scratch is not there takes the four-row
+    passes (which one earlier call of four rows sized): its graph holds their
+    launches, three and more per pass, and not the grouped path's six."""
     import undertow_amd as U
     rng = np.random.default_rng(8)
-    E, H, I, k, rows = 6, 256, 128, 2, 40
+    E, H, I, k, rows = 6, 256, 128, 2, 600
+    # the arena after four rows: 1 MiB and 1.25 times six slots of four rows
+    # (h, its digits, d) with the row digits; 600 rows' h and d alone are more
+    four = 6 * 4 * (I * 4 + 6 * I // 2 + H * 4) + 4 * 6 * H // 2 + 16384
+    assert rows * k * (H + I) * 4 > four * 1.25 + (1 << 20)
     s = torch.cuda.Stream()
     with torch.cuda.stream(s):
         c = U.Context(0)
@@ -114,12 +127,14 @@ def test_rows_under_capture_without_scratch_fall_back(ctx):
         x = dev(rng.standard_normal((rows, H)).astype(np.float32))
         want = by_fours(tbl, ids, w, x)
         s.synchronize()
-        g = torch.cuda.CUDAGraph()
+        g = torch.cuda.CUDAGraph(keep_graph=True)
         with torch.cuda.graph(g, stream=s):
             got = tbl.moe_experts(ids, w, x)
+        assert graph_nodes(g) >= 3 * rows // 4
         for _ in range(3):
             got.zero_()
             g.replay()
             s.synchronize()
             assert torch.equal(got, want)
+            # eager, the grouped products: the arena grows past the graph's block
             assert torch.equal(tbl.moe_experts(ids, w, x), want)
