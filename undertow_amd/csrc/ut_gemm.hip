@@ -267,9 +267,9 @@ constexpr int64_t kGlMinRows = 32;
 // LONG (slices of more than kGlLong stages): four waves of 4 x 2 tiles, which
 // read 10 fragments for 24 matrix instructions instead of 8 for 12, each
 // half stage's beside the matrix instructions of the half before (PIPE): a
-// wave's reads otherwise stand before its products.  (Counters of the trial
-// of four buffers below, which reads so too: matrix cores 40% busy, 39% of
-// the wave cycles waiting.)  512 rows of 129280 x 7168
+// wave's reads otherwise stand before its products.  Counters: matrix cores
+// 51% busy over 129280 x 7168 and 41% over 7168 x 16384, 29% of the wave
+// cycles waiting, no LDS bank conflicts.  512 rows of 129280 x 7168
 // 1,472 -> 1,375 us (2.07 POP/s), 18432 x 7168 251 -> 227, int4 234 -> 212,
 // 7168 x 16384 214 -> 204 and at 64 rows 65.1 -> 63.1, with the digitising.
 // The short slices' eight waves fill the pipeline sooner: 509 rows of

@@ -1262,7 +1262,10 @@ int32_t prefill_dev(ut_session *s, const int32_t *ids, int64_t n, const int32_t 
 // A prefill's argmax rows and the sticky error word behind them (prefill_dev
 // leaves it at am[n]) in one copy and one wait.  logits (optional, host):
 // the rows' logits too, through the pinned buffer where they are few (the
-// runtime stages a copy to pageable memory with a wait of its own).
+// runtime stages a copy to pageable memory with a wait of its own).  What the
+// logits add to a call, straight to the caller / through the buffer: 4 KB 22 /
+// 2 us, 64 KB 42 / 18, 256 KB 53 / 31, 512 KB 66 / 48, 2 MB 169 / 167; 256 KB
+// is as much pinned memory as a call keeps for it.
 constexpr size_t kPinLogits = size_t(256) << 10;
 int32_t read_argmax(ut_session *s, int64_t n, int32_t *out, float *logits = nullptr) {
     ut_ctx *ctx = s->ctx;
