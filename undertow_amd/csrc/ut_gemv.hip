@@ -972,27 +972,22 @@ static bool fast_ok(const ut_qtensor *w);
 // rows of int8 1024 x 4096 10.7 -> 9.5 (576 x 7168: 13.4 against 12.4 but
 // 1536 x 7168 14.7 against 16.7); four of 1024 x 256 9.7 -> 7.9 (2048 x 2048:
 // 10.8 against 12.6).
-// Each row takes about 1.4 us (int4 1.7) after the last, so four rows of a
-// weight that the GEMV reads unsplit in one short launch stay there: int8
-// 64 x 64 7.4 us, 8.0 in one launch (8 x 256 8.2 / 7.6, 1 x 512 6.9 / 7.5,
-// 1 x 1024 9.5 / 8.0); int4 256 x 256 8.5 / 9.1 and 1024 x 1024 9.4 / 10.1, at
-// three rows 64 x 256 7.1 / 7.5 (256 x 1024 8.2 / 8.1); two rows of int4
-// 64 x 2048 9.6 / 7.4, 64 x 2560 9.5 / 9.2, 64 x 4096 9.5 / 10.6.
+// Each row takes about 1.4 us (int4 1.7) after the last, so four rows of int4
+// stay with the GEMV (256 x 256 8.6 us, 9.0 in one launch; 1024 x 1024 9.4 /
+// 9.9).  The other short ends (four rows of int8 64 x 64, three of int4
+// 64 x 256, two of 64 x 4096) are behind the GEMV on a stream that the host
+// keeps full (8.0 against 7.4, 7.5 / 7.1, 10.6 / 9.5 us) and as much ahead of
+// it in calls made one after another from Python, where two or three launches
+// take the host longer than the GPU (7.9 / 8.5, 7.5 / 8.6, 10.5 / 12.3): one
+// launch is the lesser load.
 // (Its workgroups read x while others write out: not where the two overlap.)
 static bool gemv_direct_ok(const ut_qtensor *w, const float *x, int64_t M, const float *out) {
     if (w->fmt != UT_FMT_INT8 && w->fmt != UT_FMT_INT4) return false;
     if (out < x + M * w->in_dim && x < out + M * w->out_dim) return false;
-    const int64_t O = w->out_dim, K = w->in_dim;
-    bool fits;
-    if (w->fmt == UT_FMT_INT8) {
-        fits = O <= 2048 && (M <= 2 ? M * K <= 8192 : M * K <= 4096);
-        if (M == 4) fits = fits && (K >= 1024 || (K >= 256 && O >= 8));
-    } else {
-        fits = O <= 1024 && (M == 1 ? K <= 8192 : M == 2 ? K <= 2560 : M == 3 && K <= 1365 && O >= 256);
-    }
-    return M >= 1 && M <= 4 && fits && fast_ok(w) && ((uintptr_t)x & 15) == 0;
+    if (w->fmt == UT_FMT_INT4 && M == 4) return false;
+    return M >= 1 && M <= 4 && M * w->in_dim <= (M <= 2 ? 64 : 32) * kDirectCols && fast_ok(w) &&
+           ((uintptr_t)x & 15) == 0 && w->out_dim <= (w->fmt == UT_FMT_INT8 ? 2048 : 1024);
 }
-static_assert(kDirectCols * 64 == 8192, "one row's columns fit the workgroup's registers");
 
 static int32_t launch_gemv_direct(ut_ctx *ctx, const ut_qtensor *w, const float *x, int64_t M,
                                   float *out, int64_t ldo) {
