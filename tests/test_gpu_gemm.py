@@ -155,7 +155,7 @@ def test_f32_rows_equal_one_row_calls(ctx, o, i):
 # the lines of gemm_f32_min_rows: split and unsplit slices of one to four
 # steps, more tiles than one wave; (rows in passes, rows in the product)
 @pytest.mark.parametrize("o,i,few,more", [(64, 64, 4, 5), (65, 128, 8, 9), (65, 132, 12, 13), (65, 252, 13, 14),
-                                          (16500, 252, 24, 25), (130, 1028, 8, 9), (256, 1024, 4, 5),
+                                          (16500, 252, 24, 25), (130, 1028, 4, 5), (256, 1024, 4, 5),
                                           (1024, 7168, 8, 9), (3000, 1500, 12, 13),
                                           (2048, 7168, 16, 17)])
 def test_f32_rows_take_the_faster_way(ctx, o, i, few, more):

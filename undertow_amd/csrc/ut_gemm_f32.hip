@@ -145,23 +145,25 @@ __global__ __launch_bounds__(256) void k_gemm_f32_sum(F32Args a) {
 // The fewest rows whose product of whole 64-row tiles beats the GEMV's
 // four-row passes.  A tile takes about 3 us per 64 columns of its slice
 // however few of its rows are there; a pass takes 3.5 us, with split K 6 and
-// more.  Split K, slices of up to 128 columns in one wave of workgroups (two
-// per CU): from five rows on (256 x 7168 18.7 us in passes, 16.2 so,
-// 512 x 4096 21.7 / 14.9, 1024 x 1024 14.4 / 13.4); longer slices (512 x 260
-// 12.4 / 15.1, 1000 x 1028 at eight rows 15.0 / 16.7, at nine 21.3 / 16.5) or
-// more workgroups (1024 x 7168 at six 28.8 / 30.1, at nine 43.6 / 29.9): from
-// nine; two waves of the longer slices (one workgroup per CU; 3000 x 1500 at
-// nine 28.1 / 30.5) from thirteen, more (2048 x 7168 at twelve 50.4 / 77.7, at
-// seventeen 82 / 78) from seventeen.  Unsplit: 64 x 64 at five 7.0 / 6.2; two
-// steps from nine (1000 x 128 at eight 7.6 / 9.8, at nine 10.4 / 9.9), three
-// from thirteen (256 x 192 at twelve 11.6 / 13.0, at thirteen 14.6 / 13.0),
-// four from fourteen (256 x 252 at thirteen 15.6 / 16.0, at sixteen
-// 17.2 / 16.2), and where their tiles (one per CU) are more than one wave, 25
-// (20000 x 256 at 20 rows 26.7 / 32.4).
+// more and a second launch.
+// Split K, slices of up to 128 columns in one wave of workgroups (two per
+// CU): from five rows on (256 x 7168 18.7 us in passes, 16.2 so, 512 x 4096
+// 21.7 / 14.9, 1024 x 1024 14.4 / 13.4); in more (1024 x 7168 at six 28.8 /
+// 30.1, at nine 43.6 / 29.9) from nine.  Longer slices in one wave (one per
+// CU) also from five: up to eight rows the passes lead on a stream that the
+// host keeps full (512 x 260 12.5 against 15.3), the product in calls made one
+// after another from Python (16.6 / 15.2: two launches, not four); in two
+// waves (3000 x 1500 at nine 28.1 / 30.5) from thirteen, in more (2048 x 7168
+// at twelve 50.4 / 77.7, at seventeen 82 / 78) from seventeen.
+// Unsplit: 64 x 64 at five 7.0 / 6.2; two steps from nine (1000 x 128 at eight
+// 7.6 / 9.8, at nine 10.4 / 9.9), three from thirteen (256 x 192 at twelve
+// 11.6 / 13.0, at thirteen 14.6 / 13.0), four from fourteen (256 x 252 at
+// thirteen 15.6 / 16.0, at sixteen 17.2 / 16.2), and where their tiles (one
+// per CU) are more than one wave, 25 (20000 x 256 at 20 rows 26.7 / 32.4).
 static int64_t gemm_f32_min_rows(int64_t O, int ks, int64_t kslice) {
     const int64_t tiles = (O + kF32Tile - 1) / kF32Tile, steps = (kslice + 63) / 64;
     if (ks > 1 && steps <= 2) return tiles * ks <= 512 ? kGemmMinRows : 9;
-    if (ks > 1) return tiles * ks <= 256 ? 9 : tiles * ks <= 512 ? 13 : 17;
+    if (ks > 1) return tiles * ks <= 256 ? kGemmMinRows : tiles * ks <= 512 ? 13 : 17;
     if (steps <= 2) return steps == 1 ? kGemmMinRows : 9;
     return tiles > 256 ? 25 : steps == 3 ? 13 : 14;
 }
