@@ -194,12 +194,13 @@ typedef float f32x16_t __attribute__((ext_vector_type(16)));
 // 16-position tiles, at least 32 and at most UT_MLA_SLICE_CAP = 512 (so at
 // most 64 slices up to 32768 positions, n_ctx/512 beyond).  A function of
 // n_ctx alone, so a row's result does not depend on which rows share the
-// call (a prompt's slices: mla_prompt_slice); no power-of-two steps, so neighbouring context lengths get similar
-// slice counts.  The cap of 512 against 256 halves the slice partials past
-// 16384 positions: at T = 32768 two- and four-row calls went from 97.2 to
-// 88.0 us and from 179.3 to 154.6 us, one-row calls from 56.6 to 61.1 us
-// (256 workgroups, one per CU).  Verify rows outnumber single rows in
-// speculative decoding (every main-model layer of a round), so 512.
+// call (a prompt's slices: mla_prompt_slice); no power-of-two steps, so
+// neighbouring context lengths get similar slice counts.  The cap of 512
+// against 256 halves the slice partials past 16384 positions: at T = 32768
+// two- and four-row calls went from 97.2 to 88.0 us and from 179.3 to 154.6
+// us, one-row calls from 56.6 to 61.1 us (256 workgroups, one per CU).  Verify
+// rows outnumber single rows in speculative decoding (every main-model layer
+// of a round), so 512.
 #ifndef UT_MLA_SLICE_CAP
 #define UT_MLA_SLICE_CAP 512
 #endif
